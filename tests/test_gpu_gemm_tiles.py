@@ -1,0 +1,82 @@
+"""The MXFP8 GEMM's tile sizes against each other, bit for bit.
+
+The tile (256, 192 or 128 tokens by 256 features, or 128 by 128) follows from the number of tokens;
+every output element is the same sequence of MFMAs on the same operands with any of them. A call on
+the first M rows of a long activation must therefore return the first M rows of the call on all of it
+(the 256 x 256 tile: 16380 tokens fill whole rounds of it), whatever tile M takes. The long call itself
+is held to the fp64 product elsewhere (test_gpu_gemm, test_gpu_gemm_full). M covers a few rows, tile edges
+and remainders of every tile, waves without any token, and both sides of the QKV launch's split."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+LONG, D, K = 16380, 5120, 512
+ROWS = [2, 31, 128, 129, 385, 768, 1000, 1024, 1025, 1560, 2113, 3120, 3137, 4100, 5500]
+
+
+@pytest.fixture(scope="module", params=["mx", "row"])
+def operands(request, pkg, dev):
+    """Codes of N(0, 1) rows, as MX blocks or with one scale per row and per output channel."""
+    g = torch.Generator(device=dev).manual_seed(41)
+    x = torch.randn(LONG, K, device=dev, generator=g).to(torch.bfloat16)
+    a = pkg.adaln_modulate(x, eps=0.0, norm_type="none", quant=request.param)
+    w = pkg.quantize_weight_mx((torch.randn(K, 3 * D, device=dev, generator=g) * 0.02).to(torch.bfloat16),
+                               torch.randn(3 * D, device=dev, generator=g) * 0.1)
+    if request.param == "row":
+        w = w._replace(col_scale=torch.rand(3 * D, device=dev, generator=g) + 0.5)
+    res = torch.randn(LONG, D, device=dev, generator=g).to(torch.bfloat16)
+    return a, w, res, torch.randn(D, device=dev, generator=g)
+
+
+def _first(a, rows):
+    return a[:rows] if isinstance(a, torch.Tensor) else type(a)(a.codes[:rows], a.scales[:rows])
+
+
+def _cols(w, n):
+    part = lambda t: None if t is None else t[:n]  # noqa: E731
+    return w._replace(codes=w.codes[:n], scales=w.scales[:n], col_scale=part(w.col_scale), bias=part(w.bias))
+
+
+def _bits(t):
+    return t.view(torch.int16) if t.dtype == torch.bfloat16 else t.view(torch.uint8)
+
+
+@pytest.mark.parametrize("epilogue", ["bf16", "gelu_mx", "gelu_bf16", "gated_residual"])
+def test_tiles_give_the_same_bits(pkg, dev, operands, epilogue):
+    a, w, res, gate = operands
+    w = _cols(w, D)
+
+    def call(m):
+        kw, ss = {}, None
+        if epilogue == "gated_residual":
+            kw = {"residual": res[:m], "gate": gate}
+        elif epilogue == "bf16":
+            ss = torch.full((m, D // 128), -1.0, device=dev)
+            kw = {"row_sumsq": ss, "sumsq_cols": D // 2}
+        y = pkg.mxfp8_linear(_first(a, m), w, epilogue=epilogue, **kw)
+        return (*y,) if isinstance(y, tuple) else (y,) if ss is None else (y, ss)
+
+    ref = call(LONG)
+    for m in ROWS:
+        for got, want in zip(call(m), ref):
+            assert torch.equal(_bits(got), _bits(want[:m])), (epilogue, m)
+
+
+def test_qkv_tiles_give_the_same_bits(pkg, dev, operands):
+    a, w, _, _ = operands
+
+    def call(m):
+        ss = torch.full((m, 2 * D // 128), -1.0, device=dev)
+        return (*pkg.mxfp8_qkv_linear(_first(a, m), w, vt_col0=2 * D, row_sumsq=ss, sumsq_cols=D), ss)
+
+    qk_ref, vt_ref, ss_ref = call(LONG)
+    for m in ROWS:
+        qk, vt, ss = call(m)
+        assert torch.equal(_bits(qk), _bits(qk_ref[:m])) and torch.equal(ss, ss_ref[:m]), m
+        pad = vt.shape[-1]
+        slot = torch.arange(pad, device=dev)
+        key = (slot & ~15) | (slot & 3) | ((slot & 4) << 1) | ((slot & 8) >> 1)
+        want = torch.where((key < m), vt_ref[:, :, :pad], torch.zeros((), dtype=vt.dtype, device=dev))
+        assert torch.equal(_bits(vt), _bits(want)), m

@@ -38,6 +38,10 @@
 // next tile's first stage is loaded while the current tile's epilogue runs, so the epilogue overlaps
 // the next tile's load latency.
 //
+// Fewer tokens than fill whole rounds of 256-token tiles take smaller ones: 192 or 128 tokens by the
+// same 256 features (the same kernel with 3 or 2 token fragments per wave), or 128 x 128 (its own
+// kernel); select_tile has the rule and what each measured. All give the same bits.
+//
 // Reference semantics: the ROW_MX projection epilogues of _qkv_cte_mx_impl / _dequant_row_mx
 // (vllm_omni_neuron/kernels/nkilib/core/qkv/qkv_cte.py:3711-3750, 3996-4021) and of the MLP
 // (kernels/nkilib/core/mlp/mlp_cte/mx/mlp_cte_mx_projection.py:630-668, GELU-tanh then
@@ -56,7 +60,6 @@ constexpr int kStageBytes = TN * BK + TM * BK;  // e4m3 codes of one stage (W ro
 constexpr int kScaleGroup = 4;                    // stages per scale load (16 bytes per row)
 constexpr int kVecFloats = 4 * 256;  // per tile: bias[n], col_scale[n], gate[n], row_scale[m]
 constexpr int kGroupM = 4;  // m tiles per group (4: the XCD's 32 concurrent tiles are 4 m x 8 n)
-constexpr int kCodeLoads = 16;   // direct-to-LDS loads per wave per stage of codes (16 x 1 KiB)
 
 struct GemmArgs {
   const uint8_t* a;         // [M, lda]
@@ -75,8 +78,10 @@ struct GemmArgs {
   int64_t sumsq_ld;         // row stride of row_sumsq in floats
   uint16_t* vt;             // V^T epilogue: [N/128][128][vt_ld] bf16
   int64_t vt_ld;
+  int64_t vt_col0;          // kEpiQkv: first V column
   int64_t M, N, K, lda, ldo;
   int tiles_m, tiles_n;
+  int qk_wgs;               // kEpiQkv, 256-feature tiles: workgroups that walk the Q|K tiles
 };
 
 // gelu_tanh(x) = 0.5 x (1 + tanh(u)) = x / (1 + exp(-2u)),  u = sqrt(2/pi) (x + 0.044715 x^3);
@@ -120,24 +125,25 @@ __device__ __forceinline__ uint32_t scale_lane_offset() {
 // 4q + 2s + h (q = the stage's position in its scale group) of the row's 16 scale bytes in `sc`
 // ([2][256] x 16 B: W rows, then A rows), read as a byte so the MFMA takes it as is. The swizzle
 // repeats every 16 rows, so a half read at its own base matches the whole stage read at row 128 wn.
-template <int I0 = 0, int I1 = 4>
+template <int I0 = 0, int I1 = 4, int kNj = 4>
 __device__ __forceinline__ void read_slice_r(const uint8_t* wbase, const uint8_t* abase, const uint32_t* sc, int q,
                                              int s, SliceOperands& op, int wn, int wm, int h, int r32, uint32_t sl) {
   const int c0 = s * 4 + h, c1 = s * 4 + 2 + h;
   const uint8_t* scb = reinterpret_cast<const uint8_t*>(sc) + 4 * q + 2 * s;
   const uint8_t* scw = scb + wn * 128 * 16 + sl;
-  const uint8_t* sca = scb + (TN + wm * 128) * 16 + sl;
+  const uint8_t* sca = scb + (TN + wm * 32 * kNj) * 16 + sl;
 #pragma unroll
   for (int i = I0; i < I1; ++i) {
     const int rw = i * 32 + r32;
     const uint4 x0 = *reinterpret_cast<const uint4*>(wbase + swz(rw, c0));
     const uint4 x1 = *reinterpret_cast<const uint4*>(wbase + swz(rw, c1));
     op.w[i] = i32x8{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
-    const int ra = wm * 128 + i * 32 + r32;
+    op.ws[i] = (int)scw[i * 32 * 16];
+    if (i >= kNj) continue;  // fewer token fragments than weight fragments
+    const int ra = wm * 32 * kNj + i * 32 + r32;
     const uint4 y0 = *reinterpret_cast<const uint4*>(abase + swz(ra, c0));
     const uint4 y1 = *reinterpret_cast<const uint4*>(abase + swz(ra, c1));
     op.a[i] = i32x8{(int)y0.x, (int)y0.y, (int)y0.z, (int)y0.w, (int)y1.x, (int)y1.y, (int)y1.z, (int)y1.w};
-    op.ws[i] = (int)scw[i * 32 * 16];
     op.as[i] = (int)sca[i * 32 * 16];
   }
 }
@@ -175,25 +181,30 @@ struct TileLoads {
   int64_t m0, n0, m_valid;
 };
 
+// Tile v of the grid of tiles_m x tiles_n tiles of kTm tokens x 256 features: XCD v & 7 takes a
+// contiguous run of the order that walks groups of m tiles (about 1024 tokens deep) along n.
+template <int kTm>
 __device__ __forceinline__ void tile_coords(const GemmArgs& g, int v, int64_t& m0, int64_t& n0) {
+  constexpr int kGroup = kGroupM * TM / kTm;
   const int total = g.tiles_m * g.tiles_n;
-  int pid = v;
-  if ((total & 7) == 0) pid = (v & 7) * (total >> 3) + (v >> 3);
-  const int in_group = kGroupM * g.tiles_n;
+  const int x = v & 7, r = total & 7;
+  const int pid = x * (total >> 3) + min(x, r) + (v >> 3);
+  const int in_group = kGroup * g.tiles_n;
   const int group = pid / in_group;
-  const int first_m = group * kGroupM;
-  const int gsz = min(g.tiles_m - first_m, kGroupM);
+  const int first_m = group * kGroup;
+  const int gsz = min(g.tiles_m - first_m, kGroup);
   const int tm = first_m + (pid % in_group) % gsz;
   const int tn = (pid % in_group) / gsz;
   n0 = (int64_t)tn * TN;
-  m0 = (int64_t)tm * TM;
+  m0 = (int64_t)tm * kTm;
 }
 
+template <int kTm = TM>
 __device__ __forceinline__ TileLoads tile_loads(const GemmArgs& g, int v) {
   TileLoads t;
-  tile_coords(g, v, t.m0, t.n0);
+  tile_coords<kTm>(g, v, t.m0, t.n0);
   const int64_t KB = g.K / 32;
-  t.m_valid = min((int64_t)TM, g.M - t.m0);
+  t.m_valid = min((int64_t)kTm, g.M - t.m0);
   // Token rows past M fall outside the activation resources' extent and read as zero.
   t.w = buffer_rsrc(g.w + t.n0 * g.K, (uint32_t)(TN * g.K));
   t.a = buffer_rsrc(g.a + t.m0 * g.lda, (uint32_t)(t.m_valid * g.lda));
@@ -319,16 +330,17 @@ __device__ __forceinline__ void store_rows_nt16(__amdgpu_buffer_rsrc_t r, uint32
   __builtin_amdgcn_raw_buffer_store_b128(u32x4{d.x, d.y, d.z, d.w}, r, (int)off, 0, 2);
 }
 
-// The gated-residual epilogue's residual rows of one half (64 tokens x the wave's 128 features,
-// bf16) into the wave's private 16 KiB residual area by direct-to-LDS loads, so that their latency
+// The gated-residual epilogue's residual rows of one half (32 kJh tokens x the wave's 128 features,
+// bf16) into the wave's private residual area (8 KiB per 32 tokens) by direct-to-LDS loads, so that their latency
 // runs under the epilogue's math instead of after it: instruction it lands rows 4 it .. 4 it + 3,
 // lane l row 4 it + (l >> 4), 16-byte chunk l & 15, at byte 1024 it + 16 l -- where lane l reads
 // it back. Rows past M read zero (the resource ends at row M, as the stores' does).
+template <int kJh>
 __device__ __forceinline__ void residual_to_lds(const GemmArgs& g, uint8_t* rarea, int mbase, int nw, int lane) {
   // the tile's row and column pass through an empty asm so that none of this is computed ahead of
   // the k loop and held through it (which spilled registers inside the loop)
   asm volatile("" : "+s"(mbase), "+s"(nw));
-  const int rows = max(0, min(64, (int)g.M - mbase));
+  const int rows = max(0, min(32 * kJh, (int)g.M - mbase));
   const uint32_t rb = (uint32_t)g.ldo * 2;
   // the resource's words through readfirstlane, as in rows_rsrc (the inputs are wave-uniform, which
   // the compiler does not prove, and the load takes the resource in scalar registers)
@@ -338,7 +350,7 @@ __device__ __forceinline__ void residual_to_lds(const GemmArgs& g, uint8_t* rare
                    (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)rows * rb), 0x00020000u};
   const uint32_t voff = (uint32_t)(lane >> 4) * rb + (uint32_t)(lane & 15) * 16;
 #pragma unroll
-  for (int it = 0; it < 16; ++it) lds_dma_b128(r, voff + (uint32_t)(it * 4) * rb, lds_addr(rarea + it * 1024));
+  for (int it = 0; it < 8 * kJh; ++it) lds_dma_b128(r, voff + (uint32_t)(it * 4) * rb, lds_addr(rarea + it * 1024));
 }
 
 // bf16 staging: [64 tokens][256 B], 16-byte chunk index XOR (token & 15) -- the 16 lanes of an LDS
@@ -392,31 +404,33 @@ __device__ __forceinline__ void epi_values(const f32x16& a, const EpiVectors<kSc
   }
 }
 
-// One wave's 128 x 128 block: two halves of 64 tokens (accumulator columns j = 2 hf, 2 hf + 1).
-// `stage` is the wave's private LDS staging area; LDS operations of one wave complete in order, so
-// the read-back needs no barrier.
+// One wave's block of 128 features x 32 kNj tokens, kJh token fragments (a "half") at a time: 128 tokens
+// in two halves of 64 (accumulator columns j = 2 hf, 2 hf + 1) for the 256 x 256 tile's waves, 32 tokens
+// at once for the 128 x 128 tile's. `stage` is the wave's private LDS staging area (8 KiB per 32
+// tokens of a half); LDS operations of one wave complete in order, so the read-back needs no barrier.
 // kScaled / kSumsq: row or column scales given / the bf16 epilogue's per-row sums of squares
 // requested. They are template parameters so that the epilogue is straight-line code: with runtime
 // flags every 16-value block branched, and the LDS reads of its bias and scales were each waited for
 // on the spot.
-template <int EPI, bool kScaled, bool kSumsq>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[4][4], const float* vec, uint8_t* stage,
+template <int EPI, bool kScaled, bool kSumsq, int kNj = 4, int kJh = 2>
+__device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[4][kNj], const float* vec, uint8_t* stage,
                                          int m0, int n0, int wm, int wn, uint8_t* rarea = nullptr) {
 #pragma clang fp contract(off)
   const int lane = fresh_lane_id();
   const int h = lane >> 5, r32 = lane & 31;
   const int nw = n0 + wn * 128;  // first feature of the wave's block
-  // gated residual: `rarea` is 16 KiB of LDS private to the wave that no load targets during the
-  // epilogue; the first half's residual rows go there now, the second half's once the first's are read
-  if constexpr (EPI == WANMI_EPI_GATED_RESIDUAL) residual_to_lds(g, rarea, m0 + wm * 128, nw, lane);
+  constexpr int kMw = 32 * kNj;  // tokens per wave
+  // gated residual: `rarea` is LDS private to the wave that no load targets during the epilogue; the
+  // first half's residual rows go there now, the second half's once the first's are read
+  if constexpr (EPI == WANMI_EPI_GATED_RESIDUAL) residual_to_lds<kJh>(g, rarea, m0 + wm * kMw, nw, lane);
   EpiVectors<kScaled> ev;
   load_epi_vectors<kScaled>(vec, wn, h, ev);
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
+  for (int hf = 0; hf < kNj / kJh; ++hf) {
     // ---- lane-local math, results into the staging area ----
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int j = 2 * hf + jj;
+    for (int jj = 0; jj < kJh; ++jj) {
+      const int j = kJh * hf + jj;
       const int tok = jj * 32 + r32;  // token within the half
       [[maybe_unused]] uint32_t sbytes = 0;
       // bf16 epilogue with row_sumsq: this lane's part of the token's sum of squares of the rounded
@@ -425,7 +439,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float v[16];
-        epi_values<kScaled>(acc[i][j], ev, i, kScaled ? vec[768 + wm * 128 + j * 32 + r32] : 1.0f, v);
+        epi_values<kScaled>(acc[i][j], ev, i, kScaled ? vec[768 + wm * kMw + j * 32 + r32] : 1.0f, v);
         if constexpr (EPI == WANMI_EPI_GELU_MX) {
           // GELU rounded to bf16 two values per conversion; the block's largest exponent field is
           // that of its largest |y|, taken as the largest (bits & 0x7fff) of the packed bf16 pairs;
@@ -479,23 +493,23 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
         if (kSumsq && nw < g.sumsq_cols) {
           const float other = __shfl_xor(ss, 32, 64);
           const float tot = h == 0 ? ss + other : other + ss;
-          const int m = m0 + wm * 128 + j * 32 + r32;
+          const int m = m0 + wm * kMw + j * 32 + r32;
           if (h == 0 && m < (int)g.M) g.row_sumsq[(uint32_t)m * (uint32_t)g.sumsq_ld + (uint32_t)(nw / 128)] = tot;
         }
       }
       if constexpr (EPI == WANMI_EPI_GELU_MX) {
-        const int m = m0 + wm * 128 + j * 32 + r32;
+        const int m = m0 + wm * kMw + j * 32 + r32;
         if (h == 0 && m < (int)g.M)
           __builtin_nontemporal_store(sbytes, reinterpret_cast<uint32_t*>(g.out_scales + (uint32_t)m * (uint32_t)(g.N / 32) +
                                                                          (uint32_t)(nw / 32)));
       }
     }
     // ---- read back whole row segments and store them ----
-    // The half's 64 token rows go through a buffer resource whose extent ends at row M: stores to
+    // The half's token rows go through a buffer resource whose extent ends at row M: stores to
     // rows past it are dropped and residual loads from them read zero, so there is no per-row branch
     // (with one, the compiler waited for each staging read inside its branch).
-    const int mbase = m0 + wm * 128 + hf * 64;
-    const int rows = max(0, min(64, (int)g.M - mbase));
+    const int mbase = m0 + wm * kMw + hf * (32 * kJh);
+    const int rows = max(0, min(32 * kJh, (int)g.M - mbase));
     // Loads issued before the epilogue (the next tile's stage 0, when prefetched here) must be
     // complete before the first store: vmcnt counts loads and stores together and stores may finish
     // out of order with loads, so once stores are queued between them and the next tile's stage-1
@@ -507,11 +521,11 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
       const uint32_t rb = (uint32_t)g.ldo;  // bytes per output row
       const auto orsrc = rows_rsrc(reinterpret_cast<uint8_t*>(g.out) + (size_t)mbase * rb + nw, rows, rb);
       const int chunk = lane & 7;
-      uint4 d[8];
+      uint4 d[4 * kJh];
 #pragma unroll
-      for (int it = 0; it < 8; ++it) d[it] = *reinterpret_cast<const uint4*>(stage + stg8(it * 8 + (lane >> 3), chunk));
+      for (int it = 0; it < 4 * kJh; ++it) d[it] = *reinterpret_cast<const uint4*>(stage + stg8(it * 8 + (lane >> 3), chunk));
 #pragma unroll
-      for (int it = 0; it < 8; ++it)
+      for (int it = 0; it < 4 * kJh; ++it)
         store_rows_nt16(orsrc, (uint32_t)(it * 8 + (lane >> 3)) * rb + (uint32_t)chunk * 16, d[it]);
     } else if constexpr (EPI == WANMI_EPI_GATED_RESIDUAL) {
       // out = bf16(res + bf16(v) * gate), 8 features per lane; the residual rows come from the
@@ -523,7 +537,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
       const float4 g1 = *reinterpret_cast<const float4*>(vec + 512 + wn * 128 + chunk * 8 + 4);
       const float gg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
-      for (int it = 0; it < 16; ++it) {
+      for (int it = 0; it < 8 * kJh; ++it) {
         const int tok = it * 4 + (lane >> 4);
         const uint4 d = *reinterpret_cast<const uint4*>(stage + stg16(tok, chunk));
         const uint4 rs = *reinterpret_cast<const uint4*>(rarea + it * 1024 + lane * 16);
@@ -538,17 +552,17 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
         }
         store_rows_nt16(orsrc, (uint32_t)tok * rb + (uint32_t)chunk * 16, make_uint4(o[0], o[1], o[2], o[3]));
       }
-      if (hf == 0) {
-        // every read of the area is complete before the second half's rows may land in it
+      if (hf + 1 < kNj / kJh) {
+        // every read of the area is complete before the next half's rows may land in it
         __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0));
-        residual_to_lds(g, rarea, mbase + 64, nw, lane);
+        residual_to_lds<kJh>(g, rarea, mbase + 32 * kJh, nw, lane);
       }
     } else {
       const uint32_t rb = (uint32_t)g.ldo * 2;
       const auto orsrc = rows_rsrc(reinterpret_cast<uint16_t*>(g.out) + (size_t)mbase * g.ldo + nw, rows, rb);
       const int chunk = lane & 15;
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {  // two batches of 8 reads, then 8 stores
+      for (int b = 0; b < kJh; ++b) {  // batches of 8 reads, then 8 stores
         uint4 d[8];
 #pragma unroll
         for (int it = 0; it < 8; ++it)
@@ -572,14 +586,22 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const f32x16 (&acc)[
 // [128 d][64 slots] bf16 in the wave's LDS area, 16-byte chunks XOR-swizzled by (d >> 1) & 7 so that
 // the writes of 32 rows spread over the banks, then stored as whole 128-byte row segments, 8 lanes
 // per row; segments at or past vt_ld are dropped.
-constexpr int kEpiVt = 100;  // internal epilogue id (wanmi_mxfp8_gemm_qkv only)
+constexpr int kEpiVt = 100;   // internal epilogue ids (wanmi_mxfp8_gemm_qkv only): V^T alone,
+constexpr int kEpiQkv = 101;  // and both parts in one launch (bf16 below vt_col0, V^T from there)
 
-__device__ __forceinline__ int vt_chunk(int d, int c16) { return d * 128 + ((c16 ^ ((d >> 1) & 7)) << 4); }
+// (halves of 32 tokens: rows of 64 bytes, four chunks, XOR (d >> 2) & 3)
+template <int kJh>
+__device__ __forceinline__ int vt_chunk(int d, int c16) {
+  return kJh == 2 ? d * 128 + ((c16 ^ ((d >> 1) & 7)) << 4) : d * 64 + ((c16 ^ ((d >> 2) & 3)) << 4);
+}
 
-template <bool kScaled>
-__device__ __forceinline__ void epilogue_vt(const GemmArgs& g, const f32x16 (&acc)[4][4], const float* vec,
+template <bool kScaled, int kNj = 4, int kJh = 2>
+__device__ __forceinline__ void epilogue_vt(const GemmArgs& g, const f32x16 (&acc)[4][kNj], const float* vec,
                                             uint8_t* stage, int m0, int n0, int wm, int wn) {
 #pragma clang fp contract(off)
+  constexpr int kMw = 32 * kNj;              // tokens per wave
+  constexpr int kLanes = 4 * kJh;            // lanes (16-byte chunks) per staged row of 32 kJh tokens
+  constexpr int kIts = 128 * kLanes / 64;    // store instructions per half
   const int lane = fresh_lane_id();
   const int h = lane >> 5, r32 = lane & 31;
   // this lane's feature of each 32-feature fragment: bias and column scale
@@ -592,13 +614,13 @@ __device__ __forceinline__ void epilogue_vt(const GemmArgs& g, const f32x16 (&ac
   const int64_t vrow0 = (int64_t)(n0 + wn * 128);  // first V^T row of the wave (head * 128), W rows offset
   const auto vrsrc = rows_rsrc(g.vt + vrow0 * g.vt_ld, 128, (uint32_t)g.vt_ld * 2);
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
+  for (int hf = 0; hf < kNj / kJh; ++hf) {
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int j = 2 * hf + jj;
+    for (int jj = 0; jj < kJh; ++jj) {
+      const int j = kJh * hf + jj;
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
-        const int tok0 = wm * 128 + j * 32 + 8 * gq + 4 * h;  // first of the 4 tokens, within the tile
+        const int tok0 = wm * kMw + j * 32 + 8 * gq + 4 * h;  // first of the 4 tokens, within the tile
         float rs[4] = {1.0f, 1.0f, 1.0f, 1.0f};
         if constexpr (kScaled) {
           const float4 r4 = *reinterpret_cast<const float4*>(vec + 768 + tok0);
@@ -616,25 +638,25 @@ __device__ __forceinline__ void epilogue_vt(const GemmArgs& g, const f32x16 (&ac
             y[q] = q < live ? v : 0.0f;
           }
           const int d = i * 32 + r32;
-          *reinterpret_cast<uint2*>(stage + vt_chunk(d, c16) + (gq & 1) * 8) =
+          *reinterpret_cast<uint2*>(stage + vt_chunk<kJh>(d, c16) + (gq & 1) * 8) =
               make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
         }
       }
     }
-    const int mbase = m0 + wm * 128 + hf * 64;
+    const int mbase = m0 + wm * kMw + hf * (32 * kJh);
     if (hf == 0) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // loads before stores, as in epilogue()
-    const int chunk = lane & 7;
+    const int chunk = lane & (kLanes - 1);
     const uint32_t col_bytes = (uint32_t)(mbase + chunk * 8) * 2;
     const bool in_row = mbase + chunk * 8 < (int)g.vt_ld;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {  // two batches of 8 reads, then 8 stores
+    for (int b = 0; b < kIts / 8; ++b) {  // batches of 8 reads, then 8 stores
       uint4 dv[8];
 #pragma unroll
       for (int it = 0; it < 8; ++it)
-        dv[it] = *reinterpret_cast<const uint4*>(stage + vt_chunk((b * 8 + it) * 8 + (lane >> 3), chunk));
+        dv[it] = *reinterpret_cast<const uint4*>(stage + vt_chunk<kJh>((b * 8 + it) * (64 / kLanes) + lane / kLanes, chunk));
 #pragma unroll
       for (int it = 0; it < 8; ++it) {
-        const uint32_t d = (uint32_t)((b * 8 + it) * 8 + (lane >> 3));
+        const uint32_t d = (uint32_t)((b * 8 + it) * (64 / kLanes) + lane / kLanes);
         // an offset past the resource's extent drops the store (segments at or past vt_ld);
         // non-temporal, as the other epilogues' outputs (through L2 the QKV pair ran 0.5% slower)
         const uint32_t off = in_row ? d * (uint32_t)g.vt_ld * 2 + col_bytes : 0xFFFFFFF0u;
@@ -754,7 +776,9 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(GemmArgs g) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// The pipelined k loop (K a multiple of 512), with its loads split over both phases of a stage.
+// The pipelined k loop (K a multiple of 512), with its loads split over both phases of a stage; tiles of
+// 64 kNj tokens (the text has kNj = 4: with fewer, the activation slots, their loads, reads and MFMAs
+// shrink in proportion and the epilogue runs 32 tokens at a time).
 // A stage is two phases of 16 MFMAs, each split into four fragment rows (4 MFMAs each) with the LDS
 // reads of one fragment row of the next slice issued before them (phase A: MFMAs on slice 0, reads
 // of slice 1; phase B: MFMAs on slice 1, reads of slice 0 of the next stage), and the stage's loads
@@ -774,7 +798,6 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_kernel(GemmArgs g) {
 // that group would have used; the next tile's scale groups start in the other one.
 // ------------------------------------------------------------------------------------------------
 constexpr int kHalfBytes = 128 * BK;  // 16 KiB: 128 weight rows of one stage
-constexpr int kActBytes = TM * BK;    // 32 KiB: 256 token rows of one stage
 // Neutral epilogue vectors, loaded in place of an absent one: bias -0, scales and gate 1.
 #define WANMI_R8(x) x, x, x, x, x, x, x, x
 #define WANMI_R64(x) WANMI_R8(x), WANMI_R8(x), WANMI_R8(x), WANMI_R8(x), WANMI_R8(x), WANMI_R8(x), WANMI_R8(x), WANMI_R8(x)
@@ -840,8 +863,9 @@ __device__ __forceinline__ void act_dma(const GemmArgs& g, const TileLoads& t, c
     lds_dma_b128(maybe_empty(t.a, valid), off, dst + (uint32_t)(8 * p * BK));
 }
 
-// All 16 loads of stage kt outside the k loop: wave w takes weight row groups 4w .. 4w+3 of both
-// halves and activation row groups 8w .. 8w+7.
+// All 8 + 2 kNj loads of stage kt outside the k loop: wave w takes weight row groups 4w .. 4w+3 of
+// both halves and 2 kNj activation row groups from 2 kNj w on.
+template <int kNj>
 __device__ __forceinline__ void issue_stage_r(const GemmArgs& g, const TileLoads& t, int kt, uint32_t h0, uint32_t h1,
                                               uint32_t act, int wave) {
   const DmaLanes dl = dma_lanes(g);
@@ -851,54 +875,59 @@ __device__ __forceinline__ void issue_stage_r(const GemmArgs& g, const TileLoads
     w_half_dma<false>(g, t, dl, kt, 1, 4 * wave + i, h1, true);
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) act_dma<false>(g, t, dl, kt, 8 * wave + i, act, true);
+  for (int i = 0; i < 2 * kNj; ++i) act_dma<false>(g, t, dl, kt, 2 * kNj * wave + i, act, true);
 }
 
-// Phase A row I: reads of slice 1 of the stage, 4 MFMAs, and weight row group 4w + I of half 0 of
+// Phase A row I: reads of slice 1 of the stage, kNj MFMAs, and weight row group 4w + I of half 0 of
 // stage kt (two stages ahead) after the first MFMA.
-template <int I, bool kSwap>
+template <int I, bool kSwap, int kNj>
 __device__ __forceinline__ void phase_a_row_r(const uint8_t* wb, const uint8_t* ab, const uint32_t* sc, int q,
-                                              SliceOperands& nxt, const SliceOperands& cur, f32x16 (&acc)[4][4], int wn,
+                                              SliceOperands& nxt, const SliceOperands& cur, f32x16 (&acc)[4][kNj], int wn,
                                               int wm, int h, int r32, uint32_t sl, const GemmArgs& g,
                                               const TileLoads& t, const DmaLanes& dl, int kt, uint32_t h0, int wave,
                                               bool valid) {
-  read_slice_r<I, I + 1>(wb, ab, sc, q, 1, nxt, wn, wm, h, r32, sl);
+  read_slice_r<I, I + 1, kNj>(wb, ab, sc, q, 1, nxt, wn, wm, h, r32, sl);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < kNj; ++j) {
     acc[I][j] = mfma_tile<kSwap>(cur.w[I], cur.a[j], acc[I][j], cur.ws[I], cur.as[j]);
     if (j == 0) w_half_dma<true>(g, t, dl, kt, 0, 4 * wave + I, h0, valid);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// Phase B row I: reads of slice 0 of the next stage, 4 MFMAs, and three loads of stage kt: weight
-// row group 4w + I of half 1 and activation row groups 8w + 2I, 8w + 2I + 1.
-template <int I, bool kSwap>
+// Phase B row I: reads of slice 0 of the next stage, kNj MFMAs, and three loads of stage kt: weight
+// row group 4w + I of half 1 and (I < kNj) two activation row groups.
+template <int I, bool kSwap, int kNj>
 __device__ __forceinline__ void phase_b_row_r(const uint8_t* wb, const uint8_t* ab, const uint32_t* sc, int q,
-                                              SliceOperands& nxt, const SliceOperands& cur, f32x16 (&acc)[4][4], int wn,
+                                              SliceOperands& nxt, const SliceOperands& cur, f32x16 (&acc)[4][kNj], int wn,
                                               int wm, int h, int r32, uint32_t sl, const GemmArgs& g,
                                               const TileLoads& t, const DmaLanes& dl, int kt, uint32_t h1,
                                               uint32_t act, int wave, bool valid) {
-  read_slice_r<I, I + 1>(wb, ab, sc, q, 0, nxt, wn, wm, h, r32, sl);
+  read_slice_r<I, I + 1, kNj>(wb, ab, sc, q, 0, nxt, wn, wm, h, r32, sl);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < kNj; ++j) {
     acc[I][j] = mfma_tile<kSwap>(cur.w[I], cur.a[j], acc[I][j], cur.ws[I], cur.as[j]);
     if (j == 0) w_half_dma<true>(g, t, dl, kt, 1, 4 * wave + I, h1, valid);
-    if (j == 1) act_dma<true>(g, t, dl, kt, 8 * wave + 2 * I, act, valid);
-    if (j == 2) act_dma<true>(g, t, dl, kt, 8 * wave + 2 * I + 1, act, valid);
+    if (I < kNj && j == 1) act_dma<true>(g, t, dl, kt, 2 * kNj * wave + 2 * I, act, valid);
+    if (I < kNj && j == (kNj > 2 ? 2 : 1)) act_dma<true>(g, t, dl, kt, 2 * kNj * wave + 2 * I + 1, act, valid);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <int EPI>
-__global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
+// One workgroup's walk over tiles v0, v0 + stride, ... of g's grid. `ssc`: the scale groups, and the
+// tile's epilogue vectors at its end. (`g` by value: through a reference the compiler kept more scalars live
+// across the k loop and spilled some.)
+template <int EPI, int kNj>
+__device__ __forceinline__ void ring_tiles(GemmArgs g, uint8_t (&sWh)[5][kHalfBytes],
+                                           uint8_t (&sAct)[2][64 * kNj * BK], uint32_t (&ssc)[2][2 * 256 * 4], int v0,
+                                           int stride) {
 #pragma clang fp contract(off)
   constexpr bool kSwap = EPI == kEpiVt;
-  __shared__ __attribute__((aligned(16))) uint8_t sWh[5][kHalfBytes];
-  __shared__ __attribute__((aligned(16))) uint8_t sAct[2][kActBytes];
-  __shared__ __attribute__((aligned(16))) uint32_t ssc[2][2 * 256 * 4];  // scale groups; the tile's vectors at its end
+  constexpr int kTm = 64 * kNj;        // tokens per tile
+  constexpr int kJh = kNj == 4 ? 2 : 1;  // token fragments per epilogue half (8 KiB of staging each)
+  constexpr int kLoads = 8 + 2 * kNj;  // code loads per wave per stage
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -914,25 +943,25 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
   // stage S in slot S % 2. Scale group G of a tile uses buffer (G + par) & 1.
   auto prefetch0 = [&](const TileLoads& tl, int par) {
     issue_scales(g, tl, 0, ssc[par & 1], wave);
-    issue_stage_r(g, tl, 0, hs(0), hs(1), lds_addr(sAct[0]), wave);
+    issue_stage_r<kNj>(g, tl, 0, hs(0), hs(1), lds_addr(sAct[0]), wave);
   };
-  auto prefetch1 = [&](const TileLoads& tl) { issue_stage_r(g, tl, 1, hs(2), hs(3), lds_addr(sAct[1]), wave); };
+  auto prefetch1 = [&](const TileLoads& tl) { issue_stage_r<kNj>(g, tl, 1, hs(2), hs(3), lds_addr(sAct[1]), wave); };
 
-  int v = blockIdx.x;
+  int v = v0;
   int par = 0;
-  prefetch0(tile_loads(g, v), par);
-  prefetch1(tile_loads(g, v));
+  prefetch0(tile_loads<kTm>(g, v), par);
+  prefetch1(tile_loads<kTm>(g, v));
 
-  f32x16 acc[4][4];
+  f32x16 acc[4][kNj];
   for (;;) {
-    const TileLoads t = tile_loads(g, v);
+    const TileLoads t = tile_loads<kTm>(g, v);
     const int vpar = ((KT >> 2) + par) & 1;  // scale buffer that takes this tile's epilogue vectors
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kCodeLoads));
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kLoads));
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < kNj; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
@@ -949,26 +978,26 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
     const uint8_t* wcur_ = sWh[(k0_ + wn) % 5];                                                         \
     const uint8_t* wnxt_ = sWh[(k0_ + 2 + wn) % 5];                                                     \
     const uint32_t h0_ = hs(k0_ + 4), h1_ = hs(k0_ + 5);                                                \
-    phase_a_row_r<0, kSwap>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
-    phase_a_row_r<1, kSwap>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
-    phase_a_row_r<2, kSwap>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
-    phase_a_row_r<3, kSwap>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
+    phase_a_row_r<0, kSwap, kNj>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
+    phase_a_row_r<1, kSwap, kNj>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
+    phase_a_row_r<2, kSwap, kNj>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
+    phase_a_row_r<3, kSwap, kNj>(wcur_, ACT_CUR, SC_CUR, Q_CUR, opB, opA, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h0_, wave, more_); \
     __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0));                                                        \
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(4));                                                          \
     __syncthreads();                                                                                    \
     if (WITH_SCALES)                                                                                    \
       issue_scales_or_vectors(g, t, ((S) + 2) / kScaleGroup, ssc[((((S) + 2) / kScaleGroup) + par) & 1], wave, more_); \
-    phase_b_row_r<0, kSwap>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
-    phase_b_row_r<1, kSwap>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
-    phase_b_row_r<2, kSwap>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
-    phase_b_row_r<3, kSwap>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
+    phase_b_row_r<0, kSwap, kNj>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
+    phase_b_row_r<1, kSwap, kNj>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
+    phase_b_row_r<2, kSwap, kNj>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
+    phase_b_row_r<3, kSwap, kNj>(wnxt_, ACT_OTH, SC_NXT, Q_NXT, opA, opB, acc, wn, wm, h, r32, sl, g, t, dl, ktn_, h1_, lds_addr(ACT_CUR), wave, more_); \
   } while (0)
 
     {
       const DmaLanes dl = dma_lanes(g);
       const uint32_t sl = scale_lane_offset();
       SliceOperands opA, opB;
-      read_slice_r(sWh[wn], sAct[0], ssc[par & 1], 0, 0, opA, wn, wm, h, r32, sl);
+      read_slice_r<0, 4, kNj>(sWh[wn], sAct[0], ssc[par & 1], 0, 0, opA, wn, wm, h, r32, sl);
       for (int kt = 0; kt < KT; kt += 4) {
         const int sg = ((kt / kScaleGroup) + par) & 1;
         WANMI_GEMM_RSTAGE(kt, sAct[0], sAct[1], ssc[sg], 0, ssc[sg], 1, false);
@@ -986,89 +1015,467 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
     // next tile's stage 1 is loaded after it.
     const float* vec = reinterpret_cast<const float*>(ssc[vpar]);
     const int m0 = (int)t.m0, n0 = (int)t.n0;
-    const int vn = v + (int)gridDim.x;
+    const int vn = v + stride;
     const bool has_next = vn < total;
     const int par_n = vpar ^ 1;
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __syncthreads();
-    if (kPrefetchBeforeEpilogue && has_next) prefetch0(tile_loads(g, vn), par_n);
+    if (kPrefetchBeforeEpilogue && has_next) prefetch0(tile_loads<kTm>(g, vn), par_n);
     {
-      uint8_t* stage = wave < 2 ? sAct[1] + wave * kStageWave : sWh[wave];
+      uint8_t* stage = wave < 2 ? sAct[1] + wave * (8192 * kJh) : sWh[wave];
       // the gated residual's rows: activation slot 0 and half slots 0-1, which that epilogue's tile
       // only prefetches into after it
-      uint8_t* rarea = wave < 2 ? sAct[0] + wave * kStageWave : sWh[wave - 2];
+      uint8_t* rarea = wave < 2 ? sAct[0] + wave * (8192 * kJh) : sWh[wave - 2];
       const bool scaled = g.row_scale || g.col_scale;
       if constexpr (EPI == kEpiVt) {
-        if (scaled) epilogue_vt<true>(g, acc, vec, stage, m0, n0, wm, wn);
-        else epilogue_vt<false>(g, acc, vec, stage, m0, n0, wm, wn);
+        if (scaled) epilogue_vt<true, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
+        else epilogue_vt<false, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
       } else if constexpr (EPI == WANMI_EPI_BF16) {
         if (g.row_sumsq) {
-          if (scaled) epilogue<EPI, true, true>(g, acc, vec, stage, m0, n0, wm, wn);
-          else epilogue<EPI, false, true>(g, acc, vec, stage, m0, n0, wm, wn);
+          if (scaled) epilogue<EPI, true, true, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
+          else epilogue<EPI, false, true, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
         } else {
-          if (scaled) epilogue<EPI, true, false>(g, acc, vec, stage, m0, n0, wm, wn);
-          else epilogue<EPI, false, false>(g, acc, vec, stage, m0, n0, wm, wn);
+          if (scaled) epilogue<EPI, true, false, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
+          else epilogue<EPI, false, false, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn);
         }
       } else {
-        if (scaled) epilogue<EPI, true, false>(g, acc, vec, stage, m0, n0, wm, wn, rarea);
-        else epilogue<EPI, false, false>(g, acc, vec, stage, m0, n0, wm, wn, rarea);
+        if (scaled) epilogue<EPI, true, false, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn, rarea);
+        else epilogue<EPI, false, false, kNj, kJh>(g, acc, vec, stage, m0, n0, wm, wn, rarea);
       }
     }
     if (!has_next) break;
     __syncthreads();  // every wave is done with its staging area and the vectors
-    if (!kPrefetchBeforeEpilogue) prefetch0(tile_loads(g, vn), par_n);
-    prefetch1(tile_loads(g, vn));
+    if (!kPrefetchBeforeEpilogue) prefetch0(tile_loads<kTm>(g, vn), par_n);
+    prefetch1(tile_loads<kTm>(g, vn));
     v = vn;
     par = par_n;
   }
   __builtin_amdgcn_s_waitcnt(0);  // no load may still target LDS when the workgroup retires
 }
 
-// kPipelined (K a multiple of 512): the pipelined ring kernel; otherwise the simple loop.
-template <bool kPipelined>
-static void launch_gemm(int epilogue, dim3 grid, hipStream_t stream, const GemmArgs& g) {
-  if constexpr (kPipelined) {
-    switch (epilogue) {
-      case WANMI_EPI_BF16: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_BF16>), grid, dim3(256), 0, stream, g); break;
-      case WANMI_EPI_GELU_MX: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GELU_MX>), grid, dim3(256), 0, stream, g); break;
-      case WANMI_EPI_GELU_BF16: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GELU_BF16>), grid, dim3(256), 0, stream, g); break;
-      case kEpiVt: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<kEpiVt>), grid, dim3(256), 0, stream, g); break;
-      default: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GATED_RESIDUAL>), grid, dim3(256), 0, stream, g); break;
+template <int EPI, int kNj>
+__global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint8_t sWh[5][kHalfBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t sAct[2][64 * kNj * BK];
+  __shared__ __attribute__((aligned(16))) uint32_t ssc[2][2 * 256 * 4];
+  if constexpr (EPI == kEpiQkv) {
+    // workgroups [0, qk_wgs) walk the Q|K tiles, the others the V tiles
+    const int wg = (int)blockIdx.x;
+    if (wg < g.qk_wgs) {
+      g.tiles_n = (int)(g.vt_col0 / TN);
+      ring_tiles<WANMI_EPI_BF16, kNj>(g, sWh, sAct, ssc, wg, g.qk_wgs);
+    } else {
+      g.tiles_n -= (int)(g.vt_col0 / TN);
+      g.w += g.vt_col0 * g.K;
+      g.w_scales += g.vt_col0 * (g.K / 32);
+      if (g.col_scale) g.col_scale += g.vt_col0;
+      if (g.bias) g.bias += g.vt_col0;
+      ring_tiles<kEpiVt, kNj>(g, sWh, sAct, ssc, wg - g.qk_wgs, (int)gridDim.x - g.qk_wgs);
     }
   } else {
-    switch (epilogue) {
-      case WANMI_EPI_BF16: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_BF16>), grid, dim3(256), 0, stream, g); break;
-      case WANMI_EPI_GELU_MX: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GELU_MX>), grid, dim3(256), 0, stream, g); break;
-      case WANMI_EPI_GELU_BF16: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GELU_BF16>), grid, dim3(256), 0, stream, g); break;
-      case kEpiVt: hipLaunchKernelGGL((mxfp8_gemm_kernel<kEpiVt>), grid, dim3(256), 0, stream, g); break;
-      default: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GATED_RESIDUAL>), grid, dim3(256), 0, stream, g); break;
+    ring_tiles<EPI, kNj>(g, sWh, sAct, ssc, (int)blockIdx.x, (int)gridDim.x);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// 128 x 128 tiles, for the smallest token counts (select_tile has the rule). One workgroup of 4 waves
+// per tile and per CU, not persistent. A wave owns all 128 features of 32 tokens (4 x 1 MFMA tiles, 64
+// accumulator registers; the V^T epilogue: 32 features of all 128 tokens), so that the epilogue's
+// per-token sums over 128 columns stay within a wave, in the order of the 256-feature kernel's. Every
+// output element is the same sequence of MFMAs on the same operands as there: bit-identical results.
+// The operand codes go through a ring of four 32 KiB stages in LDS (W rows, then token rows; same
+// swizzle and direct-to-LDS loads), with one barrier per stage and the loads spread between the MFMAs:
+// in phase A (slice-0 MFMAs, slice-1 reads of stage S) the second half of stage S + 3's loads, after
+// the barrier in phase B (slice-1 MFMAs, slice-0 reads of S + 1) the first half of S + 4's, into the
+// slot of S that the barrier freed. A row's 16 scale bytes of four stages are held in registers.
+// What bounds it: the loads' latency. One CU streams about 58 GB/s of operand tiles that miss its
+// L2, whatever the number of CUs (32 KiB per stage, 0.55 us per stage with or without the MFMAs and
+// the LDS reads; two workgroups per CU on two stages each 0.8 us), so at few tokens the time goes with
+// the bytes per CU, and the smallest tile wins as long as its grid fits one round. Measured, 512
+// tokens, 5120 x 5120: 53.9 us with 256 x 256 tiles, 23.3 us here; 13824 deep: 126 and 49 us.
+// ------------------------------------------------------------------------------------------------
+constexpr int TS = 128;                      // features and tokens per tile
+constexpr int kTsStage = 2 * TS * BK;        // bytes of codes per stage
+constexpr int kTsLoads = 8;                  // code loads per wave per stage
+constexpr int kTsStages = 4;                 // LDS ring depth in stages
+constexpr int kTsGroupM = 8;                 // m tiles per group of the tile order
+
+// Tile of workgroup v: XCD v & 7 takes a contiguous run of the grouped order (any total).
+__device__ __forceinline__ void ts_coords(const GemmArgs& g, int v, int& m0, int& n0) {
+  const int total = g.tiles_m * g.tiles_n;
+  const int x = v & 7, q = total >> 3, r = total & 7;
+  const int pid = x * q + min(x, r) + (v >> 3);
+  const int in_group = kTsGroupM * g.tiles_n;
+  const int group = pid / in_group;
+  const int first_m = group * kTsGroupM;
+  const int gsz = min(g.tiles_m - first_m, kTsGroupM);
+  m0 = (first_m + (pid % in_group) % gsz) * TS;
+  n0 = ((pid % in_group) / gsz) * TS;
+}
+
+struct TsShared {
+  uint8_t code[kTsStages][kTsStage];
+  uint32_t sc[2 * TS * 4];  // one scale group (16 bytes per row: W rows, then token rows)
+  float vec[kVecFloats];    // epilogue vectors, one per KiB as in the 256 x 256 kernel
+};
+
+// V^T epilogue of a wave's 32 features (rows d = 32 wave .. + 31 of the head) x 128 tokens: as
+// epilogue_vt, staged as [32 d][128 slots] bf16, 16-byte chunk index XOR (d & 15).
+template <bool kScaled>
+__device__ __forceinline__ void epilogue_vt_row(const GemmArgs& g, const f32x16 (&acc)[4], const float* vec,
+                                                uint8_t* stage, int m0, int64_t vrow0, int wave) {
+#pragma clang fp contract(off)
+  const int lane = fresh_lane_id();
+  const int h = lane >> 5, r32 = lane & 31;
+  const float fb = vec[wave * 32 + r32];
+  const float fc = kScaled ? vec[256 + wave * 32 + r32] : 1.0f;
+  const auto vrsrc = rows_rsrc(g.vt + (vrow0 + wave * 32) * g.vt_ld, 32, (uint32_t)g.vt_ld * 2);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      const int tok0 = j * 32 + 8 * gq + 4 * h;
+      float rs[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+      if constexpr (kScaled) {
+        const float4 r4 = *reinterpret_cast<const float4*>(vec + 768 + tok0);
+        rs[0] = r4.x, rs[1] = r4.y, rs[2] = r4.z, rs[3] = r4.w;
+      }
+      const int live = (int)g.M - (m0 + tok0);
+      float y[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float a = acc[j][gq * 4 + q];
+        const float v = kScaled ? (a * rs[q]) * fc + fb : a + fb;
+        y[q] = q < live ? v : 0.0f;
+      }
+      const int c16 = 2 * (2 * j + (gq >> 1)) + h;  // 16-byte chunk: keys in the order 0-3, 8-11, 4-7, 12-15
+      *reinterpret_cast<uint2*>(stage + stg16(r32, c16) + (gq & 1) * 8) =
+          make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
     }
+  const int chunk = lane & 15;
+  const uint32_t col_bytes = (uint32_t)(m0 + chunk * 8) * 2;
+  const bool in_row = m0 + chunk * 8 < (int)g.vt_ld;
+  uint4 dv[8];
+#pragma unroll
+  for (int it = 0; it < 8; ++it) dv[it] = *reinterpret_cast<const uint4*>(stage + stg16(it * 4 + (lane >> 4), chunk));
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    // an offset past the resource's extent drops the store (segments at or past vt_ld)
+    const uint32_t off = in_row ? (uint32_t)(it * 4 + (lane >> 4)) * (uint32_t)g.vt_ld * 2 + col_bytes : 0xFFFFFFF0u;
+    store_rows_nt16(vrsrc, off, dv[it]);
+  }
+}
+
+// Operands of one 64-deep k slice of a wave: four fragments of the side it covers whole (features, or
+// tokens for the V^T epilogue) and one of the other.
+struct TsSlice {
+  i32x8 four[4];
+  i32x8 one;
+};
+
+template <int EPI>
+__device__ __forceinline__ void ts_tile(const GemmArgs& g, TsShared& sh, int m0, int n0) {
+#pragma clang fp contract(off)
+  constexpr bool kSwap = EPI == kEpiVt;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, r32 = lane & 31;
+  const int KT = (int)(g.K / BK);  // a multiple of 4
+  const uint32_t KB = (uint32_t)(g.K / 32);
+  TileLoads t;
+  t.m0 = m0;
+  t.n0 = n0;
+  t.m_valid = min((int64_t)TS, g.M - m0);
+  // Token rows past M fall outside the activation resources' extent and read as zero.
+  t.w = buffer_rsrc(g.w + (int64_t)n0 * g.K, (uint32_t)(TS * g.K));
+  t.a = buffer_rsrc(g.a + (int64_t)m0 * g.lda, (uint32_t)(t.m_valid * g.lda));
+  t.ws = buffer_rsrc(g.w_scales + (int64_t)n0 * KB, (uint32_t)TS * KB);
+  t.as = buffer_rsrc(g.a_scales + (int64_t)m0 * KB, (uint32_t)t.m_valid * KB);
+  const DmaLanes dl = dma_lanes(g);
+  // Load i of a stage: wave w's row group 4w + i / 2 (8 rows, 1 KiB) of W (even i) or the tokens (odd i).
+  // Past the end of K an empty extent turns a load into a zero fill that moves no memory.
+  auto issue_code = [&](int i, int kt, uint8_t* buf) {
+    const bool valid = kt < KT;
+    const uint32_t rg = (uint32_t)(wave * 32 + (i >> 1) * 8);
+    const uint32_t lds = lds_addr(buf) + rg * BK, kofs = (uint32_t)kt * BK;
+    if ((i & 1) == 0)
+      lds_dma_b128_hot(maybe_empty(t.w, valid), (((i >> 1) & 1) ? dl.wo : dl.we) + rg * (uint32_t)g.K + kofs, lds);
+    else
+      lds_dma_b128_hot(maybe_empty(t.a, valid), (((i >> 1) & 1) ? dl.ao : dl.ae) + rg * (uint32_t)g.lda + kofs, lds + TS * BK);
+  };
+  // waves 0-1: the W rows' scale group, waves 2-3 the token rows' (16 bytes per row)
+  const u32x4 sr = wave < 2 ? t.ws : t.as;
+  const uint32_t soff = (uint32_t)((wave & 1) * 64 + lane) * KB;
+  auto issue_scales_ts = [&](int grp, bool valid) {
+    lds_dma_b128(maybe_empty(sr, valid), soff + (uint32_t)grp * 16, lds_addr(sh.sc) + (uint32_t)wave * 1024);
+  };
+  {  // epilogue vector `wave` (128 floats; the load's other lanes fall past the extent)
+    const float* p = wave == 0 ? (g.bias ? g.bias + n0 : kNeutralNegZero)
+                   : wave == 1 ? (g.col_scale ? g.col_scale + n0 : kNeutralOne)
+                   : wave == 2 ? (g.gate ? g.gate + n0 : kNeutralOne)
+                               : (g.row_scale ? g.row_scale + m0 : kNeutralOne);
+    const uint32_t bytes = (wave == 3 && g.row_scale) ? (uint32_t)(t.m_valid * 4) : 512u;
+    lds_dma_b128(buffer_rsrc(p, bytes), (uint32_t)lane * 16, lds_addr(sh.vec) + (uint32_t)wave * 1024);
+  }
+  constexpr int kAhead = kTsLoads / 2;  // loads of a stage issued in phase A (the others in the phase B before)
+  issue_scales_ts(0, true);
+#pragma unroll
+  for (int s = 0; s < kTsStages; ++s)
+#pragma unroll
+    for (int i = 0; i < kTsLoads - (s == kTsStages - 1 ? kAhead : 0); ++i) issue_code(i, s, sh.code[s]);
+
+  f32x16 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+
+  // Reads of fragment f (0-3: the side covered whole, 4: the other) of slice s of a stage slot.
+  auto read_frag = [&](int f, const uint8_t* base, int s) {
+    const bool tokens = (f < 4) == kSwap;
+    const int row = f < 4 ? f * 32 + r32 : wave * 32 + r32;
+    const uint8_t* b = base + (tokens ? TS * BK : 0);
+    const uint4 x0 = *reinterpret_cast<const uint4*>(b + swz(row, s * 4 + h));
+    const uint4 x1 = *reinterpret_cast<const uint4*>(b + swz(row, s * 4 + 2 + h));
+    return i32x8{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+  };
+  // Scale bytes of the five fragments' rows for the four stages of a group (byte 4 u + 2 s + h: stage
+  // u, slice s).
+  uint32_t sc[5][4];
+  auto read_scales = [&]() {
+#pragma unroll
+    for (int f = 0; f < 5; ++f) {
+      const bool tokens = (f < 4) == kSwap;
+      const int row = (f < 4 ? f * 32 : wave * 32) + (tokens ? TS : 0) + r32;
+      const uint4 v = *reinterpret_cast<const uint4*>(sh.sc + row * 4);
+      sc[f][0] = v.x, sc[f][1] = v.y, sc[f][2] = v.z, sc[f][3] = v.w;
+    }
+  };
+  // stage 0 (and the first scale group) landed
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm((kTsStages - 1) * kTsLoads - kAhead));
+  __syncthreads();
+  read_scales();
+  TsSlice opA, opB;
+#pragma unroll
+  for (int f = 0; f < 4; ++f) opA.four[f] = read_frag(f, sh.code[0], 0);
+  opA.one = read_frag(4, sh.code[0], 0);
+
+  for (int kt = 0; kt < KT; kt += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int S = kt + u;
+      uint8_t* cur = sh.code[u % kTsStages];
+      uint8_t* nxt = sh.code[(u + 1) % kTsStages];
+      uint8_t* prv = sh.code[(u + kTsStages - 1) % kTsStages];
+      // the lane's scale bytes of the stage: byte 0 for slice 0, byte 2 for slice 1
+      int ss[5];
+#pragma unroll
+      for (int f = 0; f < 5; ++f) ss[f] = (int)(sc[f][u] >> (8 * h));
+      // phase A: slice-0 MFMAs, slice-1 reads, the last kAhead loads of stage S + kTsStages - 1
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i == 0) opB.one = read_frag(4, cur, 1);
+        opB.four[i] = read_frag(i, cur, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(opA.four[i], opA.one, acc[i], 0, 0, 0, ss[i], 0, ss[4]);
+        issue_code(kTsLoads - kAhead + i, S + kTsStages - 1, prv);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // this wave's reads of stage S are complete, and its loads of stage S + 1
+      __builtin_amdgcn_s_waitcnt(waitcnt_lgkm(0));
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm((kTsStages - 2) * kTsLoads));
+      __syncthreads();
+      if (u == 0) issue_scales_ts(kt / 4 + 1, kt + 4 < KT);
+      if (u == 3) read_scales();
+      // phase B: slice-1 MFMAs, slice-0 reads of the next stage, loads of stage S + kTsStages into this
+      // stage's slot
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i == 0) opA.one = read_frag(4, nxt, 0);
+        opA.four[i] = read_frag(i, nxt, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(opB.four[i], opB.one, acc[i], 0, 0, 2, ss[i], 2, ss[4]);
+        issue_code(i, S + kTsStages, cur);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+  __syncthreads();  // every wave is past its operand reads: the stage slots serve the epilogue
+  uint8_t* stage = sh.code[0] + wave * 8192;
+  uint8_t* rarea = sh.code[1] + wave * 8192;
+  const bool scaled = g.row_scale || g.col_scale;
+  if constexpr (kSwap) {
+    if (scaled) epilogue_vt_row<true>(g, acc, sh.vec, stage, m0, n0 - g.vt_col0, wave);
+    else epilogue_vt_row<false>(g, acc, sh.vec, stage, m0, n0 - g.vt_col0, wave);
+  } else {
+    if (m0 + wave * 32 >= (int)g.M) return;  // no token of this wave
+    f32x16 a1[4][1] = {{acc[0]}, {acc[1]}, {acc[2]}, {acc[3]}};
+    if constexpr (EPI == WANMI_EPI_BF16) {
+      if (g.row_sumsq) {
+        if (scaled) epilogue<EPI, true, true, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0);
+        else epilogue<EPI, false, true, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0);
+      } else {
+        if (scaled) epilogue<EPI, true, false, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0);
+        else epilogue<EPI, false, false, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0);
+      }
+    } else {
+      if (scaled) epilogue<EPI, true, false, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0, rarea);
+      else epilogue<EPI, false, false, 1, 1>(g, a1, sh.vec, stage, m0, n0, wave, 0, rarea);
+    }
+  }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 1) void mxfp8_gemm_tile128_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) TsShared sh;
+  int m0, n0;
+  ts_coords(g, (int)blockIdx.x, m0, n0);
+  if constexpr (EPI == kEpiQkv) {
+    if (n0 >= (int)g.vt_col0) ts_tile<kEpiVt>(g, sh, m0, n0);
+    else ts_tile<WANMI_EPI_BF16>(g, sh, m0, n0);
+  } else {
+    ts_tile<EPI>(g, sh, m0, n0);
+  }
+}
+
+static void launch_tile128(int epilogue, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+  switch (epilogue) {
+    case WANMI_EPI_BF16: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<WANMI_EPI_BF16>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_MX: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<WANMI_EPI_GELU_MX>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_BF16: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<WANMI_EPI_GELU_BF16>), grid, dim3(256), 0, stream, g); break;
+    case kEpiVt: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<kEpiVt>), grid, dim3(256), 0, stream, g); break;
+    case kEpiQkv: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<kEpiQkv>), grid, dim3(256), 0, stream, g); break;
+    default: hipLaunchKernelGGL((mxfp8_gemm_tile128_kernel<WANMI_EPI_GATED_RESIDUAL>), grid, dim3(256), 0, stream, g); break;
+  }
+}
+
+// The pipelined kernel on tiles of 64 kNj tokens (K a multiple of 512).
+template <int kNj>
+static void launch_ring(int epilogue, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+  switch (epilogue) {
+    case WANMI_EPI_BF16: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_BF16, kNj>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_MX: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GELU_MX, kNj>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_BF16: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GELU_BF16, kNj>), grid, dim3(256), 0, stream, g); break;
+    case kEpiVt: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<kEpiVt, kNj>), grid, dim3(256), 0, stream, g); break;
+    case kEpiQkv: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<kEpiQkv, kNj>), grid, dim3(256), 0, stream, g); break;
+    default: hipLaunchKernelGGL((mxfp8_gemm_ring_kernel<WANMI_EPI_GATED_RESIDUAL, kNj>), grid, dim3(256), 0, stream, g); break;
+  }
+}
+
+// The simple loop (K a multiple of 128).
+static void launch_simple(int epilogue, dim3 grid, hipStream_t stream, const GemmArgs& g) {
+  switch (epilogue) {
+    case WANMI_EPI_BF16: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_BF16>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_MX: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GELU_MX>), grid, dim3(256), 0, stream, g); break;
+    case WANMI_EPI_GELU_BF16: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GELU_BF16>), grid, dim3(256), 0, stream, g); break;
+    case kEpiVt: hipLaunchKernelGGL((mxfp8_gemm_kernel<kEpiVt>), grid, dim3(256), 0, stream, g); break;
+    default: hipLaunchKernelGGL((mxfp8_gemm_kernel<WANMI_EPI_GATED_RESIDUAL>), grid, dim3(256), 0, stream, g); break;
   }
 }
 
 }  // namespace wanmi
 
 namespace wanmi {
+// Which tile a product of M tokens takes on `cus` CUs (one workgroup each), and at what cost.
+struct TilePlan {
+  int nj;      // token fragments per wave of the 256-feature kernel (tiles of 64 nj tokens); 0: 128 x 128 tiles
+  int64_t cost;
+  int qk_wgs;  // kEpiQkv on 256-feature tiles
+};
+
+// Every CU takes one tile at a time, so a product costs its rounds of `cus` tiles times one tile's
+// time, which is the same for all full tiles of a kind but not proportional to the tile: the loads
+// bound it, and a smaller tile needs more of them per flop. Measured per k stage in rounds of 5120 x
+// 5120 (one to twenty rounds): 256 x 256 tiles 1.30-1.60 us, 192 tokens x 256 1.05-1.25, 128 x 256
+// 0.87-0.97, 128 x 128 0.55-0.58; K = 13824 and the GELU epilogue give the same ratios within 3%. A
+// smaller tile pays where it saves a round or fills the only one: 5120 x 5120 at 512 tokens 54 -> 23 us
+// (128 x 128), 1024 55 -> 37 (128 x 256), 1560 57 -> 47 (192), 3120 119 -> 83 (128 x 256), 4100 122 ->
+// 101 (192); at 5500 tokens 130 against 146 (192) and at 16380 338 against 364, the 256 x 256 tile.
+constexpr int kTileCost[5] = {40, 0, 67, 82, 100};  // by nj (0: 128 x 128 tiles)
+
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Best tile for n output columns (a multiple of 256); a larger tile wins a tie. V^T columns are
+// written for whole tiles only, so tiles that end before vt_ld are not taken.
+static TilePlan select_tile(int64_t M, int64_t n, int64_t cus, int64_t vt_ld) {
+  TilePlan best{4, kTileCost[4] * ceil_div(ceil_div(M, 256) * (n / TN), cus), 0};
+  for (int nj : {3, 2, 0}) {
+    const int64_t tm = nj ? 64 * nj : TS, tn = nj ? TN : TS;
+    const int64_t mt = ceil_div(M, tm);
+    if (mt * tm < vt_ld) continue;
+    const int64_t cost = kTileCost[nj] * ceil_div(mt * (n / tn), cus);
+    if (cost < best.cost) best = TilePlan{nj, cost, 0};
+  }
+  return best;
+}
+
+// The same for Q|K (qk columns) and V (v columns) in one launch: on 256-feature tiles the CUs are split
+// between the two parts so that the longer one is shortest; 128 x 128 tiles mix freely.
+static TilePlan select_qkv_tile(int64_t M, int64_t qk, int64_t v, int64_t cus, int64_t vt_ld) {
+  TilePlan best{4, INT64_MAX, 0};
+  for (int nj : {4, 3, 2, 0}) {
+    const int64_t tm = nj ? 64 * nj : TS;
+    const int64_t mt = ceil_div(M, tm);
+    if (mt * tm < vt_ld) continue;
+    if (nj == 0) {
+      const int64_t cost = kTileCost[0] * ceil_div(mt * ((qk + v) / TS), cus);
+      if (cost < best.cost) best = TilePlan{0, cost, 0};
+      continue;
+    }
+    const int64_t tq = mt * (qk / TN), tv = mt * (v / TN);
+    if (tq + tv <= cus) {  // one tile per workgroup
+      if (kTileCost[nj] < best.cost) best = TilePlan{nj, kTileCost[nj], (int)tq};
+      continue;
+    }
+    for (int64_t w = 1; w < cus; ++w) {
+      const int64_t cost = kTileCost[nj] * std::max(ceil_div(tq, w), ceil_div(tv, cus - w));
+      if (cost < best.cost) best = TilePlan{nj, cost, (int)w};
+    }
+  }
+  return best;
+}
+
+// One launch of the pipelined kernels with tile `plan` (g's tile counts are filled in here).
+static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t cus, hipStream_t stream) {
+  const int64_t tm = plan.nj ? 64 * plan.nj : TS, tn = plan.nj ? TN : TS;
+  g.tiles_m = (int)ceil_div(g.M, tm);
+  g.tiles_n = (int)(g.N / tn);
+  g.qk_wgs = plan.qk_wgs;
+  const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+  if (plan.nj == 0) {
+    launch_tile128(epilogue, dim3((unsigned)tiles), stream, g);
+    return check_launch("wanmi_mxfp8_gemm");
+  }
+  const dim3 grid((unsigned)std::min<int64_t>(tiles, cus));
+  if (plan.nj == 4) launch_ring<4>(epilogue, grid, stream, g);
+  else if (plan.nj == 3) launch_ring<3>(epilogue, grid, stream, g);
+  else launch_ring<2>(epilogue, grid, stream, g);
+  return check_launch("wanmi_mxfp8_gemm");
+}
+
 static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes, const uint8_t* w_scales,
                      const float* row_scale, const float* col_scale, const float* bias, int64_t M, int64_t N,
                      int64_t K, int64_t lda, int epilogue, void* out, int64_t ldo, uint8_t* out_scales,
                      const void* residual, const float* gate, float* row_sumsq, int64_t sumsq_cols, int64_t sumsq_ld,
-                     void* vt, int64_t vt_ld, void* stream) {
+                     void* vt, int64_t vt_ld, int64_t vt_col0, void* stream) {
   WANMI_REQUIRE(M >= 0 && N > 0 && K > 0, WANMI_ERR_ARG, "wanmi_mxfp8_gemm: bad sizes M=%lld N=%lld K=%lld",
                 (long long)M, (long long)N, (long long)K);
   WANMI_REQUIRE(N % TN == 0, WANMI_ERR_UNSUPPORTED, "wanmi_mxfp8_gemm: N=%lld must be a multiple of %d",
                 (long long)N, TN);
   WANMI_REQUIRE(K % BK == 0, WANMI_ERR_UNSUPPORTED, "wanmi_mxfp8_gemm: K=%lld must be a multiple of %d",
                 (long long)K, BK);
-  WANMI_REQUIRE((epilogue >= WANMI_EPI_BF16 && epilogue <= WANMI_EPI_GATED_RESIDUAL) || epilogue == kEpiVt,
+  WANMI_REQUIRE((epilogue >= WANMI_EPI_BF16 && epilogue <= WANMI_EPI_GATED_RESIDUAL) || epilogue == kEpiVt || epilogue == kEpiQkv,
                 WANMI_ERR_ARG, "wanmi_mxfp8_gemm: unknown epilogue %d", epilogue);
   WANMI_REQUIRE(lda >= K && lda % 16 == 0, WANMI_ERR_ARG, "wanmi_mxfp8_gemm: lda=%lld must be >= K and a multiple of 16",
                 (long long)lda);
-  const bool to_vt = epilogue == kEpiVt;
-  WANMI_REQUIRE(to_vt || (ldo >= N && ldo % 16 == 0), WANMI_ERR_ARG,
+  const bool to_vt = epilogue == kEpiVt, to_qkv = epilogue == kEpiQkv;
+  WANMI_REQUIRE(to_vt || (ldo >= (to_qkv ? vt_col0 : N) && ldo % 16 == 0), WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm: ldo=%lld must be >= N and a multiple of 16", (long long)ldo);
   if (M == 0) return WANMI_OK;
-  WANMI_REQUIRE(a_codes && a_scales && w_codes && w_scales && (to_vt ? vt != nullptr : out != nullptr), WANMI_ERR_ARG,
+  WANMI_REQUIRE(a_codes && a_scales && w_codes && w_scales && (to_vt || out != nullptr) &&
+                    (!(to_vt || to_qkv) || vt != nullptr), WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm: null operand");
   WANMI_REQUIRE(epilogue != WANMI_EPI_GELU_MX || out_scales, WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm: GELU_MX epilogue needs out_scales");
@@ -1086,7 +1493,7 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
   WANMI_REQUIRE(tiles < (1LL << 31), WANMI_ERR_ARG, "wanmi_mxfp8_gemm: problem too large");
   WANMI_REQUIRE(to_vt || (M * ldo < (1LL << 32) && M < (1LL << 31)), WANMI_ERR_UNSUPPORTED,
                 "wanmi_mxfp8_gemm: M=%lld x ldo=%lld output elements exceed 32-bit offsets", (long long)M, (long long)ldo);
-  WANMI_REQUIRE(!to_vt || (vt_ld >= M && vt_ld % 64 == 0 && 128 * vt_ld * 2 < (1LL << 31)), WANMI_ERR_ARG,
+  WANMI_REQUIRE(!(to_vt || to_qkv) || (vt_ld >= M && vt_ld % 64 == 0 && 128 * vt_ld * 2 < (1LL << 31)), WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm: vt_ld=%lld must be >= M, a multiple of 64 and below 2^23", (long long)vt_ld);
   // per-tile buffer offsets are 32-bit; this also keeps K and lda below 2^23 for the 24-bit
   // multiplies of the load offsets
@@ -1117,16 +1524,19 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
   g.K = K;
   g.lda = lda;
   g.ldo = ldo;
+  g.vt_col0 = to_qkv ? vt_col0 : 0;
   g.tiles_m = (int)((M + TM - 1) / TM);
   g.tiles_n = (int)(N / TN);
+  g.qk_wgs = 0;
   // persistent: one workgroup per CU (the LDS footprint allows no second one)
   const int cus = device_cu_count();
   WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm: cannot query the device's compute units");
-  const dim3 grid((unsigned)std::min<int64_t>(tiles, cus));
-  if ((K / BK) % 4 == 0)
-    launch_gemm<true>(epilogue, grid, (hipStream_t)stream, g);
-  else
-    launch_gemm<false>(epilogue, grid, (hipStream_t)stream, g);
+  if ((K / BK) % 4 == 0) {
+    const int64_t pad = to_vt || to_qkv ? vt_ld : 0;
+    const TilePlan plan = to_qkv ? select_qkv_tile(M, vt_col0, N - vt_col0, cus, pad) : select_tile(M, N, cus, pad);
+    return launch_plan(epilogue, plan, g, cus, (hipStream_t)stream);
+  }
+  launch_simple(epilogue, dim3((unsigned)std::min<int64_t>(tiles, cus)), (hipStream_t)stream, g);
   return check_launch("wanmi_mxfp8_gemm");
 }
 }  // namespace wanmi
@@ -1140,7 +1550,7 @@ extern "C" int wanmi_mxfp8_gemm(const uint8_t* a_codes, const uint8_t* a_scales,
   WANMI_REQUIRE(epilogue >= WANMI_EPI_BF16 && epilogue <= WANMI_EPI_GATED_RESIDUAL, WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm: unknown epilogue %d", epilogue);
   return wanmi::gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, N, K, lda, epilogue,
-                          out, ldo, out_scales, residual, gate, nullptr, 0, 0, nullptr, 0, stream);
+                          out, ldo, out_scales, residual, gate, nullptr, 0, 0, nullptr, 0, 0, stream);
 }
 
 extern "C" int wanmi_mxfp8_gemm_rowsumsq(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes,
@@ -1155,7 +1565,7 @@ extern "C" int wanmi_mxfp8_gemm_rowsumsq(const uint8_t* a_codes, const uint8_t* 
   WANMI_REQUIRE(sumsq_cols >= 0 && sumsq_cols <= N && sumsq_cols % 128 == 0, WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm_rowsumsq: sumsq_cols=%lld must be a multiple of 128 in [0, N]", (long long)sumsq_cols);
   return gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, N, K, lda, WANMI_EPI_BF16, out,
-                   ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, N / 128, nullptr, 0, stream);
+                   ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, N / 128, nullptr, 0, 0, stream);
 }
 
 extern "C" int wanmi_mxfp8_gemm_qkv(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes,
@@ -1178,13 +1588,24 @@ extern "C" int wanmi_mxfp8_gemm_qkv(const uint8_t* a_codes, const uint8_t* a_sca
   WANMI_REQUIRE(M > 0 && vt_ld <= (M + TM - 1) / TM * TM, WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm_qkv: M=%lld must be positive and vt_ld=%lld at most M rounded up to %d",
                 (long long)M, (long long)vt_ld, TM);
+  // In one launch where that saves a round of tiles (one latent frame, 1560 tokens: 172 -> 121 us); two
+  // launches otherwise (at 32760 tokens both parts are whole rounds).
+  if ((K / BK) % 4 == 0) {
+    const int cus = device_cu_count();
+    WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm_qkv: cannot query the device's compute units");
+    const int64_t apart = select_tile(M, vt_col0, cus, 0).cost + select_tile(M, N - vt_col0, cus, vt_ld).cost;
+    if (select_qkv_tile(M, vt_col0, N - vt_col0, cus, vt_ld).cost <= apart)
+      return gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, N, K, lda, kEpiQkv, out, ldo,
+                       nullptr, nullptr, nullptr, row_sumsq, row_sumsq ? sumsq_cols : 0, vt_col0 / 128, vt, vt_ld,
+                       vt_col0, stream);
+  }
   // Q | K: the plain bf16 epilogue (with the Q partial sums) on the weight rows [0, vt_col0)
   int st = gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, vt_col0, K, lda,
                      WANMI_EPI_BF16, out, ldo, nullptr, nullptr, nullptr, row_sumsq, row_sumsq ? sumsq_cols : 0,
-                     vt_col0 / 128, nullptr, 0, stream);
+                     vt_col0 / 128, nullptr, 0, 0, stream);
   if (st != WANMI_OK) return st;
   // V: the weight rows [vt_col0, N), transposed accumulator, V^T epilogue
   return gemm_impl(a_codes, a_scales, w_codes + vt_col0 * K, w_scales + vt_col0 * (K / 32), row_scale,
                    col_scale ? col_scale + vt_col0 : nullptr, bias ? bias + vt_col0 : nullptr, M, N - vt_col0, K, lda,
-                   kEpiVt, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0, 0, vt, vt_ld, stream);
+                   kEpiVt, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0, 0, vt, vt_ld, 0, stream);
 }
