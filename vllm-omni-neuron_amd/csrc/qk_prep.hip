@@ -273,6 +273,22 @@ __global__ void zero_f32_kernel(float* p, int n) {
   if (i < n) p[i] = 0.0f;
 }
 
+// Tokens each wave walks. A token is one latency chain (its row, the reduction, the fp64 root, the
+// write), so a wave's tokens are served one after another while other waves hide the latency: as many
+// waves as one round holds (four workgroups of four waves per CU, kQKWavesResident) come first, and
+// only a sequence longer than that gives a wave more than one token. At most 8: an S = 32760 launch is
+// then one resident round, and the gamma copy is shared by 32 tokens. With 8 tokens per wave
+// throughout, 512 / 1560 / 3600 tokens ran 34 / 43 / 47 us: 16 / 49 / 113 workgroups on 256 CUs, each
+// eight such chains long. One token per wave took 24 us off the first, 22 off the second, 21 off the
+// third (the block's cross-attention K/V 94 -> 69 us, row_mx_qkv_proj of 3600 tokens 387 -> 344).
+constexpr int64_t kQKWavesResident = 256 * 4 * 4;
+constexpr int kQKTokensPerWaveMax = 8;
+
+static int qk_tokens_per_wave(int64_t S) {
+  const int64_t n = (S + kQKWavesResident - 1) / kQKWavesResident;
+  return (int)(n < 1 ? 1 : n > kQKTokensPerWaveMax ? kQKTokensPerWaveMax : n);
+}
+
 struct TransposeArgs {
   const uint16_t* v;  // element (s, h, d) at v[s*ld + h*hs + d]
   int64_t S, ld, hs;
@@ -353,7 +369,7 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.ld = ld;
   a.heads = heads;
   a.nch = heads / 4;
-  a.tokens_per_wave = 8;
+  a.tokens_per_wave = qk_tokens_per_wave(S);
   a.gamma = gamma;
   a.cos = cos_tab;
   a.sin = sin_tab;
