@@ -20,6 +20,7 @@
 // Q fragments the MFMA consumes.
 #include "wanmi_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace wanmi {
@@ -87,6 +88,8 @@ struct AttnArgs {
   int heads_per_group;  // attention_head_group_kernel: consecutive heads per workgroup (divides heads)
   float* row_sum;       // optional: each query's row sum of P, [heads][Sq] (wanmi_attention_exact)
   const float* q_rr;    // optional (with q_gamma): each query's across-heads 1/rms [Sq], in place of q_sumsq
+  int whole_blocks;     // attention_split_kernel: blocks of BQ queries per head before the wave jobs
+  int job_waves;        // attention_split_kernel: waves per wave job (2, 4 or 8)
 };
 
 // LDS tiles, a ring of kStages (tile t in slot t % kStages):
@@ -182,91 +185,12 @@ __device__ __forceinline__ void pipeline_step(const uint8_t* cK, int i_cur, cons
   s_prev = s_cur;
 }
 
-// kShortKV: a separate instantiation for short key sequences (cross-attention over text tokens) so
-// the two uses can be specialized and profiled apart; it sums the bf16 P (see softmax_half).
-// kRebaseK: one head of K spans more than 2 GiB (the fused QKV layout, row stride 15360, at 720p), so
-// the K descriptor is rebuilt at each tile's first key; otherwise one descriptor covers the head and
-// the tile's offset travels in the wave-uniform soffset.
-template <bool kShortKV, bool kRebaseK>
-__global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs a) {
+// The wave's 32 queries (q0 + col) of head h as B operands: lane holds d = 16 t + 8 hq .. +7 of query
+// q0 + col in qf[t], pre-scaled by s log2(e), normalized and rotated first where the caller asks for
+// it. `sgam`: the wave's 1 KiB of LDS for the head's gamma. Returns the query's bound c in log2 units.
+__device__ __forceinline__ float load_queries(const AttnArgs& a, int h, int64_t q0, int lane, int col, int hq, float* sgam,
+                                              bf16x8 (&qf)[8]) {
 #pragma clang fp contract(off)
-  __shared__ __attribute__((aligned(16))) uint8_t sK[kStages][kTileK];
-  __shared__ __attribute__((aligned(16))) uint8_t sV[kStages][kTileV];
-  __shared__ __attribute__((aligned(16))) float sgam[kWaves][256];  // each wave's copy of the head's gamma
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Workgroups go to the 8 XCDs round-robin by linear index. With the heads a multiple of 8, XCD x
-  // takes heads x * heads/8 .. + heads/8 - 1 whole, query block after query block, so that all of
-  // its CUs stream the same head's K/V tiles through its L2 instead of every XCD fetching every head
-  // (the same (head, query block) pairs, each computed as before).
-  int hb = blockIdx.y, qb = blockIdx.x;
-  if ((gridDim.y & 7) == 0) {
-    const int nq = (int)gridDim.x;
-    const int L = (int)blockIdx.x + (int)blockIdx.y * nq;
-    const int k = L >> 3;
-    hb = (L & 7) * (int)(gridDim.y >> 3) + k / nq;
-    qb = k % nq;
-  }
-  const int h = hb;
-  const int64_t q0 = (int64_t)qb * BQ + wave * 32;
-  const int col = lane & 31;  // this lane's query within the wave's 32
-  const int hq = lane >> 5;
-
-  // Keys >= Sk fall outside the K descriptor's extent and read as zero. V^T ([128][vt_ld] per head,
-  // vt_ld >= Sk rounded up to 64) always fits one descriptor, and every tile lies inside it.
-  const uint16_t* k_head = a.k + h * a.k_hs;
-  const u32x4 r_k_head = buffer_rsrc(k_head, kRebaseK ? 0u : (uint32_t)(((a.Sk - 1) * a.k_ss + 128) * 2));
-  const u32x4 r_v = buffer_rsrc(a.vt + (int64_t)h * 128 * a.vt_ld, (uint32_t)(128 * a.vt_ld * 2));
-  // DMA lane mapping: each wave fills 8 K rows (4 per 1 KiB instruction) and 16 V^T rows (8 per
-  // instruction); lane l lands in physical chunk l & 15 (K) / l & 7 (V) of its row and fetches the
-  // logical chunk the XOR swizzle assigns to that slot. The loads are issued through inline asm
-  // (invisible to the compiler's wait-count pass, which would otherwise wait for the prefetches
-  // before every LDS read); the loop waits for them itself.
-  const int k_row = lane >> 4, k_pc = lane & 15;
-  const int v_row = lane >> 3, v_pc = lane & 7;
-  auto issue_tile_k = [&](int kt) {
-    const int b = kt % kStages;
-    const int64_t kbase = (int64_t)kt * BKV;
-    // The tile's key offset stays in the per-lane offset (soffset is not range-checked), so that
-    // keys >= Sk of the last tile read as zero.
-    u32x4 r_k = r_k_head;
-    int64_t key0 = kbase;
-    if constexpr (kRebaseK) {
-      const int64_t kvalid = a.Sk - kbase < BKV ? a.Sk - kbase : BKV;
-      r_k = buffer_rsrc(k_head + kbase * a.k_ss, (uint32_t)(((kvalid - 1) * a.k_ss + 128) * 2));
-      key0 = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int key = wave * 8 + i * 4 + k_row;
-      const int c = k_pc ^ (key & 15);
-      lds_dma_b128_hot(r_k, (uint32_t)(((key0 + key) * a.k_ss + c * 8) * 2), lds_addr(sK[b] + (wave * 8 + i * 4) * 256));
-    }
-  };
-  auto issue_tile_v = [&](int kt) {
-    const int b = kt % kStages;
-    const int64_t kbase = (int64_t)kt * BKV;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int d = wave * 16 + i * 8 + v_row;
-      const int c = v_pc ^ (d & 7) ^ ((d >> 3) & 1);
-      lds_dma_b128_hot(r_v, (uint32_t)((d * a.vt_ld + c * 8) * 2), (uint32_t)(kbase * 2),
-                       lds_addr(sV[b] + (wave * 16 + i * 8) * 128));
-    }
-  };
-  auto issue_tile = [&](int kt) {
-    issue_tile_k(kt);
-    issue_tile_v(kt);
-  };
-  const int ntiles = (int)((a.Sk + BKV - 1) / BKV);
-  // The first three tiles go out before anything else, so their latency overlaps the Q loads.
-  issue_tile(0);
-  if (ntiles > 1) issue_tile(1);
-  if (ntiles > 2) issue_tile(2);
-
-  // ---- Q fragments (B operand): lane holds d = 16t + 8hq .. +7 of query q0 + col, t = 0..7 ----
   // Q through a descriptor based at the wave's first query; rows >= Sq read as zero.
   const int64_t qvalid = a.Sq - q0 < 32 ? (a.Sq - q0 > 0 ? a.Sq - q0 : 0) : 32;
   const __amdgpu_buffer_rsrc_t r_q =
@@ -280,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs 
   // The head's gamma (128 floats, the same for every query) goes to LDS, one copy per wave so that no
   // barrier is needed before the wave reads it; read per lane from L2 it was 16 loads of 1 KiB per
   // wave through the texture unit, more than the wave's Q itself.
-  if (qprep) lds_dma_b128(buffer_rsrc(a.q_gamma + h * 128, 128 * 4), (uint32_t)lane * 16, lds_addr(sgam[wave]));
+  if (qprep) lds_dma_b128(buffer_rsrc(a.q_gamma + h * 128, 128 * 4), (uint32_t)lane * 16, lds_addr(sgam));
   const __amdgpu_buffer_rsrc_t r_cs =
       attn_rsrc(qrope ? a.q_cos + (qvalid > 0 ? q0 * 64 : 0) : nullptr, qrope && qvalid > 0 ? qvalid * 64 * 4 : 0);
   const __amdgpu_buffer_rsrc_t r_sn =
@@ -347,7 +271,7 @@ __global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs 
     }
     // every load of the prologue is in (the math below needs them all), the gamma copy included
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    const float4* gl = reinterpret_cast<const float4*>(sgam[wave]);
+    const float4* gl = reinterpret_cast<const float4*>(sgam);
     // x_hat = bf16((x rrms) gamma), then the pair rotation (a cos - b sin, a sin + b cos) -> bf16:
     // the same operations, in the same order, as the separate Q/K preparation pass
 #pragma unroll
@@ -369,7 +293,6 @@ __global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs 
       }
     }
   }
-  bf16x8 qf[8];
   float qn2 = 0.0f;
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
@@ -388,7 +311,152 @@ __global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs 
   }
   qn2 = qn2 + __shfl_xor(qn2, 32, 64);
   // c_i in log2 units: s * ||q_i|| * max||k|| * log2(e), from the unscaled bf16 Q
-  const float c2 = a.scale_log2 * sqrtf(qn2) * a.kmax[h];
+  return a.scale_log2 * sqrtf(qn2) * a.kmax[h];
+}
+
+// Normalizes the wave's O^T accumulators by the row sum (lsum: this lane's half of its query's keys)
+// and writes them in the caller's layout. `stg`: 4 KiB of LDS that no other wave touches any more.
+__device__ __forceinline__ void store_queries(const AttnArgs& a, int h, int64_t q0, int lane, int col, int hq,
+                                              const f32x16 (&acc_o)[4], float lsum, uint8_t* stg) {
+#pragma clang fp contract(off)
+  lsum = lsum + __shfl_xor(lsum, 32, 64);
+  const float inv = 1.0f / fmaxf(lsum, kSumFloor);
+  const int64_t qi = q0 + col;
+  const bool qok = qi < a.Sq;
+  if (a.row_sum != nullptr && qok && hq == 0) a.row_sum[(int64_t)h * a.Sq + qi] = lsum;
+  if (a.out_mode == WANMI_ATTN_OUT_TOKEN) {
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + h * a.o_hs + qi * a.o_ss;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi) {
+        const int d = dt * 32 + gi * 8 + hq * 4;
+        const float v0 = acc_o[dt][gi * 4] * inv, v1 = acc_o[dt][gi * 4 + 1] * inv;
+        const float v2 = acc_o[dt][gi * 4 + 2] * inv, v3 = acc_o[dt][gi * 4 + 3] * inv;
+        if (qok) *reinterpret_cast<uint2*>(out + d) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+      }
+  } else if (a.out_mode == WANMI_ATTN_OUT_DMAJOR) {
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + h * a.o_hs + qi;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int d = dt * 32 + (r >> 2) * 8 + hq * 4 + (r & 3);
+        if (qok) out[d * a.o_ds] = (uint16_t)(pack_bf16x2(acc_o[dt][r] * inv, 0.0f) & 0xFFFFu);
+      }
+  } else {  // MX codes, token-major; a 32-wide block of d is one d tile, split between lane and lane^32
+    // Each wave's 32 query rows (128 code bytes each) are staged in LDS and written as whole rows,
+    // 16 bytes per lane; written straight from the accumulator layout every store instruction would
+    // touch 32 rows with 4 bytes each. 16-byte chunks are XOR-swizzled by the row so that the writes
+    // and the row reads spread over the banks. A query's four scale bytes (d tiles 0-3) go out as one
+    // word.
+    uint32_t sw = 0;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      // bf16 pairs; the block's largest exponent field is that of the largest (bits & 0x7fff)
+      uint32_t pp[8];
+      u16x2_t mag = {0, 0};
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        pp[r / 2] = pack_bf16x2(acc_o[dt][r] * inv, acc_o[dt][r + 1] * inv);
+        mag = __builtin_elementwise_max(mag, __builtin_bit_cast(u16x2_t, pp[r / 2] & 0x7FFF7FFFu));
+      }
+      int e = (int)(max(mag[0], mag[1]) >> 7);
+      e = max_with_lane_xor32(e);
+      const int sx = max(e - 7, 0);
+      const float sc = __uint_as_float((uint32_t)sx << 23);
+      sw |= (uint32_t)sx << (8 * dt);
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi) {
+        const int d = dt * 32 + gi * 8 + hq * 4;
+        const uint32_t c4 = cvt_e4m3x4_scaled(pp[2 * gi], pp[2 * gi + 1], sc);
+        *reinterpret_cast<uint32_t*>(stg + col * 128 + ((((d >> 4) ^ (col & 7)) << 4) | (d & 15))) = c4;
+      }
+    }
+    // the MX rows and scales non-temporal, as the GEMMs' outputs (cross-attention 443.6 -> 429.7 us
+    // with the caches flushed between launches)
+    if (qok && hq == 0) __builtin_nontemporal_store(sw, reinterpret_cast<uint32_t*>(a.out_scales + qi * a.os_ss + h * 4));
+    uint8_t* out = reinterpret_cast<uint8_t*>(a.out) + h * a.o_hs;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int qr = it * 8 + (lane >> 3), ch = lane & 7;
+      const uint4 v = *reinterpret_cast<const uint4*>(stg + qr * 128 + ((ch ^ (qr & 7)) << 4));
+      const int64_t qg = q0 + qr;
+      if (qg < a.Sq) __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(&v), reinterpret_cast<u32x4*>(out + qg * a.o_ss + ch * 16));
+    }
+  }
+}
+
+// kShortKV: a separate instantiation for short key sequences (cross-attention over text tokens) so
+// the two uses can be specialized and profiled apart; it sums the bf16 P (see softmax_half).
+// kRebaseK: one head of K spans more than 2 GiB (the fused QKV layout, row stride 15360, at 720p), so
+// the K descriptor is rebuilt at each tile's first key; otherwise one descriptor covers the head and
+// the tile's offset travels in the wave-uniform soffset.
+template <bool kShortKV, bool kRebaseK>
+__device__ __forceinline__ void attention_block(const AttnArgs& a, int h, int qb, uint8_t (&sK)[kStages][kTileK],
+                                                uint8_t (&sV)[kStages][kTileV], float (&sgam)[kWaves][256]) {
+#pragma clang fp contract(off)
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t q0 = (int64_t)qb * BQ + wave * 32;
+  const int col = lane & 31;  // this lane's query within the wave's 32
+  const int hq = lane >> 5;
+
+  // Keys >= Sk fall outside the K descriptor's extent and read as zero. V^T ([128][vt_ld] per head,
+  // vt_ld >= Sk rounded up to 64) always fits one descriptor, and every tile lies inside it.
+  const uint16_t* k_head = a.k + h * a.k_hs;
+  const u32x4 r_k_head = buffer_rsrc(k_head, kRebaseK ? 0u : (uint32_t)(((a.Sk - 1) * a.k_ss + 128) * 2));
+  const u32x4 r_v = buffer_rsrc(a.vt + (int64_t)h * 128 * a.vt_ld, (uint32_t)(128 * a.vt_ld * 2));
+  // DMA lane mapping: each wave fills 8 K rows (4 per 1 KiB instruction) and 16 V^T rows (8 per
+  // instruction); lane l lands in physical chunk l & 15 (K) / l & 7 (V) of its row and fetches the
+  // logical chunk the XOR swizzle assigns to that slot. The loads are issued through inline asm
+  // (invisible to the compiler's wait-count pass, which would otherwise wait for the prefetches
+  // before every LDS read); the loop waits for them itself.
+  const int k_row = lane >> 4, k_pc = lane & 15;
+  const int v_row = lane >> 3, v_pc = lane & 7;
+  auto issue_tile_k = [&](int kt) {
+    const int b = kt % kStages;
+    const int64_t kbase = (int64_t)kt * BKV;
+    // The tile's key offset stays in the per-lane offset (soffset is not range-checked), so that
+    // keys >= Sk of the last tile read as zero.
+    u32x4 r_k = r_k_head;
+    int64_t key0 = kbase;
+    if constexpr (kRebaseK) {
+      const int64_t kvalid = a.Sk - kbase < BKV ? a.Sk - kbase : BKV;
+      r_k = buffer_rsrc(k_head + kbase * a.k_ss, (uint32_t)(((kvalid - 1) * a.k_ss + 128) * 2));
+      key0 = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int key = wave * 8 + i * 4 + k_row;
+      const int c = k_pc ^ (key & 15);
+      lds_dma_b128_hot(r_k, (uint32_t)(((key0 + key) * a.k_ss + c * 8) * 2), lds_addr(sK[b] + (wave * 8 + i * 4) * 256));
+    }
+  };
+  auto issue_tile_v = [&](int kt) {
+    const int b = kt % kStages;
+    const int64_t kbase = (int64_t)kt * BKV;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int d = wave * 16 + i * 8 + v_row;
+      const int c = v_pc ^ (d & 7) ^ ((d >> 3) & 1);
+      lds_dma_b128_hot(r_v, (uint32_t)((d * a.vt_ld + c * 8) * 2), (uint32_t)(kbase * 2),
+                       lds_addr(sV[b] + (wave * 16 + i * 8) * 128));
+    }
+  };
+  auto issue_tile = [&](int kt) {
+    issue_tile_k(kt);
+    issue_tile_v(kt);
+  };
+  const int ntiles = (int)((a.Sk + BKV - 1) / BKV);
+  // The first three tiles go out before anything else, so their latency overlaps the Q loads.
+  issue_tile(0);
+  if (ntiles > 1) issue_tile(1);
+  if (ntiles > 2) issue_tile(2);
+
+  bf16x8 qf[8];
+  const float c2 = load_queries(a, h, q0, lane, col, hq, sgam[wave], qf);
   f32x16 negc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) negc[r] = -c2;
@@ -451,75 +519,195 @@ __global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs 
     pv_half(sV[(ntiles - 1) % kStages], 1, pf, acc_o, col, hq);
   }
 
-  // ---- normalize and store ----
-  lsum = lsum + __shfl_xor(lsum, 32, 64);
-  const float inv = 1.0f / fmaxf(lsum, kSumFloor);
-  const int64_t qi = q0 + col;
-  const bool qok = qi < a.Sq;
-  if (a.row_sum != nullptr && qok && hq == 0) a.row_sum[(int64_t)h * a.Sq + qi] = lsum;
-  if (a.out_mode == WANMI_ATTN_OUT_TOKEN) {
-    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + h * a.o_hs + qi * a.o_ss;
+  // MX rows are staged in the slot of tile ntiles - 3 (or one never filled), which no wave reads after
+  // the last tile's barrier
+  store_queries(a, h, q0, lane, col, hq, acc_o, lsum,
+                (wave < 4 ? sK[(ntiles + 1) % kStages] : sV[(ntiles + 1) % kStages]) + (wave & 3) * 4096);
+}
+
+template <bool kShortKV, bool kRebaseK>
+__global__ __launch_bounds__(kThreads) void attention_const_max_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t sK[kStages][kTileK];
+  __shared__ __attribute__((aligned(16))) uint8_t sV[kStages][kTileV];
+  __shared__ __attribute__((aligned(16))) float sgam[kWaves][256];  // each wave's copy of the head's gamma
+
+  // Workgroups go to the 8 XCDs round-robin by linear index. With the heads a multiple of 8, XCD x
+  // takes heads x * heads/8 .. + heads/8 - 1 whole, query block after query block, so that all of
+  // its CUs stream the same head's K/V tiles through its L2 instead of every XCD fetching every head
+  // (the same (head, query block) pairs, each computed as before).
+  int hb = blockIdx.y, qb = blockIdx.x;
+  if ((gridDim.y & 7) == 0) {
+    const int nq = (int)gridDim.x;
+    const int L = (int)blockIdx.x + (int)blockIdx.y * nq;
+    const int k = L >> 3;
+    hb = (L & 7) * (int)(gridDim.y >> 3) + k / nq;
+    qb = k % nq;
+  }
+  attention_block<kShortKV, kRebaseK>(a, hb, qb, sK, sV, sgam);
+}
+
+// The sums of waves that share 32 queries: the bound does not depend on the keys a wave saw, so their row
+// sums and O accumulators simply add up, in fp32 and in the waves' order. Every wave but the first
+// leaves its own in LDS (16 KiB of `mine`, lane-major, and its row of sgam).
+__device__ __forceinline__ void leave_partial(uint8_t* mine, float* sgam, const f32x16 (&acc_o)[4], float lsum, int lane) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int gi = 0; gi < 4; ++gi) {
-        const int d = dt * 32 + gi * 8 + hq * 4;
-        const float v0 = acc_o[dt][gi * 4] * inv, v1 = acc_o[dt][gi * 4 + 1] * inv;
-        const float v2 = acc_o[dt][gi * 4 + 2] * inv, v3 = acc_o[dt][gi * 4 + 3] * inv;
-        if (qok) *reinterpret_cast<uint2*>(out + d) = make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
-      }
-  } else if (a.out_mode == WANMI_ATTN_OUT_DMAJOR) {
-    uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + h * a.o_hs + qi;
+    for (int g = 0; g < 4; ++g)
+      reinterpret_cast<float4*>(mine)[(i * 4 + g) * 64 + lane] =
+          make_float4(acc_o[i][4 * g], acc_o[i][4 * g + 1], acc_o[i][4 * g + 2], acc_o[i][4 * g + 3]);
+  sgam[lane] = lsum;
+}
+__device__ __forceinline__ void add_partial(const uint8_t* other, const float* sgam, f32x16 (&acc_o)[4], float& lsum, int lane) {
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+  for (int i = 0; i < 4; ++i) {
+    __builtin_amdgcn_sched_barrier(0);  // four reads at a time: hoisted together they spill
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int d = dt * 32 + (r >> 2) * 8 + hq * 4 + (r & 3);
-        if (qok) out[d * a.o_ds] = (uint16_t)(pack_bf16x2(acc_o[dt][r] * inv, 0.0f) & 0xFFFFu);
-      }
-  } else {  // MX codes, token-major; a 32-wide block of d is one d tile, split between lane and lane^32
-    // Each wave's 32 query rows (128 code bytes each) are staged in LDS and written as whole rows,
-    // 16 bytes per lane; written straight from the accumulator layout every store instruction would
-    // touch 32 rows with 4 bytes each. The staging slot is that of tile ntiles - 3 (or one never
-    // filled), which no wave reads after the last tile's barrier; 16-byte chunks are XOR-swizzled by
-    // the row so that the writes and the row reads spread over the banks. A query's four scale bytes
-    // (d tiles 0-3) go out as one word.
-    uint8_t* stg = (wave < 4 ? sK[(ntiles + 1) % kStages] : sV[(ntiles + 1) % kStages]) + (wave & 3) * 4096;
-    uint32_t sw = 0;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      // bf16 pairs; the block's largest exponent field is that of the largest (bits & 0x7fff)
-      uint32_t pp[8];
-      u16x2_t mag = {0, 0};
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        pp[r / 2] = pack_bf16x2(acc_o[dt][r] * inv, acc_o[dt][r + 1] * inv);
-        mag = __builtin_elementwise_max(mag, __builtin_bit_cast(u16x2_t, pp[r / 2] & 0x7FFF7FFFu));
-      }
-      int e = (int)(max(mag[0], mag[1]) >> 7);
-      e = max_with_lane_xor32(e);
-      const int sx = max(e - 7, 0);
-      const float sc = __uint_as_float((uint32_t)sx << 23);
-      sw |= (uint32_t)sx << (8 * dt);
-#pragma unroll
-      for (int gi = 0; gi < 4; ++gi) {
-        const int d = dt * 32 + gi * 8 + hq * 4;
-        const uint32_t c4 = cvt_e4m3x4_scaled(pp[2 * gi], pp[2 * gi + 1], sc);
-        *reinterpret_cast<uint32_t*>(stg + col * 128 + ((((d >> 4) ^ (col & 7)) << 4) | (d & 15))) = c4;
-      }
-    }
-    // the MX rows and scales non-temporal, as the GEMMs' outputs (cross-attention 443.6 -> 429.7 us
-    // with the caches flushed between launches)
-    if (qok && hq == 0) __builtin_nontemporal_store(sw, reinterpret_cast<uint32_t*>(a.out_scales + qi * a.os_ss + h * 4));
-    uint8_t* out = reinterpret_cast<uint8_t*>(a.out) + h * a.o_hs;
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int qr = it * 8 + (lane >> 3), ch = lane & 7;
-      const uint4 v = *reinterpret_cast<const uint4*>(stg + qr * 128 + ((ch ^ (qr & 7)) << 4));
-      const int64_t qg = q0 + qr;
-      if (qg < a.Sq) __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(&v), reinterpret_cast<u32x4*>(out + qg * a.o_ss + ch * 16));
+    for (int g = 0; g < 4; ++g) {
+      const float4 v = reinterpret_cast<const float4*>(other)[(i * 4 + g) * 64 + lane];
+      acc_o[i][4 * g] = acc_o[i][4 * g] + v.x;
+      acc_o[i][4 * g + 1] = acc_o[i][4 * g + 1] + v.y;
+      acc_o[i][4 * g + 2] = acc_o[i][4 * g + 2] + v.z;
+      acc_o[i][4 * g + 3] = acc_o[i][4 * g + 3] + v.w;
     }
   }
+  lsum = lsum + sgam[lane];
+}
+
+// Wave jobs: 32 queries of one head each, a.job_waves waves of the workgroup taking every job_waves-th
+// 32-key half. For the few queries behind the last whole block of each head: a workgroup serves
+// 8 / job_waves of them (of different heads where a head has one), and each wave streams its own keys
+// through its own 16 KiB of LDS (K of one half, V^T of one half: the next half's K is requested once
+// this half's K is in registers, and likewise V^T), without a barrier until the sums are added. Bound by
+// that stream: nothing is shared between waves, so the operand traffic per MFMA is eight times a whole
+// block's, and a workgroup takes 2.6 / job_waves of a block's time per key tile. 1560 queries and keys,
+// 40 heads (240 blocks, 40 remainders of 24 queries): 81.3 us in blocks throughout (a second round for
+// the remainders), 55.0 with two waves per job, 65.9 with four, 67.5 with eight; 512 keys: 40.1 -> 24.1.
+// Splitting the keys of 128-query runs over two groups of waves that share tiles (98.9 against 103.9 us
+// at 2048, 252 against 259 at 3600) gained too little to stay.
+template <bool kShortKV>
+__device__ __forceinline__ void attention_wave_jobs(const AttnArgs& a, int L, uint8_t (&sK)[kStages][kTileK],
+                                                    uint8_t (&sV)[kStages][kTileV], float (&sgam)[kWaves][256]) {
+#pragma clang fp contract(off)
+  static_assert(kStages == 4 && kWaves == 8 && kTileK == 16384 && kTileV == 16384);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31;
+  const int hq = lane >> 5;
+  const int64_t q_base = (int64_t)a.whole_blocks * BQ;
+  const int tiles = (int)((a.Sq - q_base + 31) / 32);  // jobs per head
+  const int groups = (a.heads & 7) == 0 ? 8 : 1;       // an XCD's jobs are those of its own heads / 8 heads
+  const int job = (L / groups) * (kWaves / a.job_waves) + wave / a.job_waves;
+  const int part = wave % a.job_waves;
+  const bool active = job < tiles * (a.heads / groups);
+  const int h = active ? (L % groups) * (a.heads / groups) + job / tiles : 0;
+  const int64_t q0 = q_base + (int64_t)(active ? job % tiles : 0) * 32;
+  uint8_t* buf = wave < 4 ? sK[wave & 3] : sV[wave & 3];
+  uint8_t *kb = buf, *vb = buf + 8192;
+
+  f32x16 acc_o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc_o[i][r] = 0.0f;
+  float lsum = 0.0f;
+  const int halves = (int)((a.Sk + 31) / 32);
+  if (active && part < halves) {
+    const u32x4 r_k = buffer_rsrc(a.k + h * a.k_hs, (uint32_t)(((a.Sk - 1) * a.k_ss + 128) * 2));
+    const u32x4 r_v = buffer_rsrc(a.vt + (int64_t)h * 128 * a.vt_ld, (uint32_t)(128 * a.vt_ld * 2));
+    // K half: 32 keys of 256 bytes as in a K tile (4 keys per instruction). V^T half: 128 rows of 64
+    // bytes (16 rows per instruction), 16-byte chunk index XOR ((d >> 2) & 3): the 16 rows an LDS cycle
+    // serves take all 64 banks.
+    auto issue_k = [&](int half) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = i * 4 + (lane >> 4);
+        const int c = (lane & 15) ^ (key & 15);
+        lds_dma_b128(r_k, (uint32_t)((((int64_t)half * 32 + key) * a.k_ss + c * 8) * 2), lds_addr(kb + i * 1024));
+      }
+    };
+    auto issue_v = [&](int half) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int d = i * 16 + (lane >> 2);
+        const int c = (lane & 3) ^ ((d >> 2) & 3);
+        lds_dma_b128(r_v, (uint32_t)((d * a.vt_ld + c * 8) * 2), (uint32_t)(half * 64), lds_addr(vb + i * 1024));
+      }
+    };
+    issue_k(part);
+    issue_v(part);
+    bf16x8 qf[8];
+    const float c2 = load_queries(a, h, q0, lane, col, hq, sgam[wave], qf);
+    f32x16 negc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) negc[r] = -c2;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int half = part; half < halves; half += a.job_waves) {
+      const bool more = half + a.job_waves < halves;  // wave-uniform
+      // K of this half is in: behind it only V^T of this half (eight loads) may be outstanding
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      bf16x8 kf[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) kf[t] = *reinterpret_cast<const bf16x8*>(kb + sk_off(col, 2 * t + hq));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: its buffer is free
+      if (more) issue_k(half + a.job_waves);
+      f32x16 s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], negc, 0, 0, 0);
+#pragma unroll
+      for (int t = 1; t < 8; ++t) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t], qf[t], s, 0, 0, 0);
+      bf16x8 pf[2];
+      softmax_half<true, kShortKV>(s, hq, (int)(a.Sk - (int64_t)half * 32), lsum, pf);
+      if (more)
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // V^T of this half, not the next half's K
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      bf16x8 vf[2][4];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          const int d = dt * 32 + col;
+          vf[u][dt] = *reinterpret_cast<const bf16x8*>(vb + d * 64 + (((2 * u + hq) ^ ((d >> 2) & 3)) << 4));
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (more) issue_v(half + a.job_waves);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+          acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u][dt], pf[u], acc_o[dt], 0, 0, 0);
+    }
+  }
+  if (part > 0) leave_partial(buf, sgam[wave], acc_o, lsum, lane);
+  __syncthreads();
+  if (part > 0 || !active) return;
+  for (int o = 1; o < a.job_waves; ++o) {
+    const int w = wave + o;
+    add_partial(w < 4 ? sK[w & 3] : sV[w & 3], sgam[w], acc_o, lsum, lane);
+  }
+  store_queries(a, h, q0, lane, col, hq, acc_o, lsum, buf);
+}
+
+// Whole blocks and wave jobs in one launch: the first heads * whole_blocks workgroups take the blocks of
+// the first whole_blocks * BQ queries of every head, the others the queries behind them. Blocks first, so
+// that the jobs fill the CUs that the last round of blocks leaves idle.
+template <bool kShortKV>
+__global__ __launch_bounds__(kThreads) void attention_split_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t sK[kStages][kTileK];
+  __shared__ __attribute__((aligned(16))) uint8_t sV[kStages][kTileV];
+  __shared__ __attribute__((aligned(16))) float sgam[kWaves][256];
+  const int L = blockIdx.x, whole = a.whole_blocks * a.heads;
+  if (L >= whole) {
+    attention_wave_jobs<kShortKV>(a, L - whole, sK, sV, sgam);
+    return;
+  }
+  int h = L / a.whole_blocks, b = L % a.whole_blocks;
+  if ((a.heads & 7) == 0) {  // an XCD takes heads / 8 heads whole, as in attention_const_max_kernel
+    const int k = L >> 3;
+    h = (L & 7) * (a.heads >> 3) + k / a.whole_blocks;
+    b = k % a.whole_blocks;
+  }
+  attention_block<kShortKV, false>(a, h, b, sK, sV, sgam);
 }
 
 // Several heads per workgroup, for short key sequences (cross-attention over the text tokens): with
@@ -1102,6 +1290,75 @@ struct QPrep {
   float eps = 0.0f;
 };
 
+static int cu_count() {
+  const int cus = device_cu_count();
+  return cus > 0 ? cus : 256;
+}
+
+// How a launch covers Sq queries. Costs are in hundredths of a whole block's time per key tile.
+struct AttnPlan {
+  int whole_blocks;    // blocks of BQ queries per head; behind them, if jobs > 0,
+  int job_waves;       // wave jobs of this many waves,
+  int64_t jobs;        // in this many workgroups (attention_split_kernel)
+  int heads_per_group; // more than 1: attention_head_group_kernel
+  int64_t cost;
+};
+
+// A workgroup's cost, a fixed part (the queries' load and preparation, the first tiles, the output) and
+// a part per key tile, fitted to launches of 40 heads over 512 to 32760 queries: about 1.6 us per tile.
+constexpr int64_t kBlockFixed = 700, kBlockTile = 100;
+constexpr int64_t kJobFixed = 500, kJobTile = 260;                       // kJobTile / job_waves per tile
+constexpr int64_t kGroupFixed = 400, kGroupHead = 300, kGroupTile = 100;  // per head, per head and tile
+
+// When every CU takes one workgroup at a time in grid order (blocks, then jobs), the time at which the
+// last one ends.
+static int64_t attention_makespan(int64_t blocks, int64_t block, int64_t jobs, int64_t job, int64_t cus) {
+  const int64_t rounds = blocks / cus, late = blocks % cus;
+  // the CUs without a block in the last round are free from t_early on, the others a block later
+  int64_t t_early = rounds * block, t_late = t_early + block, last = late > 0 ? t_late : t_early;
+  while (jobs > 0) {
+    if (late == 0 || t_early <= t_late) {
+      t_early += job;
+      jobs -= cus - late;
+      last = std::max(last, t_early);
+    } else {
+      t_late += job;
+      jobs -= late;
+      last = std::max(last, t_late);
+    }
+  }
+  return last;
+}
+
+// Blocks throughout, unless the blocks' remainders (Sq not a multiple of BQ) would open a round of their
+// own that wave jobs in the idle CUs save. 40 heads over 1560 queries: above. No gain within a round:
+// 3600 queries (600 blocks in three rounds) 259.4 us in blocks, 264.2 with jobs. (Eight waves per job would
+// pay only where the jobs of all heads fit the idle CUs, and then the blocks in their place do too.)
+// Short key sequences (`group_heads`: the divisor that cross_heads_per_group picked): the head groups
+// where their rounds cost less, which takes about 5 heads per group. 512 keys, groups against blocks (jobs
+// at 1560): 36.2 / 21.7 us at 512 queries, 40.1 / 24.1 at 1560, 69.4 / 59.9 at 3600, 98.5 / 106.5 at
+// 7800, 401 / 444 at 32760.
+static AttnPlan attention_plan(int64_t Sq, int64_t Sk, int heads, int64_t cus, int group_heads) {
+  const int64_t tiles = (Sk + BKV - 1) / BKV, blocks = (Sq + BQ - 1) / BQ, full = Sq / BQ;
+  const int64_t block = kBlockFixed + kBlockTile * tiles;
+  AttnPlan best{0, 0, 0, 1, attention_makespan(blocks * heads, block, 0, 0, cus)};
+  if (full > 0 && Sq > full * BQ) {
+    const int64_t groups = heads % 8 == 0 ? 8 : 1;  // as attention_wave_jobs deals them to the XCDs
+    const int64_t per_group = (Sq - full * BQ + 31) / 32 * (heads / groups);
+    for (int waves = 2; waves <= 4; waves *= 2) {
+      const int64_t per = kWaves / waves, jobs = (per_group + per - 1) / per * groups;
+      const int64_t cost = attention_makespan(full * heads, block, jobs, kJobFixed + kJobTile * tiles / waves, cus);
+      if (cost < best.cost) best = AttnPlan{(int)full, waves, jobs, 1, cost};
+    }
+  }
+  if (group_heads > 1) {
+    const int64_t group = kGroupFixed + group_heads * (kGroupHead + kGroupTile * tiles);
+    const int64_t cost = attention_makespan(blocks * (heads / group_heads), group, 0, 0, cus);
+    if (cost < best.cost) best = AttnPlan{0, 0, 0, group_heads, cost};
+  }
+  return best;
+}
+
 static int attention_impl(const void* q, int64_t q_head_stride, int64_t q_token_stride, const void* k,
                           int64_t k_head_stride, int64_t k_token_stride, const void* vt, int64_t vt_ld,
                           const float* kmax, int64_t Sq, int64_t Sk, int heads, int head_dim, float scale,
@@ -1166,27 +1423,35 @@ static int attention_impl(const void* q, int64_t q_head_stride, int64_t q_token_
   a.row_sum = row_sum;
   const dim3 grid((unsigned)((Sq + BQ - 1) / BQ), (unsigned)heads);
   const bool rebase_k = ((Sk - 1) * k_token_stride + 128) * 2 >= (1LL << 31);
-  // Short key sequences of three tiles or more with queries that take no RoPE (cross-attention):
-  // several heads per workgroup (cross_heads_per_group; one head per workgroup when `heads` has no
-  // divisor from 2 up).
-  int hpw = 1;
-  if (Sk <= 1024 && Sk > 2 * BKV && qp.cos == nullptr && !rebase_k) {
-    const int cus = device_cu_count();
-    hpw = cross_heads_per_group((int64_t)grid.x, heads, cus > 0 ? cus : 256);
-  }
-  a.heads_per_group = hpw;
-  if (hpw > 1)
-    hipLaunchKernelGGL(attention_head_group_kernel, dim3(grid.x, (unsigned)(heads / hpw)), dim3(kThreads), 0,
-                       (hipStream_t)stream, a);
-  else if (Sk <= 1024)
+  // Short key sequences of three tiles or more with queries that take no RoPE (cross-attention) may run
+  // several heads per workgroup.
+  const bool short_kv = Sk <= 1024;
+  const int cus = cu_count();
+  const int group_heads =
+      short_kv && Sk > 2 * BKV && qp.cos == nullptr && !rebase_k ? cross_heads_per_group((int64_t)grid.x, heads, cus) : 1;
+  const AttnPlan plan = rebase_k ? AttnPlan{0, 0, 0, 1, 0} : attention_plan(Sq, Sk, heads, cus, group_heads);
+  a.heads_per_group = plan.heads_per_group;
+  if (plan.heads_per_group > 1) {
+    hipLaunchKernelGGL(attention_head_group_kernel, dim3(grid.x, (unsigned)(heads / plan.heads_per_group)), dim3(kThreads),
+                       0, (hipStream_t)stream, a);
+  } else if (plan.jobs > 0) {
+    a.whole_blocks = plan.whole_blocks;
+    a.job_waves = plan.job_waves;
+    const dim3 sgrid((unsigned)(heads * plan.whole_blocks + plan.jobs));
+    if (short_kv)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_split_kernel<true>), sgrid, dim3(kThreads), 0, (hipStream_t)stream, a);
+    else
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_split_kernel<false>), sgrid, dim3(kThreads), 0, (hipStream_t)stream, a);
+  } else if (short_kv) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_const_max_kernel<true, false>), grid, dim3(kThreads), 0,
                        (hipStream_t)stream, a);
-  else if (!rebase_k)
+  } else if (!rebase_k) {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_const_max_kernel<false, false>), grid, dim3(kThreads), 0,
                        (hipStream_t)stream, a);
-  else
+  } else {
     hipLaunchKernelGGL(HIP_KERNEL_NAME(attention_const_max_kernel<false, true>), grid, dim3(kThreads), 0,
                        (hipStream_t)stream, a);
+  }
   return check_launch("wanmi_attention_const_max");
 }
 }  // namespace wanmi
