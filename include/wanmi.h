@@ -304,6 +304,14 @@ int wanmi_qk_rmsnorm_rope_to(const void* x, int64_t S, int64_t ld, int heads, co
                              int64_t out_head_stride, void* stream);
 
 /*
+ * The reference's packed rows -> the GEMM's operands, one pass: row t of `packed` (ld bytes apart, 4-byte
+ * aligned, ld a multiple of 4) holds K e4m3 codes and the row's fp32 dequant scale (row_mx_kernels.py:12-45);
+ * codes [T, K], neutral block scales (2^0) [T, K/32] and row_scale [T] take them apart. K a multiple of 32.
+ */
+int wanmi_row_unpack(const void* packed, int64_t T, int64_t K, int64_t ld, void* codes, uint8_t* scales,
+                     float* row_scale, void* stream);
+
+/*
  * d-major bf16 attention output -> token-major MX activation, one pass: x holds element (b, n, d, s)
  * at x[b*b_stride + n*h_stride + d*d_stride + s] (d < 128); codes [B*S, heads*128] e4m3fn and scales
  * [B*S, heads*4] e8m0 (one per 32 consecutive channels, the adaLN kernel's MX rule), the layout

@@ -100,10 +100,19 @@ def packed_weight_to_mx(weight: torch.Tensor, weight_scales: torch.Tensor | None
 def _split_row_packed(packed: torch.Tensor):
     """Reference ROW-packed ``[T, K + 4]`` -> (codes [T, K], neutral scales, row scale [T])."""
     raw = packed.view(torch.uint8)
-    K = raw.shape[-1] - 4
-    codes = raw[:, :K].contiguous()
-    row_scale = raw[:, K:].contiguous().view(torch.float32).reshape(-1)
-    scales = torch.full((raw.shape[0], K // 32), _NEUTRAL_SCALE, dtype=torch.uint8, device=raw.device)
+    T, K = raw.shape[0], raw.shape[1] - 4
+    if raw.device.type != "cuda":  # for the callers' shape checks; their launches refuse host tensors
+        row_scale = raw[:, K:].contiguous().view(torch.float32).reshape(-1)
+        return raw[:, :K].contiguous(), torch.full((T, K // 32), _NEUTRAL_SCALE, dtype=torch.uint8), row_scale
+    ld = raw.stride(0) if T > 1 else K + 4
+    if raw.stride(1) != 1 or ld % 4 or ld < K + 4 or raw.data_ptr() % 4:  # the kernel reads whole 4-byte words
+        raw, ld = raw.clone(memory_format=torch.contiguous_format), K + 4
+    codes = torch.empty((T, K), dtype=torch.uint8, device=raw.device)
+    scales = torch.empty((T, K // 32), dtype=torch.uint8, device=raw.device)
+    row_scale = torch.empty(T, dtype=torch.float32, device=raw.device)
+    if T:
+        _lib.check(_lib.load().wanmi_row_unpack(_lib.ptr(raw), T, K, ld, _lib.ptr(codes), _lib.ptr(scales),
+                                                _lib.ptr(row_scale), _lib.stream_of(raw)), "wanmi_row_unpack")
     return codes, scales, row_scale
 
 
