@@ -304,6 +304,18 @@ int wanmi_qk_rmsnorm_rope_to(const void* x, int64_t S, int64_t ld, int heads, co
                              int64_t out_head_stride, void* stream);
 
 /*
+ * wanmi_qk_rmsnorm_rope on two parts of every row in one launch: Q at columns [0, heads*128) with gamma_q and
+ * K, k_offset columns on, with gamma_k (each its own across-heads norm; the same rotation). The tables'
+ * rows are tab_ld floats apart (a multiple of 4, at least 64: the first halves of rotate-half caches can
+ * be read in place). `out` null: in place; otherwise as wanmi_qk_rmsnorm_rope_to, K's heads
+ * out_k_offset elements after Q's (heads <= 40). Bits as two calls.
+ */
+int wanmi_qk_rmsnorm_rope_pair(void* x, int64_t S, int64_t ld, int heads, const float* gamma_q, const float* gamma_k,
+                               int64_t k_offset, const float* cos_tab, const float* sin_tab, int64_t tab_ld,
+                               int rope_pairs, float eps, void* out, int64_t out_token_stride, int64_t out_head_stride,
+                               int64_t out_k_offset, void* stream);
+
+/*
  * The reference's packed rows -> the GEMM's operands, one pass: row t of `packed` (ld bytes apart, 4-byte
  * aligned, ld a multiple of 4) holds K e4m3 codes and the row's fp32 dequant scale (row_mx_kernels.py:12-45);
  * codes [T, K], neutral block scales (2^0) [T, K/32] and row_scale [T] take them apart. K a multiple of 32.

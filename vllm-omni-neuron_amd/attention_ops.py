@@ -354,13 +354,49 @@ def ring_attention_const_max_fwd(q, k, v, replica_groups=None, num_workers=1, so
 
 def _base_angles(cache: torch.Tensor, B: int, S: int, what: str) -> list[torch.Tensor]:
     """Rotate-half cache ``[B, S, 128]`` (or ``[S, 128]``, ``[1, S, 128]``) = ``cat([base, base])``
-    (row_mx_modules.py:51-76) -> per batch element the fp32 ``[S, 64]`` base angles."""
+    (row_mx_modules.py:51-76) -> per batch element the fp32 ``[S, 64]`` base angles, a view where the
+    cache is fp32."""
     if not isinstance(cache, torch.Tensor) or cache.shape[-1] != HEAD_DIM or cache.dim() not in (2, 3):
         raise ValueError(f"{what} must be [B, S, {HEAD_DIM}] (rotate-half cache)")
     c = cache if cache.dim() == 3 else cache.unsqueeze(0)
     if c.shape[1] != S or c.shape[0] not in (1, B):
         raise ValueError(f"{what} must be [{B}, {S}, {HEAD_DIM}], got {list(cache.shape)}")
-    return [c[min(b, c.shape[0] - 1), :, : HEAD_DIM // 2].to(torch.float32).contiguous() for b in range(B)]
+    return [c[min(b, c.shape[0] - 1), :, : HEAD_DIM // 2].to(torch.float32) for b in range(B)]
+
+
+def _table_stride(cos: torch.Tensor | None, sin: torch.Tensor | None) -> int:
+    """The row stride that both pair tables ``[S, 64]`` share, if the kernel can read them as they are
+    (unit column stride, 16-byte aligned rows); 0 otherwise."""
+    if cos is None:
+        return HEAD_DIM // 2
+    lds = {t.stride(0) if t.shape[0] > 1 else HEAD_DIM // 2 for t in (cos, sin)}
+    ld = lds.pop()
+    ok = not lds and ld >= HEAD_DIM // 2 and ld % 4 == 0
+    return ld if ok and all(t.stride(1) == 1 and t.data_ptr() % 16 == 0 for t in (cos, sin)) else 0
+
+
+def _qk_rmsnorm_rope_pair(rows: torch.Tensor, heads: int, gammas, cos, sin, eps: float, rope_pairs: str, out) -> None:
+    """:func:`qk_rmsnorm_rope_` on Q (columns ``[0, heads*128)`` of ``rows``) and K (the next ``heads*128``)
+    in one launch; ``out`` (a contiguous-head ``[2*heads, S, 128]`` view): the results go there instead, as
+    :func:`qk_rmsnorm_rope_to` does. Same bits as the two passes."""
+    lib = _lib.load()
+    W, S = heads * HEAD_DIM, rows.shape[0]
+    for gamma in gammas:
+        if not isinstance(gamma, torch.Tensor) or gamma.numel() != W or not gamma.is_floating_point():
+            raise ValueError(f"gamma must be a floating-point tensor of {W} elements")
+    ld = _table_stride(cos, sin)
+    if not ld:
+        cos, sin = (t.clone(memory_format=torch.contiguous_format) for t in (cos, sin))
+        ld = HEAD_DIM // 2
+        _check_rope_tables(cos, sin, S, "qk_rmsnorm_rope")
+    _lib.require_gpu(rows, *gammas, cos, sin, out, what="qk_rmsnorm_rope")
+    gq, gk = (g.reshape(W).to(torch.float32).contiguous() for g in gammas)
+    o_ts, o_hs = (0, 0) if out is None else (out.stride(1), out.stride(0))
+    st = lib.wanmi_qk_rmsnorm_rope_pair(
+        _lib.ptr(rows), S, rows.stride(0), heads, _lib.ptr(gq), _lib.ptr(gk), W, _lib.ptr(cos), _lib.ptr(sin), ld,
+        _ROTATE[rope_pairs], float(eps), _lib.ptr(out), o_ts, o_hs, heads * o_hs, _lib.stream_of(rows),
+    )
+    _lib.check(st, "wanmi_qk_rmsnorm_rope_pair")
 
 
 def _norm_kind(kind, what: str) -> bool:
@@ -446,8 +482,17 @@ def row_mx_qkv_proj(
     # pass); the other heads are copied there
     out = torch.empty(width // head_dim, B, S, head_dim, dtype=y.dtype, device=y.device) if nbsd else None
     direct = [False, False]
+    # Q and K in one launch where both are normalized and alike (the self-attention)
+    pair = norm_q and norm_k and nq == nkv and nq % 4 == 0 and nq <= (40 if nbsd else 128)
     for b in range(B):  # the caches may differ per batch element; the norm is per row
         rows = y2[b * S : (b + 1) * S]
+        if pair:
+            _qk_rmsnorm_rope_pair(rows, nq, (qk_norm_pre_rope_q_gamma, qk_norm_pre_rope_k_gamma), cos[b], sin[b], eps,
+                                  w.rope_pairs, out[: 2 * nq, b] if nbsd else None)
+            direct = [nbsd, nbsd]
+            continue
+        if cos[b] is not None:
+            cos[b], sin[b] = cos[b].contiguous(), sin[b].contiguous()
         for i, (on, h0, nh, gam) in enumerate(((norm_q, 0, nq, qk_norm_pre_rope_q_gamma),
                                                (norm_k, nq, nkv, qk_norm_pre_rope_k_gamma))):
             if not on:

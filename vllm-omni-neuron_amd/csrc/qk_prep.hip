@@ -33,8 +33,9 @@ struct QKNormArgs {
   int64_t S, ld;
   int heads, nch, tokens_per_wave;
   const float* gamma;
-  const float* cos;  // [S, 64]
-  const float* sin;  // [S, 64]
+  const float* cos;  // [S] rows of 64, tab_ld apart
+  const float* sin;
+  int64_t tab_ld;
   float eps;
   float* maxnorm;  // [heads] or null (must be zeroed first)
   // optional: the queries' across-heads 1/rms from the QKV GEMM's per-128-column partial sums of
@@ -48,6 +49,9 @@ struct QKNormArgs {
   // (token t, head h, d) at out[t*out_ts + h*out_hs + d] (e.g. the head-major [N, S, 128] layout)
   uint16_t* out;
   int64_t out_ts, out_hs;
+  // a second part of as many heads (gridDim.y = 2; no maxnorm, no q_rr): x, gamma and out of part 1
+  const float* gamma1;
+  int64_t x_part, out_part;  // elements from part 0 to part 1
 };
 
 
@@ -69,6 +73,11 @@ __global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kern
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = a.heads * 128;
   const int64_t t0 = ((int64_t)blockIdx.x * 4 + wave) * a.tokens_per_wave;
+  if (blockIdx.y != 0) {
+    a.x += a.x_part;
+    a.out += a.out_part;
+    a.gamma = a.gamma1;
+  }
   const __amdgpu_buffer_rsrc_t r_g = make_rsrc(a.gamma, 4 * (int64_t)W);
   if constexpr (kLdsGamma) {
     const u32x4 rg = buffer_rsrc(a.gamma, 4u * (uint32_t)W);  // columns past W read as zero
@@ -152,8 +161,8 @@ __global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kern
     constexpr int kAngles = kHalves ? 8 : 4;
     float cs[kAngles], sn[kAngles];
     if (a.cos) {
-      const __amdgpu_buffer_rsrc_t r_c = make_rsrc(a.cos + t * 64, 256);
-      const __amdgpu_buffer_rsrc_t r_s = make_rsrc(a.sin + t * 64, 256);
+      const __amdgpu_buffer_rsrc_t r_c = make_rsrc(a.cos + t * a.tab_ld, 256);
+      const __amdgpu_buffer_rsrc_t r_s = make_rsrc(a.sin + t * a.tab_ld, 256);
       const uint32_t off = kHalves ? (uint32_t)(lane & 7) * 32 : (uint32_t)(lane & 15) * 16;
 #pragma unroll
       for (int u = 0; u < kAngles / 4; ++u) {
@@ -284,8 +293,8 @@ __global__ void zero_f32_kernel(float* p, int n) {
 constexpr int64_t kQKWavesResident = 256 * 4 * 4;
 constexpr int kQKTokensPerWaveMax = 8;
 
-static int qk_tokens_per_wave(int64_t S) {
-  const int64_t n = (S + kQKWavesResident - 1) / kQKWavesResident;
+static int qk_tokens_per_wave(int64_t rows) {
+  const int64_t n = (rows + kQKWavesResident - 1) / kQKWavesResident;
   return (int)(n < 1 ? 1 : n > kQKTokensPerWaveMax ? kQKTokensPerWaveMax : n);
 }
 
@@ -342,7 +351,8 @@ namespace wanmi {
 static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const float* gamma, const float* cos_tab,
                                 const float* sin_tab, int rope_pairs, float eps, float* maxnorm, const float* q_sumsq,
                                 int64_t q_sumsq_ld, int q_heads, float q_eps, float* q_rr, void* stream,
-                                void* out = nullptr, int64_t out_ts = 0, int64_t out_hs = 0) {
+                                void* out = nullptr, int64_t out_ts = 0, int64_t out_hs = 0, int64_t tab_ld = 64,
+                                const float* gamma1 = nullptr, int64_t x_part = 0, int64_t out_part = 0) {
   WANMI_REQUIRE(S >= 0 && heads > 0 && heads % 4 == 0 && heads <= 128, WANMI_ERR_ARG,
                 "wanmi_qk_rmsnorm_rope: need S >= 0 and heads a positive multiple of 4 (<= 128), got S=%lld heads=%d",
                 (long long)S, heads);
@@ -369,10 +379,12 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.ld = ld;
   a.heads = heads;
   a.nch = heads / 4;
-  a.tokens_per_wave = qk_tokens_per_wave(S);
+  const int parts = gamma1 ? 2 : 1;
+  a.tokens_per_wave = qk_tokens_per_wave(S * parts);
   a.gamma = gamma;
   a.cos = cos_tab;
   a.sin = sin_tab;
+  a.tab_ld = tab_ld;
   a.eps = eps;
   a.maxnorm = maxnorm;
   a.q_sumsq = q_sumsq;
@@ -383,8 +395,11 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.out = static_cast<uint16_t*>(out);
   a.out_ts = out_ts;
   a.out_hs = out_hs;
+  a.gamma1 = gamma1;
+  a.x_part = x_part;
+  a.out_part = out_part;
   const int64_t waves = (S + a.tokens_per_wave - 1) / a.tokens_per_wave;
-  const dim3 grid((unsigned)((waves + 3) / 4));
+  const dim3 grid((unsigned)((waves + 3) / 4), (unsigned)parts);
   if (out) {
     WANMI_REQUIRE(a.nch <= 10, WANMI_ERR_UNSUPPORTED, "wanmi_qk_rmsnorm_rope_to: at most 40 heads");
     if (rope_pairs == WANMI_ROTATE_HALVES) {
@@ -432,6 +447,31 @@ extern "C" int wanmi_qk_rmsnorm_rope_to(const void* x, int64_t S, int64_t ld, in
                 "wanmi_qk_rmsnorm_rope_to: one token's heads span more than 2 GiB of out");
   return qk_rmsnorm_rope_impl(const_cast<void*>(x), S, ld, heads, gamma, cos_tab, sin_tab, rope_pairs, eps, nullptr,
                               nullptr, 0, 0, 0.0f, nullptr, stream, out, out_token_stride, out_head_stride);
+}
+
+extern "C" int wanmi_qk_rmsnorm_rope_pair(void* x, int64_t S, int64_t ld, int heads, const float* gamma_q,
+                                          const float* gamma_k, int64_t k_offset, const float* cos_tab,
+                                          const float* sin_tab, int64_t tab_ld, int rope_pairs, float eps, void* out,
+                                          int64_t out_token_stride, int64_t out_head_stride, int64_t out_k_offset,
+                                          void* stream) {
+  using namespace wanmi;
+  clear_error();
+  WANMI_REQUIRE(S == 0 || (gamma_k && ((uintptr_t)gamma_k % 16) == 0), WANMI_ERR_ARG,
+                "wanmi_qk_rmsnorm_rope_pair: gamma_k must be a 16-byte aligned pointer");
+  WANMI_REQUIRE(heads > 0 && k_offset >= (int64_t)heads * 128 && k_offset % 8 == 0 && ld >= k_offset + (int64_t)heads * 128,
+                WANMI_ERR_ARG, "wanmi_qk_rmsnorm_rope_pair: Q and K must lie apart in the row (heads=%d k_offset=%lld ld=%lld)",
+                heads, (long long)k_offset, (long long)ld);
+  WANMI_REQUIRE(!cos_tab || (tab_ld >= 64 && tab_ld % 4 == 0), WANMI_ERR_ARG,
+                "wanmi_qk_rmsnorm_rope_pair: tab_ld=%lld must be >= 64 and a multiple of 4", (long long)tab_ld);
+  WANMI_REQUIRE(!out || (((uintptr_t)out % 16) == 0 && out_token_stride % 8 == 0 && out_head_stride % 8 == 0 &&
+                         out_k_offset % 8 == 0 && out_token_stride >= 0 && out_head_stride >= 0 && out_k_offset >= 0),
+                WANMI_ERR_ARG,
+                "wanmi_qk_rmsnorm_rope_pair: out must be 16-byte aligned with strides that are multiples of 8 elements");
+  WANMI_REQUIRE(((int64_t)(heads - 1) * out_head_stride + 128) * 2 < (1LL << 31), WANMI_ERR_UNSUPPORTED,
+                "wanmi_qk_rmsnorm_rope_pair: one token's heads span more than 2 GiB of out");
+  return qk_rmsnorm_rope_impl(x, S, ld, heads, gamma_q, cos_tab, sin_tab, rope_pairs, eps, nullptr, nullptr, 0, 0, 0.0f,
+                              nullptr, stream, out, out_token_stride, out_head_stride, tab_ld, gamma_k, k_offset,
+                              out_k_offset);
 }
 
 extern "C" int wanmi_qk_rmsnorm_rope_qrr(void* x, int64_t S, int64_t ld, int heads, const float* gamma,
