@@ -147,14 +147,15 @@ def check(status: int, what: str) -> None:
     raise WanmiError(f"{what}: status {status}: {msg}")
 
 
-def ptr(t: torch.Tensor | None):
+def ptr(t: torch.Tensor | None) -> int | None:
     """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor):
-    """The current HIP stream of ``t``'s device, as the void* the C ABI takes."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def stream_of(t: torch.Tensor) -> int:
+    """The current HIP stream of ``t``'s device, as the void* the C ABI takes (the handle that
+    ``torch.cuda.current_stream(t.device).cuda_stream`` holds, without the stream object: 0.2 against 2.5 us)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def expect(t: torch.Tensor | None, what: str, *, dtype: torch.dtype, shape: tuple | None = None,
@@ -169,7 +170,7 @@ def expect(t: torch.Tensor | None, what: str, *, dtype: torch.dtype, shape: tupl
         raise ValueError(f"{what} must be a torch.Tensor, got {type(t).__name__}")
     if t.dtype != dtype:
         raise ValueError(f"{what} must be {dtype}, got {t.dtype}")
-    if shape is not None:
+    if shape is not None and t.shape != shape:
         if t.dim() != len(shape) or any(want is not None and have != want for have, want in zip(t.shape, shape)):
             want = "[" + ", ".join("*" if w is None else str(w) for w in shape) + "]"
             raise ValueError(f"{what} must have shape {want}, got {list(t.shape)}")
@@ -181,16 +182,16 @@ def expect(t: torch.Tensor | None, what: str, *, dtype: torch.dtype, shape: tupl
 
 def require_gpu(*tensors: torch.Tensor | None, what: str) -> torch.device:
     """Every tensor must live on the same GPU; the kernels never run on the host."""
-    dev = None
+    first, index = None, -1
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(f"{what}: tensors must be on a ROCm GPU (got {t.device}); no CPU fallback")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"{what}: tensors on different devices ({dev} vs {t.device})")
-    if dev is None:
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise RuntimeError(f"{what}: tensors on different devices ({first.device} vs {t.device})")
+    if first is None:
         raise RuntimeError(f"{what}: no tensor given")
-    return dev
+    return first.device

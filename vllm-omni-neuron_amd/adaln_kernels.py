@@ -48,6 +48,8 @@ def _row(vec: torch.Tensor | None, b: int, H: int) -> torch.Tensor | None:
     """[B, 1, H] (per batch) or [H] / [1, H] (shared) -> contiguous fp32 [H] for batch ``b``."""
     if vec is None:
         return None
+    if vec.dtype == torch.float32 and vec.shape == (H,) and vec.is_contiguous():
+        return vec
     v = vec[b] if vec.dim() == 3 else vec
     return v.reshape(H).to(torch.float32).contiguous()
 
@@ -81,10 +83,10 @@ def adaln_quant_2d(
     if quant == "none":
         out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
     elif quant == "mx":
-        out = torch.empty((T, H), dtype=torch.uint8, device=dev)
+        out = torch.empty((T, H), dtype=torch.float8_e4m3fn, device=dev)
         scales = torch.empty((T, H // 32), dtype=torch.uint8, device=dev)
     else:
-        out = torch.empty((T, H + 4), dtype=torch.uint8, device=dev)
+        out = torch.empty((T, H + 4), dtype=torch.float8_e4m3fn, device=dev)
     residual_out = torch.empty_like(x) if residual is not None else None
     status = lib.wanmi_adaln_quant(
         _lib.ptr(x),
@@ -104,9 +106,7 @@ def adaln_quant_2d(
     )
     _lib.check(status, "wanmi_adaln_quant")
     if quant == "mx":
-        out = MXTensor(out.view(torch.float8_e4m3fn), scales)
-    elif quant == "row":
-        out = out.view(torch.float8_e4m3fn)
+        out = MXTensor(out, scales)
     return out if residual is None else (residual_out, out)
 
 
@@ -131,7 +131,12 @@ def adaln_modulate(
     """
     _validate(hidden, norm_type, quant, ocp)
     have_residual = residual is not None
-    hidden_3d = hidden.unsqueeze(0) if hidden.dim() == 2 else hidden
+    if hidden.dim() == 2:
+        H = hidden.shape[1]
+        r2 = None if residual is None else (residual if residual.dim() == 2 else residual[0]).reshape(-1, H)
+        return adaln_quant_2d(hidden, _row(mul, 0, H), _row(add, 0, H), eps=eps, norm_type=norm_type, quant=quant,
+                              residual=r2, gate=_row(gate, 0, H) if have_residual else None)
+    hidden_3d = hidden
     residual_3d = None
     if have_residual:
         residual_3d = residual.unsqueeze(0) if residual.dim() == 2 else residual
@@ -167,18 +172,11 @@ def adaln_modulate(
             _stack([o.codes for o in outs], lambda p: p.shape[-1]),
             _stack([o.scales for o in outs], lambda p: p.shape[-1]),
         )
-        if hidden.dim() == 2:
-            out = MXTensor(out.codes[0], out.scales[0])
     else:
         out = _stack(outs, lambda p: p.shape[-1])
-        if hidden.dim() == 2:
-            out = out[0]
     if not have_residual:
         return out
-    residual_out = _stack(res_outs, lambda p: p.shape[-1])
-    if hidden.dim() == 2:
-        residual_out = residual_out[0]
-    return residual_out, out
+    return _stack(res_outs, lambda p: p.shape[-1]), out
 
 
 @dataclass(frozen=True)

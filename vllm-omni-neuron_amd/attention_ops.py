@@ -242,7 +242,7 @@ def attention_core(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, kmax: tor
         out = torch.empty((N, D, Sq), dtype=torch.bfloat16, device=dev) if out is None else out
         o_hs, o_ss, o_ds = out.stride(0), 1, out.stride(1)
     else:
-        out = torch.empty((Sq, N * D), dtype=torch.uint8, device=dev) if out is None else out
+        out = torch.empty((Sq, N * D), dtype=torch.float8_e4m3fn, device=dev) if out is None else out
         scales = torch.empty((Sq, N * D // 32), dtype=torch.uint8, device=dev)
         o_hs, o_ss, o_ds = D, out.stride(0), 1
     common = (

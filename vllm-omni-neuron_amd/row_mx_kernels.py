@@ -125,9 +125,10 @@ def _as_mx_2d(x):
         if K % 32:
             raise ValueError(f"MX activation width {K} must be a multiple of 32")
         lead = x.codes.shape[:-1]
-        codes = x.codes.reshape(-1, K).view(torch.uint8)
-        _lib.expect(x.scales, "activation scales", dtype=torch.uint8, shape=(*lead, K // 32), contiguous=False)
-        scales = x.scales.reshape(-1, K // 32)
+        codes, scales = x.codes, x.scales
+        _lib.expect(scales, "activation scales", dtype=torch.uint8, shape=(*lead, K // 32), contiguous=False)
+        if len(lead) != 1:
+            codes, scales = codes.reshape(-1, K), scales.reshape(-1, K // 32)
         if codes.stride(1) != 1 or scales.stride(1) != 1:
             raise ValueError("MX codes and scales must have unit stride along the last dimension")
         return codes, scales, None, lead
@@ -211,7 +212,7 @@ def mxfp8_linear(
     dev = codes.device
     out_scales = None
     if epilogue == "gelu_mx":
-        out = torch.empty((M, N), dtype=torch.uint8, device=dev) if out is None else out
+        out = torch.empty((M, N), dtype=torch.float8_e4m3fn, device=dev) if out is None else out
         out_scales = torch.empty((M, N // 32), dtype=torch.uint8, device=dev)
     else:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=dev) if out is None else out
@@ -245,8 +246,10 @@ def mxfp8_linear(
     )
     _lib.check(status, "wanmi_mxfp8_gemm")
     if epilogue == "gelu_mx":
-        return MXTensor(out.view(torch.float8_e4m3fn).reshape(*lead, N), out_scales.reshape(*lead, N // 32))
-    return out.reshape(*lead, N)
+        out = out.view(torch.float8_e4m3fn)
+        return MXTensor(out, out_scales) if len(lead) == 1 else MXTensor(out.reshape(*lead, N),
+                                                                        out_scales.reshape(*lead, N // 32))
+    return out if len(lead) == 1 else out.reshape(*lead, N)
 
 
 def mxfp8_qkv_linear(x, weight: MXWeight, *, vt_col0: int, row_sumsq: torch.Tensor | None = None,
