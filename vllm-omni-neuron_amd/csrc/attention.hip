@@ -1187,8 +1187,8 @@ __global__ __launch_bounds__(256) void head_max_norm_kernel(const uint16_t* x, i
 // loads of two tokens in flight) instead of one head's 256 bytes per token row, so the reads are
 // sequential; lane group l >> 4 of chunk c holds head 4 c + (l >> 4). Each wave keeps per-head maxima
 // of ||x||^2 in registers; the workgroup reduces them through LDS and issues one atomic per head.
-constexpr int kHmnRowWaves = 4;
-__global__ __launch_bounds__(256) void head_max_norm_rows_kernel(const uint16_t* x, int64_t ss, int64_t S, int heads,
+constexpr int kHmnRowWaves = 8;
+__global__ __launch_bounds__(64 * kHmnRowWaves) void head_max_norm_rows_kernel(const uint16_t* x, int64_t ss, int64_t S, int heads,
                                                                  float* out) {
   __shared__ float smax[kHmnRowWaves][40];
   const int lane = threadIdx.x & 63;
@@ -1267,9 +1267,9 @@ extern "C" int wanmi_head_max_norm(const void* x, int64_t head_stride, int64_t t
   if (st || S == 0) return st;
   WANMI_REQUIRE(x && ((uintptr_t)x % 16) == 0, WANMI_ERR_ARG, "wanmi_head_max_norm: x must be 16-byte aligned");
   if (head_stride == 128 && heads % 4 == 0 && heads <= 40 && token_stride >= heads * 128) {
-    // heads contiguous within a token: whole rows per wave (two tokens per step, so 8 per workgroup)
+    // heads contiguous within a token: whole rows per wave, two tokens per step
     const int64_t blocks = min((S + 2 * kHmnRowWaves - 1) / (2 * kHmnRowWaves), (int64_t)1024);
-    hipLaunchKernelGGL(head_max_norm_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, s,
+    hipLaunchKernelGGL(head_max_norm_rows_kernel, dim3((unsigned)blocks), dim3(64 * kHmnRowWaves), 0, s,
                        static_cast<const uint16_t*>(x), token_stride, S, heads, out);
     return check_launch("wanmi_head_max_norm");
   }

@@ -64,15 +64,16 @@ struct QKNormArgs {
 // Up to 40 heads the fp32 gamma (8 bytes per column, as much as the token's own bf16 read and write)
 // is copied into LDS once per workgroup of 32 tokens instead of being read from L2 per token: per
 // chunk, every lane's first four values (16 bytes, lane-major), then the second four.
-template <int NCH, bool kHalves, bool kOut = false>
-__global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kernel(QKNormArgs a) {
+// kWgWaves: waves per workgroup; with the key-norm maximum, more of them (launch_qk_waves has the reason).
+template <int NCH, bool kHalves, bool kOut = false, int kWgWaves = 4>
+__global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kernel(QKNormArgs a) {
 #pragma clang fp contract(off)
   constexpr bool kLdsGamma = NCH <= 10;
   __shared__ __attribute__((aligned(16))) float sgam[kLdsGamma ? 2 * NCH * 64 * 4 : 4];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = a.heads * 128;
-  const int64_t t0 = ((int64_t)blockIdx.x * 4 + wave) * a.tokens_per_wave;
+  const int64_t t0 = ((int64_t)blockIdx.x * kWgWaves + wave) * a.tokens_per_wave;
   if (blockIdx.y != 0) {
     a.x += a.x_part;
     a.out += a.out_part;
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kern
   if constexpr (kLdsGamma) {
     const u32x4 rg = buffer_rsrc(a.gamma, 4u * (uint32_t)W);  // columns past W read as zero
     const uint32_t base = lds_addr(sgam);
-    for (int k = wave; k < 2 * NCH; k += 4) {
+    for (int k = wave; k < 2 * NCH; k += kWgWaves) {
       const int hh = k / NCH, c = k % NCH;
       lds_dma_b128(rg, (uint32_t)(c * 512 + 8 * lane + 4 * hh) * 4, base + (uint32_t)k * 1024);
     }
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kern
     // Workgroup maximum first (through LDS), then one atomic per head per workgroup: every wave of
     // the grid finishes at about the same time, and per-wave atomics on the same few cache lines
     // serialize at the L2 (measured: 180 us of a 340 us launch).
-    __shared__ float smax[4][NCH * 4];
+    __shared__ float smax[kWgWaves][NCH * 4];
     if ((lane & 15) == 0) {
 #pragma unroll
       for (int c = 0; c < NCH; ++c) smax[wave][c * 4 + (lane >> 4)] = kmx[c];
@@ -270,7 +271,9 @@ __global__ __launch_bounds__(256, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kern
     __syncthreads();
     const int hd = threadIdx.x;
     if (hd < a.heads) {
-      const float m = fmaxf(fmaxf(smax[0][hd], smax[1][hd]), fmaxf(smax[2][hd], smax[3][hd]));
+      float m = smax[0][hd];
+#pragma unroll
+      for (int w = 1; w < kWgWaves; ++w) m = fmaxf(m, smax[w][hd]);
       // non-negative floats order like their bit patterns
       atomicMax(reinterpret_cast<unsigned int*>(a.maxnorm) + hd, __float_as_uint(sqrtf(m)));
     }
@@ -348,6 +351,30 @@ __global__ __launch_bounds__(256) void transpose_heads_kernel(TransposeArgs a) {
 }  // namespace wanmi
 
 namespace wanmi {
+// With the key-norm maximum every workgroup ends in atomics on the same 160 bytes, which the XCDs' separate
+// L2s leave to the memory side: about 45 ns a workgroup, one after another, so half as many workgroups
+// of eight waves take half of it off (16 waves: as good, and 392 against 356 us at 75600 tokens). With 4 / 8
+// waves: 20.6 / 17.9 us at 2500 tokens, 30.2 / 23.9 at 4096, 39.3 / 32.9 at 7800, 144 either way at 32760.
+template <int NCH, bool kHalves, bool kOut, int kWgWaves>
+static void launch_qk_waves(const QKNormArgs& a, int parts, hipStream_t s) {
+  const int64_t waves = (a.S + a.tokens_per_wave - 1) / a.tokens_per_wave;
+  const dim3 grid((unsigned)((waves + kWgWaves - 1) / kWgWaves), (unsigned)parts);
+  hipLaunchKernelGGL((qk_rmsnorm_rope_kernel<NCH, kHalves, kOut, kWgWaves>), grid, dim3(64 * kWgWaves), 0, s, a);
+}
+
+template <bool kHalves>
+static void launch_qk(const QKNormArgs& a, int parts, hipStream_t s) {
+  if (a.out) {
+    if (a.nch <= 4) launch_qk_waves<4, kHalves, true, 4>(a, parts, s);
+    else launch_qk_waves<10, kHalves, true, 4>(a, parts, s);
+  } else if (a.nch <= 10 && a.maxnorm) {
+    launch_qk_waves<10, kHalves, false, 8>(a, parts, s);
+  } else if (a.nch <= 4) launch_qk_waves<4, kHalves, false, 4>(a, parts, s);
+  else if (a.nch <= 10) launch_qk_waves<10, kHalves, false, 4>(a, parts, s);
+  else if (a.nch <= 16) launch_qk_waves<16, kHalves, false, 4>(a, parts, s);
+  else launch_qk_waves<32, kHalves, false, 4>(a, parts, s);
+}
+
 static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const float* gamma, const float* cos_tab,
                                 const float* sin_tab, int rope_pairs, float eps, float* maxnorm, const float* q_sumsq,
                                 int64_t q_sumsq_ld, int q_heads, float q_eps, float* q_rr, void* stream,
@@ -398,30 +425,9 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.gamma1 = gamma1;
   a.x_part = x_part;
   a.out_part = out_part;
-  const int64_t waves = (S + a.tokens_per_wave - 1) / a.tokens_per_wave;
-  const dim3 grid((unsigned)((waves + 3) / 4), (unsigned)parts);
-  if (out) {
-    WANMI_REQUIRE(a.nch <= 10, WANMI_ERR_UNSUPPORTED, "wanmi_qk_rmsnorm_rope_to: at most 40 heads");
-    if (rope_pairs == WANMI_ROTATE_HALVES) {
-      if (a.nch <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<4, true, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<10, true, true>), grid, dim3(256), 0, s, a);
-    } else {
-      if (a.nch <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<4, false, true>), grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<10, false, true>), grid, dim3(256), 0, s, a);
-    }
-    return check_launch("wanmi_qk_rmsnorm_rope_to");
-  }
-  if (rope_pairs == WANMI_ROTATE_HALVES) {
-    if (a.nch <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<4, true>), grid, dim3(256), 0, s, a);
-    else if (a.nch <= 10) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<10, true>), grid, dim3(256), 0, s, a);
-    else if (a.nch <= 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<16, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<32, true>), grid, dim3(256), 0, s, a);
-  } else {
-    if (a.nch <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<4, false>), grid, dim3(256), 0, s, a);
-    else if (a.nch <= 10) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<10, false>), grid, dim3(256), 0, s, a);
-    else if (a.nch <= 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<16, false>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(qk_rmsnorm_rope_kernel<32, false>), grid, dim3(256), 0, s, a);
-  }
+  if (out) WANMI_REQUIRE(a.nch <= 10, WANMI_ERR_UNSUPPORTED, "wanmi_qk_rmsnorm_rope_to: at most 40 heads");
+  if (rope_pairs == WANMI_ROTATE_HALVES) launch_qk<true>(a, parts, s);
+  else launch_qk<false>(a, parts, s);
   return check_launch("wanmi_qk_rmsnorm_rope");
 }
 }  // namespace wanmi
