@@ -304,6 +304,16 @@ int wanmi_qk_rmsnorm_rope_to(const void* x, int64_t S, int64_t ld, int heads, co
                              int64_t out_head_stride, void* stream);
 
 /*
+ * wanmi_mxfp8_gemm_qkv for K and V held as two weights of N rows each (the cross-attention's projections of
+ * the text context): K token-major into out [M, ldo], V into vt as V^T [N/128][128][vt_ld]. N a multiple
+ * of 256; M, vt_ld and the one or two launches as there.
+ */
+int wanmi_mxfp8_gemm_kv(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* k_codes, const uint8_t* k_scales,
+                        const float* k_col_scale, const float* k_bias, const uint8_t* v_codes, const uint8_t* v_scales,
+                        const float* v_col_scale, const float* v_bias, const float* row_scale, int64_t M, int64_t N,
+                        int64_t K, int64_t lda, void* out, int64_t ldo, void* vt, int64_t vt_ld, void* stream);
+
+/*
  * wanmi_qk_rmsnorm_rope on two parts of every row in one launch: Q at columns [0, heads*128) with gamma_q and
  * K, k_offset columns on, with gamma_k (each its own across-heads norm; the same rotation). The tables'
  * rows are tab_ld floats apart (a multiple of 4, at least 64: the first halves of rotate-half caches can

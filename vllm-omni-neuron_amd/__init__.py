@@ -15,6 +15,7 @@ from .common_types import DtypeMode, MXTensor, NormType, QKNormConfig, QKVOutput
 from .row_mx_kernels import (  # noqa: F401
     MXWeight,
     mxfp8_linear,
+    mxfp8_kv_linear,
     mxfp8_qkv_linear,
     packed_weight_to_mx,
     quantize_weight_mx,

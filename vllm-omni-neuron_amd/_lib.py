@@ -55,6 +55,8 @@ _SIGNATURES = {
     ],
     "wanmi_hbm_stream_copy": [_vp, _vp, _i64, _vp],
     "wanmi_hbm_stream_fold": [_vp, _vp, _i64, _vp],
+    "wanmi_mxfp8_gemm_kv": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp,
+                            _i64, _vp],
     "wanmi_qk_rmsnorm_rope_pair": [_vp, _i64, _i64, _i32, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _f32, _vp, _i64, _i64,
                                    _i64, _vp],
     "wanmi_row_unpack": [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp],

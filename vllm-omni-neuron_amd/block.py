@@ -35,7 +35,7 @@ import torch
 from . import attention_ops as ops
 from .adaln_kernels import adaln_quant_2d
 from .rope import rope_tables
-from .row_mx_kernels import MXWeight, mxfp8_linear, mxfp8_qkv_linear, quantize_weight_mx
+from .row_mx_kernels import MXWeight, mxfp8_kv_linear, mxfp8_linear, mxfp8_qkv_linear, quantize_weight_mx
 
 DIM, HEADS, HEAD_DIM, FFN = 5120, 40, 128, 13824
 
@@ -101,12 +101,9 @@ def project_cross_kv(w: BlockWeights, context: torch.Tensor, eps: float = 1e-6) 
     """Text context ``[S_txt, DIM]`` bf16 -> normalized K, V^T and the key-norm bound (once per
     generation; the reference row-packs the context once and projects K/V per expert)."""
     ctx = adaln_quant_2d(context.contiguous(), None, None, eps=0.0, norm_type="none", quant="mx")
-    k = mxfp8_linear(ctx, w.k2)
+    k, vt = mxfp8_kv_linear(ctx, w.k2, w.v2)
     kmax = ops.qk_rmsnorm_rope_(k, w.norm_k2, eps=eps, want_max=True)
-    v = mxfp8_linear(ctx, w.v2)
-    heads = k.shape[1] // HEAD_DIM
-    vt, _ = ops.transpose_heads(v.view(-1, heads, HEAD_DIM))
-    return CrossKV(k.view(-1, heads, HEAD_DIM), vt, kmax)
+    return CrossKV(k.view(-1, k.shape[1] // HEAD_DIM, HEAD_DIM), vt, kmax)
 
 
 _ONES: dict = {}

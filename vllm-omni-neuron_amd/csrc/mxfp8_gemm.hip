@@ -78,11 +78,23 @@ struct GemmArgs {
   int64_t sumsq_ld;         // row stride of row_sumsq in floats
   uint16_t* vt;             // V^T epilogue: [N/128][128][vt_ld] bf16
   int64_t vt_ld;
-  int64_t vt_col0;          // kEpiQkv: first V column
+  int64_t vt_col0;          // kEpiQkv: first V column; its weight, scales and bias from column vt_col0 on:
+  const uint8_t* v_w;
+  const uint8_t* v_w_scales;
+  const float* v_col_scale;
+  const float* v_bias;
   int64_t M, N, K, lda, ldo;
   int tiles_m, tiles_n;
   int qk_wgs;               // kEpiQkv, 256-feature tiles: workgroups that walk the Q|K tiles
 };
+
+// kEpiQkv: the arguments of the V part, a product of its own.
+__device__ __forceinline__ void to_v_weight(GemmArgs& g) {
+  g.w = g.v_w;
+  g.w_scales = g.v_w_scales;
+  g.col_scale = g.v_col_scale;
+  g.bias = g.v_bias;
+}
 
 // gelu_tanh(x) = 0.5 x (1 + tanh(u)) = x / (1 + exp(-2u)),  u = sqrt(2/pi) (x + 0.044715 x^3);
 // exp(-2u) = 2^(x (k0 + k1 x^2)) with k0 = -2 log2(e) sqrt(2/pi), k1 = 0.044715 k0 folded into one
@@ -1066,10 +1078,7 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
       ring_tiles<WANMI_EPI_BF16, kNj>(g, sWh, sAct, ssc, wg, g.qk_wgs);
     } else {
       g.tiles_n -= (int)(g.vt_col0 / TN);
-      g.w += g.vt_col0 * g.K;
-      g.w_scales += g.vt_col0 * (g.K / 32);
-      if (g.col_scale) g.col_scale += g.vt_col0;
-      if (g.bias) g.bias += g.vt_col0;
+      to_v_weight(g);
       ring_tiles<kEpiVt, kNj>(g, sWh, sAct, ssc, wg - g.qk_wgs, (int)gridDim.x - g.qk_wgs);
     }
   } else {
@@ -1307,8 +1316,8 @@ __device__ __forceinline__ void ts_tile(const GemmArgs& g, TsShared& sh, int m0,
   uint8_t* rarea = sh.code[1] + wave * 8192;
   const bool scaled = g.row_scale || g.col_scale;
   if constexpr (kSwap) {
-    if (scaled) epilogue_vt_row<true>(g, acc, sh.vec, stage, m0, n0 - g.vt_col0, wave);
-    else epilogue_vt_row<false>(g, acc, sh.vec, stage, m0, n0 - g.vt_col0, wave);
+    if (scaled) epilogue_vt_row<true>(g, acc, sh.vec, stage, m0, n0, wave);
+    else epilogue_vt_row<false>(g, acc, sh.vec, stage, m0, n0, wave);
   } else {
     if (m0 + wave * 32 >= (int)g.M) return;  // no token of this wave
     f32x16 a1[4][1] = {{acc[0]}, {acc[1]}, {acc[2]}, {acc[3]}};
@@ -1333,8 +1342,11 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_tile128_kernel(GemmArgs g) 
   int m0, n0;
   ts_coords(g, (int)blockIdx.x, m0, n0);
   if constexpr (EPI == kEpiQkv) {
-    if (n0 >= (int)g.vt_col0) ts_tile<kEpiVt>(g, sh, m0, n0);
-    else ts_tile<WANMI_EPI_BF16>(g, sh, m0, n0);
+    if (n0 >= (int)g.vt_col0) {
+      n0 -= (int)g.vt_col0;
+      to_v_weight(g);
+      ts_tile<kEpiVt>(g, sh, m0, n0);
+    } else ts_tile<WANMI_EPI_BF16>(g, sh, m0, n0);
   } else {
     ts_tile<EPI>(g, sh, m0, n0);
   }
@@ -1455,11 +1467,25 @@ static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t 
   return check_launch("wanmi_mxfp8_gemm");
 }
 
+// One projection weight: codes [N, K], block scales, per-channel scales and bias (either may be null).
+struct WeightPart {
+  const uint8_t* codes;
+  const uint8_t* scales;
+  const float* col_scale;
+  const float* bias;
+};
+
+static bool aligned_weight(const WeightPart& w) {
+  return ((uintptr_t)w.codes % 16) == 0 && ((uintptr_t)w.scales % 4) == 0 && ((uintptr_t)w.col_scale % 16) == 0 &&
+         ((uintptr_t)w.bias % 16) == 0;
+}
+
+// `v`: the V weight of kEpiQkv (columns [vt_col0, N)).
 static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes, const uint8_t* w_scales,
                      const float* row_scale, const float* col_scale, const float* bias, int64_t M, int64_t N,
                      int64_t K, int64_t lda, int epilogue, void* out, int64_t ldo, uint8_t* out_scales,
                      const void* residual, const float* gate, float* row_sumsq, int64_t sumsq_cols, int64_t sumsq_ld,
-                     void* vt, int64_t vt_ld, int64_t vt_col0, void* stream) {
+                     void* vt, int64_t vt_ld, int64_t vt_col0, void* stream, const WeightPart& v = WeightPart{}) {
   WANMI_REQUIRE(M >= 0 && N > 0 && K > 0, WANMI_ERR_ARG, "wanmi_mxfp8_gemm: bad sizes M=%lld N=%lld K=%lld",
                 (long long)M, (long long)N, (long long)K);
   WANMI_REQUIRE(N % TN == 0, WANMI_ERR_UNSUPPORTED, "wanmi_mxfp8_gemm: N=%lld must be a multiple of %d",
@@ -1487,7 +1513,7 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
                     (!bias || ((uintptr_t)bias % 16) == 0) &&
                     (!col_scale || ((uintptr_t)col_scale % 16) == 0) &&
                     (!gate || ((uintptr_t)gate % 16) == 0) && (!residual || ((uintptr_t)residual % 16) == 0) &&
-                    ((uintptr_t)vt % 16) == 0,
+                    ((uintptr_t)vt % 16) == 0 && aligned_weight(v),
                 WANMI_ERR_ARG, "wanmi_mxfp8_gemm: misaligned operand");
   const int64_t tiles = (N / TN) * ((M + TM - 1) / TM);
   WANMI_REQUIRE(tiles < (1LL << 31), WANMI_ERR_ARG, "wanmi_mxfp8_gemm: problem too large");
@@ -1525,6 +1551,10 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
   g.lda = lda;
   g.ldo = ldo;
   g.vt_col0 = to_qkv ? vt_col0 : 0;
+  g.v_w = v.codes;
+  g.v_w_scales = v.scales;
+  g.v_col_scale = v.col_scale;
+  g.v_bias = v.bias;
   g.tiles_m = (int)((M + TM - 1) / TM);
   g.tiles_n = (int)(N / TN);
   g.qk_wgs = 0;
@@ -1568,6 +1598,34 @@ extern "C" int wanmi_mxfp8_gemm_rowsumsq(const uint8_t* a_codes, const uint8_t* 
                    ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, N / 128, nullptr, 0, 0, stream);
 }
 
+namespace wanmi {
+// out [M, n_out] (bf16, with optional partial sums of squares) = A w^T and V^T = A v^T (n_v columns).
+static int projection_with_vt(const uint8_t* a_codes, const uint8_t* a_scales, const float* row_scale, int64_t M,
+                              int64_t K, int64_t lda, const WeightPart& w, int64_t n_out, const WeightPart& v, int64_t n_v,
+                              void* out, int64_t ldo, float* row_sumsq, int64_t sumsq_cols, void* vt, int64_t vt_ld,
+                              void* stream) {
+  // In one launch where that saves a round of tiles (one latent frame, 1560 tokens: 172 -> 121 us) or one
+  // launch as such; two launches otherwise (at 32760 tokens both parts are whole rounds).
+  if ((K / BK) % 4 == 0) {
+    const int cus = device_cu_count();
+    WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm_qkv: cannot query the device's compute units");
+    const int64_t apart = select_tile(M, n_out, cus, 0).cost + select_tile(M, n_v, cus, vt_ld).cost;
+    if (select_qkv_tile(M, n_out, n_v, cus, vt_ld).cost <= apart)
+      return gemm_impl(a_codes, a_scales, w.codes, w.scales, row_scale, w.col_scale, w.bias, M, n_out + n_v, K, lda,
+                       kEpiQkv, out, ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, n_out / 128, vt, vt_ld, n_out,
+                       stream, v);
+  }
+  // the plain bf16 epilogue (with the partial sums)
+  int st = gemm_impl(a_codes, a_scales, w.codes, w.scales, row_scale, w.col_scale, w.bias, M, n_out, K, lda,
+                     WANMI_EPI_BF16, out, ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, n_out / 128, nullptr, 0, 0,
+                     stream);
+  if (st != WANMI_OK) return st;
+  // V: transposed accumulator, V^T epilogue
+  return gemm_impl(a_codes, a_scales, v.codes, v.scales, row_scale, v.col_scale, v.bias, M, n_v, K, lda, kEpiVt, nullptr,
+                   0, nullptr, nullptr, nullptr, nullptr, 0, 0, vt, vt_ld, 0, stream);
+}
+}  // namespace wanmi
+
 extern "C" int wanmi_mxfp8_gemm_qkv(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes,
                                     const uint8_t* w_scales, const float* row_scale, const float* col_scale,
                                     const float* bias, int64_t M, int64_t N, int64_t K, int64_t lda, void* out,
@@ -1588,24 +1646,26 @@ extern "C" int wanmi_mxfp8_gemm_qkv(const uint8_t* a_codes, const uint8_t* a_sca
   WANMI_REQUIRE(M > 0 && vt_ld <= (M + TM - 1) / TM * TM, WANMI_ERR_ARG,
                 "wanmi_mxfp8_gemm_qkv: M=%lld must be positive and vt_ld=%lld at most M rounded up to %d",
                 (long long)M, (long long)vt_ld, TM);
-  // In one launch where that saves a round of tiles (one latent frame, 1560 tokens: 172 -> 121 us); two
-  // launches otherwise (at 32760 tokens both parts are whole rounds).
-  if ((K / BK) % 4 == 0) {
-    const int cus = device_cu_count();
-    WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm_qkv: cannot query the device's compute units");
-    const int64_t apart = select_tile(M, vt_col0, cus, 0).cost + select_tile(M, N - vt_col0, cus, vt_ld).cost;
-    if (select_qkv_tile(M, vt_col0, N - vt_col0, cus, vt_ld).cost <= apart)
-      return gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, N, K, lda, kEpiQkv, out, ldo,
-                       nullptr, nullptr, nullptr, row_sumsq, row_sumsq ? sumsq_cols : 0, vt_col0 / 128, vt, vt_ld,
-                       vt_col0, stream);
-  }
-  // Q | K: the plain bf16 epilogue (with the Q partial sums) on the weight rows [0, vt_col0)
-  int st = gemm_impl(a_codes, a_scales, w_codes, w_scales, row_scale, col_scale, bias, M, vt_col0, K, lda,
-                     WANMI_EPI_BF16, out, ldo, nullptr, nullptr, nullptr, row_sumsq, row_sumsq ? sumsq_cols : 0,
-                     vt_col0 / 128, nullptr, 0, 0, stream);
-  if (st != WANMI_OK) return st;
-  // V: the weight rows [vt_col0, N), transposed accumulator, V^T epilogue
-  return gemm_impl(a_codes, a_scales, w_codes + vt_col0 * K, w_scales + vt_col0 * (K / 32), row_scale,
-                   col_scale ? col_scale + vt_col0 : nullptr, bias ? bias + vt_col0 : nullptr, M, N - vt_col0, K, lda,
-                   kEpiVt, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0, 0, vt, vt_ld, 0, stream);
+  const WeightPart w{w_codes, w_scales, col_scale, bias};
+  const WeightPart v{w_codes ? w_codes + vt_col0 * K : nullptr, w_scales ? w_scales + vt_col0 * (K / 32) : nullptr,
+                     col_scale ? col_scale + vt_col0 : nullptr, bias ? bias + vt_col0 : nullptr};
+  return projection_with_vt(a_codes, a_scales, row_scale, M, K, lda, w, vt_col0, v, N - vt_col0, out, ldo, row_sumsq,
+                            row_sumsq ? sumsq_cols : 0, vt, vt_ld, stream);
+}
+
+extern "C" int wanmi_mxfp8_gemm_kv(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* k_codes,
+                                   const uint8_t* k_scales, const float* k_col_scale, const float* k_bias,
+                                   const uint8_t* v_codes, const uint8_t* v_scales, const float* v_col_scale,
+                                   const float* v_bias, const float* row_scale, int64_t M, int64_t N, int64_t K,
+                                   int64_t lda, void* out, int64_t ldo, void* vt, int64_t vt_ld, void* stream) {
+  using namespace wanmi;
+  clear_error();
+  WANMI_REQUIRE(vt && v_codes && v_scales, WANMI_ERR_ARG, "wanmi_mxfp8_gemm_kv: null pointer");
+  WANMI_REQUIRE(N > 0 && N % TN == 0 && K > 0 && K % 32 == 0, WANMI_ERR_UNSUPPORTED,
+                "wanmi_mxfp8_gemm_kv: N=%lld must be a multiple of %d and K=%lld of 32", (long long)N, TN, (long long)K);
+  WANMI_REQUIRE(M > 0 && vt_ld <= (M + TM - 1) / TM * TM, WANMI_ERR_ARG,
+                "wanmi_mxfp8_gemm_kv: M=%lld must be positive and vt_ld=%lld at most M rounded up to %d", (long long)M,
+                (long long)vt_ld, TM);
+  return projection_with_vt(a_codes, a_scales, row_scale, M, K, lda, WeightPart{k_codes, k_scales, k_col_scale, k_bias}, N,
+                            WeightPart{v_codes, v_scales, v_col_scale, v_bias}, N, out, ldo, nullptr, 0, vt, vt_ld, stream);
 }

@@ -290,6 +290,35 @@ def mxfp8_qkv_linear(x, weight: MXWeight, *, vt_col0: int, row_sumsq: torch.Tens
     return qk.reshape(*lead, vt_col0), vt
 
 
+def mxfp8_kv_linear(x, k_weight: MXWeight, v_weight: MXWeight, head_dim: int = 128):
+    """K and V of one activation from two weights of the same shape, in the attention's layouts: returns
+    ``(k, vt)`` with ``k`` bf16 ``[M, N]`` token-major and ``vt`` as :func:`mxfp8_qkv_linear` returns it."""
+    lib = _lib.load()
+    _check_weight(k_weight, "k_weight")
+    _check_weight(v_weight, "v_weight")
+    codes, scales, row_scale, lead = _as_mx_2d(x)
+    M, K = codes.shape
+    N = k_weight.out_features
+    if k_weight.in_features != K or v_weight.codes.shape != k_weight.codes.shape:
+        raise ValueError(f"activation K={K} does not match the weights {list(k_weight.codes.shape)} and "
+                         f"{list(v_weight.codes.shape)}")
+    w = (k_weight.codes, k_weight.scales, k_weight.col_scale, k_weight.bias,
+         v_weight.codes, v_weight.scales, v_weight.col_scale, v_weight.bias)
+    _lib.require_gpu(codes, scales, row_scale, *w, what="mxfp8_kv_linear")
+    dev = codes.device
+    s_pad = (max(M, 1) + 63) // 64 * 64
+    k = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    if M == 0:  # no tokens: nothing to project, V^T is all padding
+        return k.reshape(*lead, N), torch.zeros((N // head_dim, head_dim, s_pad), dtype=torch.bfloat16, device=dev)
+    vt = torch.empty((N // head_dim, head_dim, s_pad), dtype=torch.bfloat16, device=dev)
+    status = lib.wanmi_mxfp8_gemm_kv(
+        _lib.ptr(codes), _lib.ptr(scales), *(_lib.ptr(t) for t in w), _lib.ptr(row_scale), M, N, K, codes.stride(0),
+        _lib.ptr(k), N, _lib.ptr(vt), s_pad, _lib.stream_of(codes),
+    )
+    _lib.check(status, "wanmi_mxfp8_gemm_kv")
+    return k.reshape(*lead, N), vt
+
+
 def row_quantize_packed(hidden: torch.Tensor) -> torch.Tensor:
     """bf16 rows ``[T, H]`` or ``[B, T, H]`` -> ROW-packed ``[..., H + 4]`` float8_e4m3fn bytes: each
     row's e4m3 codes, then the 4 little-endian bytes of its fp32 dequant scale
