@@ -80,3 +80,24 @@ def test_qkv_tiles_give_the_same_bits(pkg, dev, operands):
         key = (slot & ~15) | (slot & 3) | ((slot & 4) << 1) | ((slot & 8) >> 1)
         want = torch.where((key < m), vt_ref[:, :, :pad], torch.zeros((), dtype=vt.dtype, device=dev))
         assert torch.equal(_bits(vt), _bits(want)), m
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 256, 512), (100, 512, 1024), (129, 256, 512), (1400, 1024, 512), (3900, 256, 512),
+                                   (1000, 5120, 1024), (1560, 5120, 1024)])
+def test_fetching_ahead_keeps_the_bits(pkg, dev, M, N, K):
+    """Products of fewer tiles than CUs, where idle workgroups fetch the operand panels ahead of the tiles: one or
+    several groups of m tiles per XCD, XCDs without a tile, a last tile of one row. The first half of the
+    tokens and the rest, each on its own, must give the same rows."""
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
+    a = pkg.adaln_modulate(x, eps=0.0, norm_type="none", quant="mx")
+    w = pkg.quantize_weight_mx((torch.randn(K, N, device=dev, generator=g) * 0.02).to(torch.bfloat16))
+    y, h = pkg.mxfp8_linear(a, w), M // 2
+    ref = torch.cat([pkg.mxfp8_linear(type(a)(a.codes[i:j], a.scales[i:j]), w) for i, j in ((0, h), (h, M))])
+    assert torch.equal(y, ref)
+    # and each element within the bound of bf16 rounding and fp32 accumulation of the fp64 product
+    v = [t.codes.float().double().reshape(t.codes.shape[0], -1, 32) * torch.exp2(t.scales.double() - 127)[..., None]
+         for t in (a, w)]
+    p, q = (t.reshape(t.shape[0], K) for t in v)
+    bound = 2.0**-8 * (p @ q.T).abs() + 2.0**-14 * (p.abs() @ q.T.abs())
+    assert bool(((y.double() - p @ q.T).abs() <= bound).all())

@@ -86,6 +86,7 @@ struct GemmArgs {
   int64_t M, N, K, lda, ldo;
   int tiles_m, tiles_n;
   int qk_wgs;               // kEpiQkv, 256-feature tiles: workgroups that walk the Q|K tiles
+  int tile_wgs;             // workgroups that compute tiles; the launch's others fetch ahead
 };
 
 // kEpiQkv: the arguments of the V part, a product of its own.
@@ -1065,11 +1066,104 @@ __device__ __forceinline__ void ring_tiles(GemmArgs g, uint8_t (&sWh)[5][kHalfBy
   __builtin_amdgcn_s_waitcnt(0);  // no load may still target LDS when the workgroup retires
 }
 
+// ------------------------------------------------------------------------------------------------
+// Fetching ahead. Where a product fills only part of the chip (one round of fewer tiles than CUs), its
+// workgroups wait for operand lines that miss their XCD's L2: a CU streams about 58 KB/us of such lines
+// against 120 of lines that hit, and all CUs of an XCD reach a panel at the same time, so each line's
+// first request finds it absent and the others wait with it. A few of the idle CUs of every XCD then walk
+// that XCD's panels in the order of k, one 4-byte load per 128-byte line, and leave the lines in its L2.
+// They set their own pace: with two per XCD the tiles overtake them (and the launch ends with them: 70.8
+// against 49.4 us below), with three it makes little difference, and past six they run too far ahead. Results
+// do not depend on it. Measured, weights not in the caches, without / with: 1560 tokens, 5120 columns, 5120
+// deep 49.4 / 45.4 us, 13824 deep 119 / 113; 1000 tokens 36.3 / 33.9 and 120 / 87; 512 tokens 22.3 / 18.4 and
+// 72 / 50; 100 tokens 20.7 / 16.2.
+// ------------------------------------------------------------------------------------------------
+constexpr int kFetchWgs = 5;       // per XCD, at most (5 / 6 / 8: 87.0 / 89.2 / 90.8 us at 1000 tokens, 13824 deep)
+constexpr int kFetchWgsSmall = 6;  // with 128 x 128 tiles (53.7 / 50.2 / 51.4 us at 512 tokens, 13824 deep)
+constexpr int kFetchWgsMin = 4;    // or none
+
+// Tiles of kTm tokens x kTn features in the order of tile_coords (kGroup m tiles per group). Workgroup
+// `j` of `count` on the XCD that takes run `x` of that order. kTwoWeights: the features from vt_col0 on are
+// those of the V weight.
+template <int kTm, int kTn, int kGroup, bool kTwoWeights>
+__device__ __forceinline__ void fetch_ahead(const GemmArgs& g, int x, int j, int count, uint32_t* sink) {
+  const int total = g.tiles_m * g.tiles_n, r = total & 7;
+  const int first = x * (total >> 3) + min(x, r), tiles = (total >> 3) + (x < r ? 1 : 0);
+  if (tiles == 0) return;
+  const int in_group = kGroup * g.tiles_n;
+  const int last = first + tiles - 1;
+  const int g0 = first / in_group, g1 = last / in_group;
+  const int tn0 = first % in_group / min(g.tiles_m - g0 * kGroup, kGroup);
+  const int tn1 = last % in_group / min(g.tiles_m - g1 * kGroup, kGroup);
+  // the run's token rows, and its n tiles: [tn0, tn1], or [tn0, tiles_n) and [0, tn1] over two groups
+  const int64_t m_lo = (int64_t)g0 * kGroup * kTm, m_hi = min(g.M, (int64_t)(g1 + 1) * kGroup * kTm);
+  const int n_hi = g0 == g1 ? tn1 - tn0 + 1 : g.tiles_n - tn0, n_lo = g0 == g1 ? 0 : min(tn1 + 1, tn0);
+  const int m_runs = (int)((m_hi - m_lo + 63) / 64), runs = m_runs + (n_hi + n_lo) * (kTn / 64);  // of 64 rows
+  const int lane = threadIdx.x & 63;
+  auto line = [&](int i) -> uint32_t {  // run i % runs of stage i / runs: the lane's row
+    const int stage = i / runs, b = i % runs;
+    if (b < m_runs) {
+      const int64_t row = min(m_lo + b * 64 + lane, m_hi - 1);
+      return *reinterpret_cast<const uint32_t*>(g.a + row * g.lda + stage * BK);
+    }
+    const int q = (b - m_runs) / (kTn / 64), tn = q < n_hi ? tn0 + q : q - n_hi;
+    int64_t row = (int64_t)tn * kTn + (b - m_runs) % (kTn / 64) * 64 + lane;
+    const uint8_t* w = g.w;
+    if constexpr (kTwoWeights) {
+      if (tn * kTn >= g.vt_col0) {
+        row -= g.vt_col0;
+        w = g.v_w;
+      }
+    }
+    return *reinterpret_cast<const uint32_t*>(w + row * g.K + stage * BK);
+  };
+  const int end = runs * (int)(g.K / BK), step = 4 * count;
+  uint32_t acc = 0;
+  int i = 4 * j + (int)(threadIdx.x >> 6);
+  for (; i + 7 * step < end; i += 8 * step) {  // eight loads in flight per wave
+    uint32_t v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = line(i + k * step);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc ^= v[k];
+  }
+  for (; i < end; i += step) acc ^= line(i);
+  sink[threadIdx.x] = acc;  // LDS: keeps the loads
+}
+
+// The launch's workgroups past the tiles' (a multiple of 8 of them behind the next multiple of 8). In a
+// Q|K and V launch of 256-feature tiles every other one serves the V part, whose tile v runs in workgroup
+// qk_wgs + v; 128 x 128 tiles have one order over both parts.
+template <int EPI, int kTm, int kTn, int kGroup>
+__device__ __forceinline__ void fetch_ahead_wg(GemmArgs g, uint32_t* sink) {
+  const int base = (g.tile_wgs + 7) & ~7;
+  if ((int)blockIdx.x < base) return;
+  int x = blockIdx.x & 7, j = ((int)blockIdx.x - base) >> 3, count = ((int)gridDim.x - base) >> 3;
+  if constexpr (EPI == kEpiQkv && kTn == TN) {
+    const int n_qk = (int)(g.vt_col0 / kTn);
+    if (j & 1) {
+      x = (x - g.qk_wgs) & 7;
+      g.tiles_n -= n_qk;
+      to_v_weight(g);
+      count = count >> 1;
+    } else {
+      g.tiles_n = n_qk;
+      count = (count + 1) >> 1;
+    }
+    j >>= 1;
+  }
+  fetch_ahead<kTm, kTn, kGroup, EPI == kEpiQkv && kTn != TN>(g, x, j, count, sink);
+}
+
 template <int EPI, int kNj>
 __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint8_t sWh[5][kHalfBytes];
   __shared__ __attribute__((aligned(16))) uint8_t sAct[2][64 * kNj * BK];
   __shared__ __attribute__((aligned(16))) uint32_t ssc[2][2 * 256 * 4];
+  if ((int)blockIdx.x >= g.tile_wgs) {
+    fetch_ahead_wg<EPI, 64 * kNj, TN, kGroupM * TM / (64 * kNj)>(g, ssc[0]);
+    return;
+  }
   if constexpr (EPI == kEpiQkv) {
     // workgroups [0, qk_wgs) walk the Q|K tiles, the others the V tiles
     const int wg = (int)blockIdx.x;
@@ -1079,10 +1173,10 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
     } else {
       g.tiles_n -= (int)(g.vt_col0 / TN);
       to_v_weight(g);
-      ring_tiles<kEpiVt, kNj>(g, sWh, sAct, ssc, wg - g.qk_wgs, (int)gridDim.x - g.qk_wgs);
+      ring_tiles<kEpiVt, kNj>(g, sWh, sAct, ssc, wg - g.qk_wgs, g.tile_wgs - g.qk_wgs);
     }
   } else {
-    ring_tiles<EPI, kNj>(g, sWh, sAct, ssc, (int)blockIdx.x, (int)gridDim.x);
+    ring_tiles<EPI, kNj>(g, sWh, sAct, ssc, (int)blockIdx.x, g.tile_wgs);
   }
 }
 
@@ -1339,6 +1433,10 @@ __device__ __forceinline__ void ts_tile(const GemmArgs& g, TsShared& sh, int m0,
 template <int EPI>
 __global__ __launch_bounds__(256, 1) void mxfp8_gemm_tile128_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) TsShared sh;
+  if ((int)blockIdx.x >= g.tile_wgs) {
+    fetch_ahead_wg<EPI, TS, TS, kTsGroupM>(g, sh.sc);
+    return;
+  }
   int m0, n0;
   ts_coords(g, (int)blockIdx.x, m0, n0);
   if constexpr (EPI == kEpiQkv) {
@@ -1456,11 +1554,15 @@ static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t 
   g.tiles_n = (int)(g.N / tn);
   g.qk_wgs = plan.qk_wgs;
   const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+  g.tile_wgs = (int)(plan.nj == 0 ? tiles : std::min(tiles, cus));
+  int64_t wgs = g.tile_wgs;
+  const int64_t idle = (cus - (wgs + 7) / 8 * 8) / 8;  // per XCD
+  if (idle >= kFetchWgsMin) wgs = (wgs + 7) / 8 * 8 + 8 * std::min<int64_t>(idle, plan.nj ? kFetchWgs : kFetchWgsSmall);
+  const dim3 grid((unsigned)wgs);
   if (plan.nj == 0) {
-    launch_tile128(epilogue, dim3((unsigned)tiles), stream, g);
+    launch_tile128(epilogue, grid, stream, g);
     return check_launch("wanmi_mxfp8_gemm");
   }
-  const dim3 grid((unsigned)std::min<int64_t>(tiles, cus));
   if (plan.nj == 4) launch_ring<4>(epilogue, grid, stream, g);
   else if (plan.nj == 3) launch_ring<3>(epilogue, grid, stream, g);
   else launch_ring<2>(epilogue, grid, stream, g);
@@ -1558,6 +1660,7 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
   g.tiles_m = (int)((M + TM - 1) / TM);
   g.tiles_n = (int)(N / TN);
   g.qk_wgs = 0;
+  g.tile_wgs = 0;
   // persistent: one workgroup per CU (the LDS footprint allows no second one)
   const int cus = device_cu_count();
   WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm: cannot query the device's compute units");
