@@ -185,11 +185,42 @@ __device__ __forceinline__ void pipeline_step(const uint8_t* cK, int i_cur, cons
   s_prev = s_cur;
 }
 
+// 32 rows of 256 bytes (queries of one head, or their RoPE table rows), `stride` bytes apart, loaded as whole
+// 128-byte row halves: load t covers rows 8 (t & 3) .. + 7, half t >> 2 of each (lane l: row 8 (t & 3) +
+// (l >> 3), 16-byte chunk l & 7), eight lines per instruction. Gathered straight into the MFMA's lane layout
+// each instruction touched 32 bytes of 32 rows, and every line was fetched four times.
+__device__ __forceinline__ void load_rows(__amdgpu_buffer_rsrc_t r, uint32_t stride, int lane, u32x4 (&v)[8]) {
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    v[t] = __builtin_amdgcn_raw_buffer_load_b128(
+        r, (uint32_t)(8 * (t & 3) + (lane >> 3)) * stride + (uint32_t)(128 * (t >> 2) + 16 * (lane & 7)), 0, 0);
+}
+// The loaded rows into the lane layout: v[t] = bytes 32 t + 16 hq .. of row lane & 31, through 4 KiB of LDS
+// private to the wave, one half row at a time, held as [row][8 chunks] with chunk c ^ ((row >> 1) & 7): writes
+// (two rows of eight chunks per 16 lanes) and reads (sixteen rows of one chunk) without bank conflicts. A
+// wave's LDS operations complete in order.
+__device__ __forceinline__ void rows_to_lanes(uint8_t* scratch, int lane, u32x4 (&v)[8]) {
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 8 * t + (lane >> 3);
+      *reinterpret_cast<u32x4*>(scratch + row * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4)) = v[4 * hf + t];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = lane & 31, c = 2 * t + (lane >> 5);
+      v[4 * hf + t] = *reinterpret_cast<const u32x4*>(scratch + row * 128 + ((c ^ ((row >> 1) & 7)) << 4));
+    }
+  }
+}
+
 // The wave's 32 queries (q0 + col) of head h as B operands: lane holds d = 16 t + 8 hq .. +7 of query
 // q0 + col in qf[t], pre-scaled by s log2(e), normalized and rotated first where the caller asks for
-// it. `sgam`: the wave's 1 KiB of LDS for the head's gamma. Returns the query's bound c in log2 units.
+// it. `sgam`: the wave's 1 KiB of LDS for the head's gamma, `scratch`: 4 KiB of LDS that nothing else
+// touches meanwhile. Returns the query's bound c in log2 units.
 __device__ __forceinline__ float load_queries(const AttnArgs& a, int h, int64_t q0, int lane, int col, int hq, float* sgam,
-                                              bf16x8 (&qf)[8]) {
+                                              uint8_t* scratch, bf16x8 (&qf)[8]) {
 #pragma clang fp contract(off)
   // Q through a descriptor based at the wave's first query; rows >= Sq read as zero.
   const int64_t qvalid = a.Sq - q0 < 32 ? (a.Sq - q0 > 0 ? a.Sq - q0 : 0) : 32;
@@ -210,18 +241,15 @@ __device__ __forceinline__ float load_queries(const AttnArgs& a, int h, int64_t 
   const __amdgpu_buffer_rsrc_t r_sn =
       attn_rsrc(qrope ? a.q_sin + (qvalid > 0 ? q0 * 64 : 0) : nullptr, qrope && qvalid > 0 ? qvalid * 64 * 4 : 0);
   u32x4 qv[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-    qv[t] = __builtin_amdgcn_raw_buffer_load_b128(r_q, (uint32_t)((col * a.q_ss + 16 * t + 8 * hq) * 2), 0, 0);
-  if (qprep) {
+  load_rows(r_q, (uint32_t)(a.q_ss * 2), lane, qv);
+  if (!qprep) {
+    rows_to_lanes(scratch, lane, qv);
+  } else {
     // the RoPE tables only when there is a rotation (the cross-attention query has none)
     u32x4 cv[8], sv[8];
     if (qrope) {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        cv[t] = __builtin_amdgcn_raw_buffer_load_b128(r_cs, (uint32_t)((col * 64 + 8 * t + 4 * hq) * 4), 0, 0);
-        sv[t] = __builtin_amdgcn_raw_buffer_load_b128(r_sn, (uint32_t)((col * 64 + 8 * t + 4 * hq) * 4), 0, 0);
-      }
+      load_rows(r_cs, 256, lane, cv);
+      load_rows(r_sn, 256, lane, sv);
     } else {
 #pragma unroll
       for (int t = 0; t < 8; ++t) cv[t] = sv[t] = u32x4{0u, 0u, 0u, 0u};
@@ -271,6 +299,11 @@ __device__ __forceinline__ float load_queries(const AttnArgs& a, int h, int64_t 
     }
     // every load of the prologue is in (the math below needs them all), the gamma copy included
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    rows_to_lanes(scratch, lane, qv);
+    if (qrope) {
+      rows_to_lanes(scratch, lane, cv);
+      rows_to_lanes(scratch, lane, sv);
+    }
     const float4* gl = reinterpret_cast<const float4*>(sgam);
     // x_hat = bf16((x rrms) gamma), then the pair rotation (a cos - b sin, a sin + b cos) -> bf16:
     // the same operations, in the same order, as the separate Q/K preparation pass
@@ -456,7 +489,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int h, int qb
   if (ntiles > 2) issue_tile(2);
 
   bf16x8 qf[8];
-  const float c2 = load_queries(a, h, q0, lane, col, hq, sgam[wave], qf);
+  // (scratch: ring slot 3, loaded first with tile 3, after two barriers)
+  static_assert(kStages == 4 && kWaves == 8);
+  const float c2 =
+      load_queries(a, h, q0, lane, col, hq, sgam[wave], (wave < 4 ? sK[3] : sV[3]) + (wave & 3) * 4096, qf);
   f32x16 negc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) negc[r] = -c2;
@@ -636,9 +672,10 @@ __device__ __forceinline__ void attention_wave_jobs(const AttnArgs& a, int L, ui
       }
     };
     issue_k(part);
-    issue_v(part);
     bf16x8 qf[8];
-    const float c2 = load_queries(a, h, q0, lane, col, hq, sgam[wave], qf);
+    const float c2 = load_queries(a, h, q0, lane, col, hq, sgam[wave], vb, qf);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // its scratch reads are done
+    issue_v(part);
     f32x16 negc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) negc[r] = -c2;
