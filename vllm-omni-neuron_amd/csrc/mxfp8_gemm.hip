@@ -1072,33 +1072,41 @@ __device__ __forceinline__ void ring_tiles(GemmArgs g, uint8_t (&sWh)[5][kHalfBy
 // against 120 of lines that hit, and all CUs of an XCD reach a panel at the same time, so each line's
 // first request finds it absent and the others wait with it. A few of the idle CUs of every XCD then walk
 // that XCD's panels in the order of k, one 4-byte load per 128-byte line, and leave the lines in its L2.
-// They set their own pace: with two per XCD the tiles overtake them (and the launch ends with them: 70.8
-// against 49.4 us below), with three it makes little difference, and past six they run too far ahead. Results
-// do not depend on it. Measured, weights not in the caches, without / with: 1560 tokens, 5120 columns, 5120
-// deep 49.4 / 45.4 us, 13824 deep 119 / 113; 1000 tokens 36.3 / 33.9 and 120 / 87; 512 tokens 22.3 / 18.4 and
-// 72 / 50; 100 tokens 20.7 / 16.2.
+// They set their own pace, and the launch ends with them if the tiles overtake them (fetch_wgs says how many
+// it takes). Results do not depend on it. Measured, weights not in the caches, without / with: 1560 tokens,
+// 5120 columns, 5120 deep 49.4 / 45.4 us, 13824 deep 119 / 113; 1000 tokens 36.3 / 33.9 and 120 / 87; 512
+// tokens 22.3 / 18.4 and 72 / 50; 100 tokens 20.7 / 16.2.
 // ------------------------------------------------------------------------------------------------
-constexpr int kFetchWgs = 5;       // per XCD, at most (5 / 6 / 8: 87.0 / 89.2 / 90.8 us at 1000 tokens, 13824 deep)
-constexpr int kFetchWgsSmall = 6;  // with 128 x 128 tiles (53.7 / 50.2 / 51.4 us at 512 tokens, 13824 deep)
-constexpr int kFetchWgsMin = 4;    // or none
+
+// What the run of tiles of XCD `x` reads: its token rows [m_lo, m_hi) and n tiles, [n0, n0 + n_hi) and, over
+// several groups, [0, n_lo) (kGroup m tiles of kTm tokens per group, in the order of tile_coords).
+struct RunPanels {
+  int64_t m_lo, m_hi;
+  int n0, n_hi, n_lo;
+};
+template <int kTm, int kGroup>
+__host__ __device__ __forceinline__ RunPanels run_panels(int64_t M, int tiles_m, int tiles_n, int x) {
+  const int total = tiles_m * tiles_n, r = total & 7;
+  const int first = x * (total >> 3) + (x < r ? x : r), tiles = (total >> 3) + (x < r ? 1 : 0);
+  if (tiles == 0) return RunPanels{0, 0, 0, 0, 0};
+  const int in_group = kGroup * tiles_n, last = first + tiles - 1;
+  const int g0 = first / in_group, g1 = last / in_group;
+  const int s0 = tiles_m - g0 * kGroup, s1 = tiles_m - g1 * kGroup;  // m tiles of the groups
+  const int tn0 = first % in_group / (s0 < kGroup ? s0 : kGroup), tn1 = last % in_group / (s1 < kGroup ? s1 : kGroup);
+  const int64_t m_end = (int64_t)(g1 + 1) * kGroup * kTm;
+  return RunPanels{(int64_t)g0 * kGroup * kTm, m_end < M ? m_end : M, tn0, g0 == g1 ? tn1 - tn0 + 1 : tiles_n - tn0,
+                   g0 == g1 ? 0 : (tn1 + 1 < tn0 ? tn1 + 1 : tn0)};
+}
 
 // Tiles of kTm tokens x kTn features in the order of tile_coords (kGroup m tiles per group). Workgroup
 // `j` of `count` on the XCD that takes run `x` of that order. kTwoWeights: the features from vt_col0 on are
 // those of the V weight.
 template <int kTm, int kTn, int kGroup, bool kTwoWeights>
 __device__ __forceinline__ void fetch_ahead(const GemmArgs& g, int x, int j, int count, uint32_t* sink) {
-  const int total = g.tiles_m * g.tiles_n, r = total & 7;
-  const int first = x * (total >> 3) + min(x, r), tiles = (total >> 3) + (x < r ? 1 : 0);
-  if (tiles == 0) return;
-  const int in_group = kGroup * g.tiles_n;
-  const int last = first + tiles - 1;
-  const int g0 = first / in_group, g1 = last / in_group;
-  const int tn0 = first % in_group / min(g.tiles_m - g0 * kGroup, kGroup);
-  const int tn1 = last % in_group / min(g.tiles_m - g1 * kGroup, kGroup);
-  // the run's token rows, and its n tiles: [tn0, tn1], or [tn0, tiles_n) and [0, tn1] over two groups
-  const int64_t m_lo = (int64_t)g0 * kGroup * kTm, m_hi = min(g.M, (int64_t)(g1 + 1) * kGroup * kTm);
-  const int n_hi = g0 == g1 ? tn1 - tn0 + 1 : g.tiles_n - tn0, n_lo = g0 == g1 ? 0 : min(tn1 + 1, tn0);
-  const int m_runs = (int)((m_hi - m_lo + 63) / 64), runs = m_runs + (n_hi + n_lo) * (kTn / 64);  // of 64 rows
+  const RunPanels p = run_panels<kTm, kGroup>(g.M, g.tiles_m, g.tiles_n, x);
+  if (p.m_hi == 0) return;
+  const int64_t m_lo = p.m_lo, m_hi = p.m_hi;
+  const int m_runs = (int)((m_hi - m_lo + 63) / 64), runs = m_runs + (p.n_hi + p.n_lo) * (kTn / 64);  // of 64 rows
   const int lane = threadIdx.x & 63;
   auto line = [&](int i) -> uint32_t {  // run i % runs of stage i / runs: the lane's row
     const int stage = i / runs, b = i % runs;
@@ -1106,7 +1114,7 @@ __device__ __forceinline__ void fetch_ahead(const GemmArgs& g, int x, int j, int
       const int64_t row = min(m_lo + b * 64 + lane, m_hi - 1);
       return *reinterpret_cast<const uint32_t*>(g.a + row * g.lda + stage * BK);
     }
-    const int q = (b - m_runs) / (kTn / 64), tn = q < n_hi ? tn0 + q : q - n_hi;
+    const int q = (b - m_runs) / (kTn / 64), tn = q < p.n_hi ? p.n0 + q : q - p.n_hi;
     int64_t row = (int64_t)tn * kTn + (b - m_runs) % (kTn / 64) * 64 + lane;
     const uint8_t* w = g.w;
     if constexpr (kTwoWeights) {
@@ -1547,6 +1555,41 @@ static TilePlan select_qkv_tile(int64_t M, int64_t qk, int64_t v, int64_t cus, i
   return best;
 }
 
+// Workgroups per XCD that fetch ahead of a product of one round: as many as walk the longest run's panels at
+// twice the tiles' pace, one CU touching about 900 lines per us and a k stage (one line per row) taking the
+// tiles of nj `kStageNs`; none if the idle CUs cannot at least keep pace. 1000 tokens, 13824 deep, 0 / 2 / 3 /
+// 4 / 5 / 6 / 8 of them: 120 / 117 / 108 / 92 / 87 / 89 / 91 us; 512 tokens 72 / 74 / 70 / 61 / 54 / 50 / 51;
+// four where the rule asks for thirteen (2000 tokens) 127 -> 212. Not with 256 x 256 tiles, whose MFMAs take
+// as long as the loads (216 tiles: 56.5 -> 58.2 us).
+constexpr int kStageNs[5] = {560, 0, 920, 1100, 0};
+
+template <int kTm, int kTn, int kGroup>
+static int64_t fetch_wgs(int64_t M, int tiles_m, int tiles_n, int64_t idle, int nj) {
+  int64_t lines = 0;
+  for (int x = 0; x < 8; ++x) {
+    const RunPanels p = run_panels<kTm, kGroup>(M, tiles_m, tiles_n, x);
+    lines = std::max(lines, p.m_hi - p.m_lo + (int64_t)(p.n_hi + p.n_lo) * kTn);
+  }
+  const int64_t pace = 900 * kStageNs[nj] / 1000;  // lines per stage and workgroup
+  const int64_t n = std::min(idle, (2 * lines + pace / 2) / pace);
+  return n * pace >= lines ? n : 0;
+}
+
+// The same for one launch (`tiles_n` as launched); Q|K and V on 256-feature tiles have as many each.
+static int64_t fetch_wgs(int epilogue, const TilePlan& plan, const GemmArgs& g, int64_t idle) {
+  auto count = [&](int tiles_n, int64_t n) -> int64_t {
+    if (plan.nj == 0) return fetch_wgs<TS, TS, kTsGroupM>(g.M, g.tiles_m, tiles_n, n, 0);
+    if (plan.nj == 2) return fetch_wgs<128, TN, kGroupM * TM / 128>(g.M, g.tiles_m, tiles_n, n, 2);
+    if (plan.nj == 3) return fetch_wgs<192, TN, kGroupM * TM / 192>(g.M, g.tiles_m, tiles_n, n, 3);
+    return 0;
+  };
+  if (idle <= 0) return 0;
+  if (epilogue != kEpiQkv || plan.nj == 0) return count(g.tiles_n, idle);
+  const int n_qk = (int)(g.vt_col0 / TN);
+  const int64_t a = count(n_qk, idle / 2), b = count(g.tiles_n - n_qk, idle / 2);
+  return a > 0 && b > 0 ? 2 * std::max(a, b) : 0;
+}
+
 // One launch of the pipelined kernels with tile `plan` (g's tile counts are filled in here).
 static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t cus, hipStream_t stream) {
   const int64_t tm = plan.nj ? 64 * plan.nj : TS, tn = plan.nj ? TN : TS;
@@ -1557,7 +1600,7 @@ static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t 
   g.tile_wgs = (int)(plan.nj == 0 ? tiles : std::min(tiles, cus));
   int64_t wgs = g.tile_wgs;
   const int64_t idle = (cus - (wgs + 7) / 8 * 8) / 8;  // per XCD
-  if (idle >= kFetchWgsMin) wgs = (wgs + 7) / 8 * 8 + 8 * std::min<int64_t>(idle, plan.nj ? kFetchWgs : kFetchWgsSmall);
+  if (const int64_t n = fetch_wgs(epilogue, plan, g, idle)) wgs = (wgs + 7) / 8 * 8 + 8 * n;
   const dim3 grid((unsigned)wgs);
   if (plan.nj == 0) {
     launch_tile128(epilogue, grid, stream, g);
