@@ -616,7 +616,7 @@ __device__ __forceinline__ void add_partial(const uint8_t* other, const float* s
 // through its own 16 KiB of LDS (K of one half, V^T of one half: the next half's K is requested once
 // this half's K is in registers, and likewise V^T), without a barrier until the sums are added. Bound by
 // that stream: nothing is shared between waves, so the operand traffic per MFMA is eight times a whole
-// block's, and a workgroup takes 2.6 / job_waves of a block's time per key tile. 1560 queries and keys,
+// block's, and a workgroup takes 2.2 / job_waves of a block's time per key tile. 1560 queries and keys,
 // 40 heads (240 blocks, 40 remainders of 24 queries): 81.3 us in blocks throughout (a second round for
 // the remainders), 55.0 with two waves per job, 65.9 with four, 67.5 with eight; 512 keys: 40.1 -> 24.1.
 // Splitting the keys of 128-query runs over two groups of waves that share tiles (98.9 against 103.9 us
@@ -1344,7 +1344,7 @@ struct AttnPlan {
 // A workgroup's cost, a fixed part (the queries' load and preparation, the first tiles, the output) and
 // a part per key tile, fitted to launches of 40 heads over 512 to 32760 queries: about 1.6 us per tile.
 constexpr int64_t kBlockFixed = 700, kBlockTile = 100;
-constexpr int64_t kJobFixed = 500, kJobTile = 260;                       // kJobTile / job_waves per tile
+constexpr int64_t kJobFixed = 800, kJobTile = 220;                       // kJobTile / job_waves per tile
 constexpr int64_t kGroupFixed = 400, kGroupHead = 300, kGroupTile = 100;  // per head, per head and tile
 
 // When every CU takes one workgroup at a time in grid order (blocks, then jobs), the time at which the
