@@ -32,7 +32,7 @@
 // scheduling barriers (10% faster than the compiler's own order, which moved MFMAs across the
 // stage barriers and left the reads of a slice exposed).
 //
-// The kernel is persistent: one workgroup per CU walks tiles v = blockIdx.x, + gridDim.x, ... in an
+// The kernel is persistent: one workgroup per CU walks tiles v = blockIdx.x, + tile_wgs, ... in an
 // order where each XCD (workgroup ids are dealt round-robin over 8 XCDs) owns a contiguous,
 // L2-friendly run of tiles grouped 4 deep along m (measured against 2, 8 and 16: 1-5% faster). The
 // next tile's first stage is loaded while the current tile's epilogue runs, so the epilogue overlaps
@@ -1750,8 +1750,8 @@ static int projection_with_vt(const uint8_t* a_codes, const uint8_t* a_scales, c
                               int64_t K, int64_t lda, const WeightPart& w, int64_t n_out, const WeightPart& v, int64_t n_v,
                               void* out, int64_t ldo, float* row_sumsq, int64_t sumsq_cols, void* vt, int64_t vt_ld,
                               void* stream) {
-  // In one launch where that saves a round of tiles (one latent frame, 1560 tokens: 172 -> 121 us) or one
-  // launch as such; two launches otherwise (at 32760 tokens both parts are whole rounds).
+  // In one launch where that costs no more rounds of tiles (one latent frame, 1560 tokens: 172 -> 121 us);
+  // two launches otherwise (at 32760 tokens both parts are whole rounds).
   if ((K / BK) % 4 == 0) {
     const int cus = device_cu_count();
     WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm_qkv: cannot query the device's compute units");
