@@ -1,0 +1,67 @@
+"""The GEMM's launch rules (csrc/gemm_plan.h) on the CPU, over their whole range.
+
+The header is plain C++; a small program compiled here walks what the kernels would walk. No GPU."""
+
+import pathlib
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+CSRC = ROOT / "vllm-omni-neuron_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """Compiles a C++ main that includes gemm_plan.h and returns what it prints."""
+
+    def go(name: str, body: str) -> str:
+        d = tmp_path_factory.mktemp(name)
+        (d / "main.cc").write_text('#include "gemm_plan.h"\n#include <cstdio>\n#include <vector>\n'
+                                   "using namespace wanmi;\n" + body)
+        subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Wextra", "-Werror", f"-I{CSRC}", str(d / "main.cc"),
+                        "-o", str(d / "main")], check=True)
+        return subprocess.run([str(d / "main")], check=True, capture_output=True, text=True, timeout=300).stdout
+
+    return go
+
+
+# Q|K and V widths: one and two weights of the model's 5120, grouped K/V heads (V narrow against Q|K), V wider
+QKV_SWEEP = r"""
+struct Width { int64_t qk, v; };
+static const Width kWidths[] = {{10240, 5120}, {5120, 5120}, {6144, 1024}, {5120, 1024}, {5120, 512}, {5120, 256},
+                                {10240, 2560}, {10240, 256}, {256, 256}, {256, 5120}, {1024, 10240}, {768, 512}};
+template <class F>
+void sweep(F f) {
+  for (const Width& w : kWidths)
+    for (int64_t cus : {256, 304, 128, 64, 38, 8, 2})
+      for (int64_t M = 1; M <= 33000; M += M < 4200 && cus == 256 ? 1 : 61) {
+        const int64_t vt_ld = (M + 63) / 64 * 64;
+        f(M, w.qk, w.v, cus, select_qkv_tile(M, w.qk, w.v, cus, vt_ld));
+      }
+}
+"""
+
+
+def test_qkv_launch_has_a_tile_for_every_workgroup(run):
+    """Q|K and V in one launch: both parts get a workgroup, and neither more workgroups than it has tiles (a
+    workgroup without a tile of its own would compute one past the end of the weight and of V^T)."""
+    out = run("qkv", QKV_SWEEP + r"""
+int main() {
+  long checked = 0, bad = 0;
+  sweep([&](int64_t M, int64_t qk, int64_t v, int64_t cus, const TilePlan& p) {
+    if (p.nj == 0 || p.cost == INT64_MAX) return;
+    const int64_t mt = ceil_div(M, 64 * p.nj), tq = mt * (qk / TN), tv = mt * (v / TN);
+    const int64_t v_wgs = tile_workgroups(p, tq + tv, cus) - p.qk_wgs;
+    const int64_t rounds = std::max(ceil_div(tq, std::max<int64_t>(p.qk_wgs, 1)), ceil_div(tv, std::max<int64_t>(v_wgs, 1)));
+    ++checked;
+    if (p.qk_wgs < 1 || p.qk_wgs > tq || v_wgs < 1 || v_wgs > tv || p.qk_wgs + v_wgs > cus || p.cost != kTileCost[p.nj] * rounds) {
+      if (bad++ < 5)
+        printf("M=%ld qk=%ld v=%ld cus=%ld: nj=%d, %d workgroups for %ld tiles, %ld for %ld\n", (long)M, (long)qk, (long)v,
+               (long)cus, p.nj, p.qk_wgs, (long)tq, (long)v_wgs, (long)tv);
+    }
+  });
+  printf("checked %ld bad %ld\n", checked, bad);
+}
+""")
+    assert out.splitlines()[-1].startswith("checked ") and out.endswith(" bad 0\n"), out

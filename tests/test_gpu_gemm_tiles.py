@@ -82,6 +82,38 @@ def test_qkv_tiles_give_the_same_bits(pkg, dev, operands):
         assert torch.equal(_bits(vt), _bits(want)), m
 
 
+# V narrower than Q|K / 2 (grouped K/V heads) and wider: the split of the CUs between the parts follows the widths
+@pytest.mark.parametrize("M,qk,v", [(2561, 6144, 1024), (2880, 6144, 1024), (3840, 6144, 1024), (2048, 10240, 2560),
+                                    (3073, 5120, 256), (4416, 5120, 256), (3000, 1024, 10240)])
+def test_qkv_of_any_widths_writes_its_own_outputs_only(pkg, dev, M, qk, v):
+    """Q|K, V^T and the partial sums inside larger buffers, against one product per part and the transposing
+    pass; what lies around them must stay as it was."""
+    K, guard = 512, 1 << 20
+    g = torch.Generator(device=dev).manual_seed(M + qk)
+    x = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
+    a = pkg.adaln_modulate(x, eps=0.0, norm_type="none", quant="mx")
+    w = pkg.quantize_weight_mx((torch.randn(K, qk + v, device=dev, generator=g) * 0.02).to(torch.bfloat16),
+                               torch.randn(qk + v, device=dev, generator=g) * 0.1)
+    ld = (M + 63) // 64 * 64
+    sizes = {"qk": M * qk, "vt": v * ld, "ss": M * (qk // 128)}
+    bufs = {n: torch.full((k + 2 * guard,), -7.0, dtype=torch.float32 if n == "ss" else torch.bfloat16, device=dev)
+            for n, k in sizes.items()}
+    own = {n: bufs[n][guard : guard + k] for n, k in sizes.items()}
+    ptr, lib = pkg._lib.ptr, pkg._lib.load()
+    st = lib.wanmi_mxfp8_gemm_qkv(ptr(a.codes), ptr(a.scales), ptr(w.codes), ptr(w.scales), None, None, ptr(w.bias), M,
+                                  qk + v, K, K, ptr(own["qk"]), qk, ptr(own["ss"]), qk, ptr(own["vt"]), qk, ld,
+                                  pkg._lib.stream_of(a.codes))
+    pkg._lib.check(st, "wanmi_mxfp8_gemm_qkv")
+    for n, k in sizes.items():
+        assert bool((bufs[n][:guard] == -7.0).all()) and bool((bufs[n][guard + k :] == -7.0).all()), n
+    ss = torch.empty(M, qk // 128, device=dev)
+    y = pkg.mxfp8_linear(a, _cols(w, qk), row_sumsq=ss, sumsq_cols=qk)
+    rest = w._replace(codes=w.codes[qk:], scales=w.scales[qk:], bias=w.bias[qk:])
+    vt, _ = pkg.attention_ops.transpose_heads(pkg.mxfp8_linear(a, rest).view(M, v // 128, 128))
+    assert torch.equal(own["qk"].view(M, qk), y) and torch.equal(own["ss"].view(M, -1), ss)
+    assert torch.equal(own["vt"].view(vt.shape), vt)
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 256, 512), (100, 512, 1024), (129, 256, 512), (1400, 1024, 512), (3900, 256, 512),
                                    (1000, 5120, 1024), (1560, 5120, 1024)])
 def test_fetching_ahead_keeps_the_bits(pkg, dev, M, N, K):

@@ -48,18 +48,14 @@
 // quantize_mx in mlp_cte_mx_quantization.py:113-154); the torch statement is _mlp_ref_standard
 // (kernels/nkilib/core/mlp/mlp_torch.py:401-599).
 #include "wanmi_common.h"
-
-#include <algorithm>
+#include "gemm_plan.h"
 
 namespace wanmi {
 
-constexpr int TN = 256;  // weight rows (output features) per tile
-constexpr int TM = 256;  // tokens per tile
 constexpr int BK = 128;  // k bytes per stage (4 MX blocks)
 constexpr int kStageBytes = TN * BK + TM * BK;  // e4m3 codes of one stage (W rows, then A rows)
 constexpr int kScaleGroup = 4;                    // stages per scale load (16 bytes per row)
 constexpr int kVecFloats = 4 * 256;  // per tile: bias[n], col_scale[n], gate[n], row_scale[m]
-constexpr int kGroupM = 4;  // m tiles per group (4: the XCD's 32 concurrent tiles are 4 m x 8 n)
 
 struct GemmArgs {
   const uint8_t* a;         // [M, lda]
@@ -194,22 +190,13 @@ struct TileLoads {
   int64_t m0, n0, m_valid;
 };
 
-// Tile v of the grid of tiles_m x tiles_n tiles of kTm tokens x 256 features: XCD v & 7 takes a
-// contiguous run of the order that walks groups of m tiles (about 1024 tokens deep) along n.
+// Tile v of the grid of tiles_m x tiles_n tiles of kTm tokens x 256 features (groups of m tiles about 1024
+// tokens deep).
 template <int kTm>
 __device__ __forceinline__ void tile_coords(const GemmArgs& g, int v, int64_t& m0, int64_t& n0) {
-  constexpr int kGroup = kGroupM * TM / kTm;
-  const int total = g.tiles_m * g.tiles_n;
-  const int x = v & 7, r = total & 7;
-  const int pid = x * (total >> 3) + min(x, r) + (v >> 3);
-  const int in_group = kGroup * g.tiles_n;
-  const int group = pid / in_group;
-  const int first_m = group * kGroup;
-  const int gsz = min(g.tiles_m - first_m, kGroup);
-  const int tm = first_m + (pid % in_group) % gsz;
-  const int tn = (pid % in_group) / gsz;
-  n0 = (int64_t)tn * TN;
-  m0 = (int64_t)tm * kTm;
+  const TileAt t = tile_at(v, g.tiles_m, g.tiles_n, kGroupM * TM / kTm);
+  n0 = (int64_t)t.tn * TN;
+  m0 = (int64_t)t.tm * kTm;
 }
 
 template <int kTm = TM>
@@ -1078,26 +1065,6 @@ __device__ __forceinline__ void ring_tiles(GemmArgs g, uint8_t (&sWh)[5][kHalfBy
 // tokens 22.3 / 18.4 and 72 / 50; 100 tokens 20.7 / 16.2.
 // ------------------------------------------------------------------------------------------------
 
-// What the run of tiles of XCD `x` reads: its token rows [m_lo, m_hi) and n tiles, [n0, n0 + n_hi) and, over
-// several groups, [0, n_lo) (kGroup m tiles of kTm tokens per group, in the order of tile_coords).
-struct RunPanels {
-  int64_t m_lo, m_hi;
-  int n0, n_hi, n_lo;
-};
-template <int kTm, int kGroup>
-__host__ __device__ __forceinline__ RunPanels run_panels(int64_t M, int tiles_m, int tiles_n, int x) {
-  const int total = tiles_m * tiles_n, r = total & 7;
-  const int first = x * (total >> 3) + (x < r ? x : r), tiles = (total >> 3) + (x < r ? 1 : 0);
-  if (tiles == 0) return RunPanels{0, 0, 0, 0, 0};
-  const int in_group = kGroup * tiles_n, last = first + tiles - 1;
-  const int g0 = first / in_group, g1 = last / in_group;
-  const int s0 = tiles_m - g0 * kGroup, s1 = tiles_m - g1 * kGroup;  // m tiles of the groups
-  const int tn0 = first % in_group / (s0 < kGroup ? s0 : kGroup), tn1 = last % in_group / (s1 < kGroup ? s1 : kGroup);
-  const int64_t m_end = (int64_t)(g1 + 1) * kGroup * kTm;
-  return RunPanels{(int64_t)g0 * kGroup * kTm, m_end < M ? m_end : M, tn0, g0 == g1 ? tn1 - tn0 + 1 : tiles_n - tn0,
-                   g0 == g1 ? 0 : (tn1 + 1 < tn0 ? tn1 + 1 : tn0)};
-}
-
 // Tiles of kTm tokens x kTn features in the order of tile_coords (kGroup m tiles per group). Workgroup
 // `j` of `count` on the XCD that takes run `x` of that order. kTwoWeights: the features from vt_col0 on are
 // those of the V weight.
@@ -1177,9 +1144,11 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
     const int wg = (int)blockIdx.x;
     if (wg < g.qk_wgs) {
       g.tiles_n = (int)(g.vt_col0 / TN);
+      if (wg >= g.tiles_m * g.tiles_n) return;  // never more workgroups than tiles, by select_qkv_tile
       ring_tiles<WANMI_EPI_BF16, kNj>(g, sWh, sAct, ssc, wg, g.qk_wgs);
     } else {
       g.tiles_n -= (int)(g.vt_col0 / TN);
+      if (wg - g.qk_wgs >= g.tiles_m * g.tiles_n) return;
       to_v_weight(g);
       ring_tiles<kEpiVt, kNj>(g, sWh, sAct, ssc, wg - g.qk_wgs, g.tile_wgs - g.qk_wgs);
     }
@@ -1205,23 +1174,15 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
 // the bytes per CU, and the smallest tile wins as long as its grid fits one round. Measured, 512
 // tokens, 5120 x 5120: 53.9 us with 256 x 256 tiles, 23.3 us here; 13824 deep: 126 and 49 us.
 // ------------------------------------------------------------------------------------------------
-constexpr int TS = 128;                      // features and tokens per tile
 constexpr int kTsStage = 2 * TS * BK;        // bytes of codes per stage
 constexpr int kTsLoads = 8;                  // code loads per wave per stage
 constexpr int kTsStages = 4;                 // LDS ring depth in stages
-constexpr int kTsGroupM = 8;                 // m tiles per group of the tile order
 
-// Tile of workgroup v: XCD v & 7 takes a contiguous run of the grouped order (any total).
+// Tile of workgroup v.
 __device__ __forceinline__ void ts_coords(const GemmArgs& g, int v, int& m0, int& n0) {
-  const int total = g.tiles_m * g.tiles_n;
-  const int x = v & 7, q = total >> 3, r = total & 7;
-  const int pid = x * q + min(x, r) + (v >> 3);
-  const int in_group = kTsGroupM * g.tiles_n;
-  const int group = pid / in_group;
-  const int first_m = group * kTsGroupM;
-  const int gsz = min(g.tiles_m - first_m, kTsGroupM);
-  m0 = (first_m + (pid % in_group) % gsz) * TS;
-  n0 = ((pid % in_group) / gsz) * TS;
+  const TileAt t = tile_at(v, g.tiles_m, g.tiles_n, kTsGroupM);
+  m0 = t.tm * TS;
+  n0 = t.tn * TS;
 }
 
 struct TsShared {
@@ -1496,86 +1457,7 @@ static void launch_simple(int epilogue, dim3 grid, hipStream_t stream, const Gem
 }  // namespace wanmi
 
 namespace wanmi {
-// Which tile a product of M tokens takes on `cus` CUs (one workgroup each), and at what cost.
-struct TilePlan {
-  int nj;      // token fragments per wave of the 256-feature kernel (tiles of 64 nj tokens); 0: 128 x 128 tiles
-  int64_t cost;
-  int qk_wgs;  // kEpiQkv on 256-feature tiles
-};
-
-// Every CU takes one tile at a time, so a product costs its rounds of `cus` tiles times one tile's
-// time, which is the same for all full tiles of a kind but not proportional to the tile: the loads
-// bound it, and a smaller tile needs more of them per flop. Measured per k stage in rounds of 5120 x
-// 5120 (one to twenty rounds): 256 x 256 tiles 1.30-1.60 us, 192 tokens x 256 1.05-1.25, 128 x 256
-// 0.87-0.97, 128 x 128 0.55-0.58; K = 13824 and the GELU epilogue give the same ratios within 3%. A
-// smaller tile pays where it saves a round or fills the only one: 5120 x 5120 at 512 tokens 54 -> 23 us
-// (128 x 128), 1024 55 -> 37 (128 x 256), 1560 57 -> 47 (192), 3120 119 -> 83 (128 x 256), 4100 122 ->
-// 101 (192); at 5500 tokens 130 against 146 (192) and at 16380 338 against 364, the 256 x 256 tile.
-constexpr int kTileCost[5] = {40, 0, 67, 82, 100};  // by nj (0: 128 x 128 tiles)
-
-inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Best tile for n output columns (a multiple of 256); a larger tile wins a tie. V^T columns are
-// written for whole tiles only, so tiles that end before vt_ld are not taken.
-static TilePlan select_tile(int64_t M, int64_t n, int64_t cus, int64_t vt_ld) {
-  TilePlan best{4, kTileCost[4] * ceil_div(ceil_div(M, 256) * (n / TN), cus), 0};
-  for (int nj : {3, 2, 0}) {
-    const int64_t tm = nj ? 64 * nj : TS, tn = nj ? TN : TS;
-    const int64_t mt = ceil_div(M, tm);
-    if (mt * tm < vt_ld) continue;
-    const int64_t cost = kTileCost[nj] * ceil_div(mt * (n / tn), cus);
-    if (cost < best.cost) best = TilePlan{nj, cost, 0};
-  }
-  return best;
-}
-
-// The same for Q|K (qk columns) and V (v columns) in one launch: on 256-feature tiles the CUs are split
-// between the two parts so that the longer one is shortest; 128 x 128 tiles mix freely.
-static TilePlan select_qkv_tile(int64_t M, int64_t qk, int64_t v, int64_t cus, int64_t vt_ld) {
-  TilePlan best{4, INT64_MAX, 0};
-  for (int nj : {4, 3, 2, 0}) {
-    const int64_t tm = nj ? 64 * nj : TS;
-    const int64_t mt = ceil_div(M, tm);
-    if (mt * tm < vt_ld) continue;
-    if (nj == 0) {
-      const int64_t cost = kTileCost[0] * ceil_div(mt * ((qk + v) / TS), cus);
-      if (cost < best.cost) best = TilePlan{0, cost, 0};
-      continue;
-    }
-    const int64_t tq = mt * (qk / TN), tv = mt * (v / TN);
-    if (tq + tv <= cus) {  // one tile per workgroup
-      if (kTileCost[nj] < best.cost) best = TilePlan{nj, kTileCost[nj], (int)tq};
-      continue;
-    }
-    for (int64_t w = 1; w < cus; ++w) {
-      const int64_t cost = kTileCost[nj] * std::max(ceil_div(tq, w), ceil_div(tv, cus - w));
-      if (cost < best.cost) best = TilePlan{nj, cost, (int)w};
-    }
-  }
-  return best;
-}
-
-// Workgroups per XCD that fetch ahead of a product of one round: as many as walk the longest run's panels at
-// twice the tiles' pace, one CU touching about 900 lines per us and a k stage (one line per row) taking the
-// tiles of nj `kStageNs`; none if the idle CUs cannot at least keep pace. 1000 tokens, 13824 deep, 0 / 2 / 3 /
-// 4 / 5 / 6 / 8 of them: 120 / 117 / 108 / 92 / 87 / 89 / 91 us; 512 tokens 72 / 74 / 70 / 61 / 54 / 50 / 51;
-// four where the rule asks for thirteen (2000 tokens) 127 -> 212. Not with 256 x 256 tiles, whose MFMAs take
-// as long as the loads (216 tiles: 56.5 -> 58.2 us).
-constexpr int kStageNs[5] = {560, 0, 920, 1100, 0};
-
-template <int kTm, int kTn, int kGroup>
-static int64_t fetch_wgs(int64_t M, int tiles_m, int tiles_n, int64_t idle, int nj) {
-  int64_t lines = 0;
-  for (int x = 0; x < 8; ++x) {
-    const RunPanels p = run_panels<kTm, kGroup>(M, tiles_m, tiles_n, x);
-    lines = std::max(lines, p.m_hi - p.m_lo + (int64_t)(p.n_hi + p.n_lo) * kTn);
-  }
-  const int64_t pace = 900 * kStageNs[nj] / 1000;  // lines per stage and workgroup
-  const int64_t n = std::min(idle, (2 * lines + pace / 2) / pace);
-  return n * pace >= lines ? n : 0;
-}
-
-// The same for one launch (`tiles_n` as launched); Q|K and V on 256-feature tiles have as many each.
+// fetch_wgs for one launch (`tiles_n` as launched); Q|K and V on 256-feature tiles have as many each.
 static int64_t fetch_wgs(int epilogue, const TilePlan& plan, const GemmArgs& g, int64_t idle) {
   auto count = [&](int tiles_n, int64_t n) -> int64_t {
     if (plan.nj == 0) return fetch_wgs<TS, TS, kTsGroupM>(g.M, g.tiles_m, tiles_n, n, 0);
@@ -1597,7 +1479,7 @@ static int launch_plan(int epilogue, const TilePlan& plan, GemmArgs& g, int64_t 
   g.tiles_n = (int)(g.N / tn);
   g.qk_wgs = plan.qk_wgs;
   const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
-  g.tile_wgs = (int)(plan.nj == 0 ? tiles : std::min(tiles, cus));
+  g.tile_wgs = (int)tile_workgroups(plan, tiles, cus);
   int64_t wgs = g.tile_wgs;
   const int64_t idle = (cus - (wgs + 7) / 8 * 8) / 8;  // per XCD
   if (const int64_t n = fetch_wgs(epilogue, plan, g, idle)) wgs = (wgs + 7) / 8 * 8 + 8 * n;
