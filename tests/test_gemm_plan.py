@@ -65,3 +65,41 @@ int main() {
 }
 """)
     assert out.splitlines()[-1].startswith("checked ") and out.endswith(" bad 0\n"), out
+
+
+def test_run_panels_name_every_panel_a_run_reads(run):
+    """The n tiles that an XCD's run of tiles reads, exactly, and token rows that hold all it reads, for every
+    grid of at most 304 tiles (products of one round) of each tile that is fetched ahead of."""
+    out = run("panels", r"""
+static long checked, bad;
+template <int kTm, int kGroup>
+void grids() {
+  for (int tm = 1; tm <= 304; ++tm)
+    for (int tn = 1; tm * tn <= 304; ++tn)
+      for (int64_t M : {(int64_t)(tm - 1) * kTm + 1, (int64_t)tm * kTm})
+        for (int x = 0; x < 8; ++x) {
+          const RunPanels p = run_panels<kTm, kGroup>(M, tm, tn, x);
+          std::vector<int> want(tn, 0), got(tn, 0);
+          bool rows = true;
+          for (int v = x; v < tm * tn; v += 8) {
+            const TileAt t = tile_at(v, tm, tn, kGroup);
+            want[t.tn] = 1;
+            rows &= (int64_t)t.tm * kTm >= p.m_lo && std::min<int64_t>((int64_t)(t.tm + 1) * kTm, M) <= p.m_hi;
+          }
+          bool inside = p.m_lo >= 0 && p.m_hi <= M && p.n0 + p.n_hi <= tn && p.n_lo <= tn;
+          for (int i = 0; inside && i < p.n_hi; ++i) inside &= !got[p.n0 + i]++;
+          for (int i = 0; inside && i < p.n_lo; ++i) inside &= !got[i]++;
+          ++checked;
+          if (!rows || !inside || want != got) {
+            if (bad++ < 5) printf("%d x %d tiles of %d tokens, XCD %d: n [%d, +%d) and [0, %d)\n", tm, tn, kTm, x, p.n0, p.n_hi, p.n_lo);
+          }
+        }
+}
+int main() {
+  grids<192, kGroupM * TM / 192>();
+  grids<128, kGroupM * TM / 128>();
+  grids<TS, kTsGroupM>();
+  printf("checked %ld bad %ld\n", checked, bad);
+}
+""")
+    assert out.splitlines()[-1].startswith("checked ") and out.endswith(" bad 0\n"), out

@@ -52,8 +52,10 @@ constexpr RunPanels run_panels(int64_t M, int tiles_m, int tiles_n, int x) {
   const int s0 = tiles_m - g0 * kGroup, s1 = tiles_m - g1 * kGroup;  // m tiles of the groups
   const int tn0 = first % in_group / (s0 < kGroup ? s0 : kGroup), tn1 = last % in_group / (s1 < kGroup ? s1 : kGroup);
   const int64_t m_end = (int64_t)(g1 + 1) * kGroup * kTm;
+  // the first group's n tiles from tn0 on, the last group's up to tn1; a group between walks all of them
+  const int n_lo = g1 - g0 > 1 || tn1 + 1 > tn0 ? tn0 : tn1 + 1;
   return RunPanels{(int64_t)g0 * kGroup * kTm, m_end < M ? m_end : M, tn0, g0 == g1 ? tn1 - tn0 + 1 : tiles_n - tn0,
-                   g0 == g1 ? 0 : (tn1 + 1 < tn0 ? tn1 + 1 : tn0)};
+                   g0 == g1 ? 0 : n_lo};
 }
 
 // ------------------------------------------------------------------------------------------------
