@@ -33,9 +33,8 @@ struct QKNormArgs {
   int64_t S, ld;
   int heads, nch, tokens_per_wave;
   const float* gamma;
-  const float* cos;  // [S] rows of 64, tab_ld apart
+  const float* cos;  // [S, 64] (kPair: rows tab_ld apart)
   const float* sin;
-  int64_t tab_ld;
   float eps;
   float* maxnorm;  // [heads] or null (must be zeroed first)
   // optional: the queries' across-heads 1/rms from the QKV GEMM's per-128-column partial sums of
@@ -49,7 +48,9 @@ struct QKNormArgs {
   // (token t, head h, d) at out[t*out_ts + h*out_hs + d] (e.g. the head-major [N, S, 128] layout)
   uint16_t* out;
   int64_t out_ts, out_hs;
-  // a second part of as many heads (gridDim.y = 2; no maxnorm, no q_rr): x, gamma and out of part 1
+  // kPair instantiation: a second part of as many heads (gridDim.y = 2; no maxnorm, no q_rr): x, gamma and
+  // out of part 1, and the tables' row stride
+  int64_t tab_ld;
   const float* gamma1;
   int64_t x_part, out_part;  // elements from part 0 to part 1
 };
@@ -65,7 +66,12 @@ struct QKNormArgs {
 // is copied into LDS once per workgroup of 32 tokens instead of being read from L2 per token: per
 // chunk, every lane's first four values (16 bytes, lane-major), then the second four.
 // kWgWaves: waves per workgroup; with the key-norm maximum, more of them (launch_qk_waves has the reason).
-template <int NCH, bool kHalves, bool kOut = false, int kWgWaves = 4>
+// kPair: Q and K in one launch, its own instantiation: selected at run time, the second part's pointers and the
+// tables' stride took the single passes (the block's, at 128 registers) from 2 / 11 spilled registers
+// (interleaved / halves) to 5 / 21. 40 heads, halves, 32760 tokens: with the maximum 166.5 us in one
+// instantiation, 149.4 apart; without it 139.4 and 137.1. The pair itself, without the maximum's registers, spills
+// none (2 with out).
+template <int NCH, bool kHalves, bool kOut, int kWgWaves, bool kPair>
 __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm_rope_kernel(QKNormArgs a) {
 #pragma clang fp contract(off)
   constexpr bool kLdsGamma = NCH <= 10;
@@ -74,11 +80,12 @@ __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = a.heads * 128;
   const int64_t t0 = ((int64_t)blockIdx.x * kWgWaves + wave) * a.tokens_per_wave;
-  if (blockIdx.y != 0) {
+  if (kPair && blockIdx.y != 0) {
     a.x += a.x_part;
     a.out += a.out_part;
     a.gamma = a.gamma1;
   }
+  const int64_t tab_ld = kPair ? a.tab_ld : 64;
   const __amdgpu_buffer_rsrc_t r_g = make_rsrc(a.gamma, 4 * (int64_t)W);
   if constexpr (kLdsGamma) {
     const u32x4 rg = buffer_rsrc(a.gamma, 4u * (uint32_t)W);  // columns past W read as zero
@@ -94,7 +101,7 @@ __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm
 #pragma unroll
   for (int c = 0; c < NCH; ++c) kmx[c] = 0.0f;
 
-  if (a.q_rr != nullptr) {
+  if (!kPair && a.q_rr != nullptr) {
     // lane i < tokens_per_wave: the Q 1/rms of token t0 + i, its partial sums added in block order
     // and the root taken in fp64 -- the operations, in the order, the attention's Q load performs on
     // the same partials (so the attention may read this instead, bit for bit)
@@ -162,8 +169,8 @@ __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm
     constexpr int kAngles = kHalves ? 8 : 4;
     float cs[kAngles], sn[kAngles];
     if (a.cos) {
-      const __amdgpu_buffer_rsrc_t r_c = make_rsrc(a.cos + t * a.tab_ld, 256);
-      const __amdgpu_buffer_rsrc_t r_s = make_rsrc(a.sin + t * a.tab_ld, 256);
+      const __amdgpu_buffer_rsrc_t r_c = make_rsrc(a.cos + t * tab_ld, 256);
+      const __amdgpu_buffer_rsrc_t r_s = make_rsrc(a.sin + t * tab_ld, 256);
       const uint32_t off = kHalves ? (uint32_t)(lane & 7) * 32 : (uint32_t)(lane & 15) * 16;
 #pragma unroll
       for (int u = 0; u < kAngles / 4; ++u) {
@@ -245,7 +252,7 @@ __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm
         } else {
           __builtin_amdgcn_raw_buffer_store_b128(ov, r_x, lane * 16, c * 1024, 0);
         }
-        if (a.maxnorm) {
+        if (!kPair && a.maxnorm) {
           // one head = 16 consecutive lanes of a chunk (one DPP row): sum over the row with DPP
           // moves (quad xor 1, quad xor 2, half-row mirror, row mirror -- the pairs of an xor 1, 2,
           // 4, 8 butterfly, no LDS round trips); the max is kept on ||k||^2 and square-rooted once
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(64 * kWgWaves, (NCH <= 10 ? 4 : 2)) void qk_rmsnorm
       }
     }
   }
-  if (a.maxnorm) {
+  if (!kPair && a.maxnorm) {
     // Workgroup maximum first (through LDS), then one atomic per head per workgroup: every wave of
     // the grid finishes at about the same time, and per-wave atomics on the same few cache lines
     // serialize at the L2 (measured: 180 us of a 340 us launch).
@@ -355,24 +362,30 @@ namespace wanmi {
 // L2s leave to the memory side: about 45 ns a workgroup, one after another, so half as many workgroups
 // of eight waves take half of it off (16 waves: as good, and 392 against 356 us at 75600 tokens). With 4 / 8
 // waves: 20.6 / 17.9 us at 2500 tokens, 30.2 / 23.9 at 4096, 39.3 / 32.9 at 7800, 144 either way at 32760.
-template <int NCH, bool kHalves, bool kOut, int kWgWaves>
-static void launch_qk_waves(const QKNormArgs& a, int parts, hipStream_t s) {
+template <int NCH, bool kHalves, bool kOut, int kWgWaves, bool kPair>
+static void launch_qk_waves(const QKNormArgs& a, hipStream_t s) {
   const int64_t waves = (a.S + a.tokens_per_wave - 1) / a.tokens_per_wave;
-  const dim3 grid((unsigned)((waves + kWgWaves - 1) / kWgWaves), (unsigned)parts);
-  hipLaunchKernelGGL((qk_rmsnorm_rope_kernel<NCH, kHalves, kOut, kWgWaves>), grid, dim3(64 * kWgWaves), 0, s, a);
+  const dim3 grid((unsigned)((waves + kWgWaves - 1) / kWgWaves), kPair ? 2u : 1u);
+  hipLaunchKernelGGL((qk_rmsnorm_rope_kernel<NCH, kHalves, kOut, kWgWaves, kPair>), grid, dim3(64 * kWgWaves), 0, s, a);
 }
 
-template <bool kHalves>
-static void launch_qk(const QKNormArgs& a, int parts, hipStream_t s) {
+template <bool kHalves, bool kPair>
+static void launch_qk(const QKNormArgs& a, hipStream_t s) {
   if (a.out) {
-    if (a.nch <= 4) launch_qk_waves<4, kHalves, true, 4>(a, parts, s);
-    else launch_qk_waves<10, kHalves, true, 4>(a, parts, s);
-  } else if (a.nch <= 10 && a.maxnorm) {
-    launch_qk_waves<10, kHalves, false, 8>(a, parts, s);
-  } else if (a.nch <= 4) launch_qk_waves<4, kHalves, false, 4>(a, parts, s);
-  else if (a.nch <= 10) launch_qk_waves<10, kHalves, false, 4>(a, parts, s);
-  else if (a.nch <= 16) launch_qk_waves<16, kHalves, false, 4>(a, parts, s);
-  else launch_qk_waves<32, kHalves, false, 4>(a, parts, s);
+    if (a.nch <= 4) launch_qk_waves<4, kHalves, true, 4, kPair>(a, s);
+    else launch_qk_waves<10, kHalves, true, 4, kPair>(a, s);
+    return;
+  }
+  if constexpr (!kPair) {
+    if (a.nch <= 10 && a.maxnorm) {
+      launch_qk_waves<10, kHalves, false, 8, false>(a, s);
+      return;
+    }
+  }
+  if (a.nch <= 4) launch_qk_waves<4, kHalves, false, 4, kPair>(a, s);
+  else if (a.nch <= 10) launch_qk_waves<10, kHalves, false, 4, kPair>(a, s);
+  else if (a.nch <= 16) launch_qk_waves<16, kHalves, false, 4, kPair>(a, s);
+  else launch_qk_waves<32, kHalves, false, 4, kPair>(a, s);
 }
 
 static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const float* gamma, const float* cos_tab,
@@ -426,8 +439,9 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.x_part = x_part;
   a.out_part = out_part;
   if (out) WANMI_REQUIRE(a.nch <= 10, WANMI_ERR_UNSUPPORTED, "wanmi_qk_rmsnorm_rope_to: at most 40 heads");
-  if (rope_pairs == WANMI_ROTATE_HALVES) launch_qk<true>(a, parts, s);
-  else launch_qk<false>(a, parts, s);
+  const bool halves = rope_pairs == WANMI_ROTATE_HALVES;
+  if (gamma1) halves ? launch_qk<true, true>(a, s) : launch_qk<false, true>(a, s);
+  else halves ? launch_qk<true, false>(a, s) : launch_qk<false, false>(a, s);
   return check_launch("wanmi_qk_rmsnorm_rope");
 }
 }  // namespace wanmi
