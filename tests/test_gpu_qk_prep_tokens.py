@@ -40,3 +40,24 @@ def test_tokens_per_wave_give_the_same_bits(pkg, dev, operands, S, pairs):
     ref = outs[1][0].double().view(S, N, 128).norm(dim=-1).amax(0)
     # fp32 sums of 128 squares, every partial sum rounded up or down by at most 2^-24 of itself
     assert bool(((kmax.double() - ref).abs() <= 128 * 2.0**-24 * ref).all())
+
+
+@pytest.mark.parametrize("pairs", ["interleaved", "halves"])
+@pytest.mark.parametrize("heads", [4, 16, 20, 40])
+@pytest.mark.parametrize("S", [1, 65, 4097, 28673])
+def test_key_norm_maximum_of_every_workgroup_size(pkg, dev, S, heads, pairs):
+    """The pass with the key-norm maximum against the pass without it, bit for bit, and the maximum against
+    the norms of its rows (the last of them the longest in every other head)."""
+    g = torch.Generator(device=dev).manual_seed(S + heads)
+    x = torch.randn(S, heads * 128, device=dev, generator=g).to(torch.bfloat16)
+    gamma = 1.0 + 0.1 * torch.randn(heads * 128, device=dev, generator=g)
+    ang = torch.randn(S, 64, device=dev, generator=g)
+    x.view(S, heads, 128)[-1, ::2] *= 4
+    kw = dict(cos=ang.cos(), sin=ang.sin(), rope_pairs=pairs)
+    y = x.clone()
+    kmax = pkg.attention_ops.qk_rmsnorm_rope_(y, gamma, want_max=True, **kw)
+    pkg.attention_ops.qk_rmsnorm_rope_(x, gamma, **kw)
+    assert torch.equal(x, y)
+    ref = y.double().view(S, heads, 128).norm(dim=-1).amax(0)
+    # fp32 sums of 128 squares, every partial sum rounded up or down by at most 2^-24 of itself
+    assert bool(((kmax.double() - ref).abs() <= 128 * 2.0**-24 * ref).all())

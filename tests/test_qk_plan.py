@@ -1,0 +1,44 @@
+"""The Q/K pass's launch rule (csrc/qk_plan.h) on the CPU, over its whole range. No GPU."""
+
+import pathlib
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parents[1] / "vllm-omni-neuron_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    """[(heads, rows, maxnorm, cus, chunks, waves, tokens per wave)]"""
+    d = tmp_path_factory.mktemp("qk_plan")
+    (d / "main.cc").write_text(r"""
+#include "qk_plan.h"
+#include <cstdio>
+#include <initializer_list>
+int main() {
+  for (int heads = 4; heads <= 128; heads += 4)
+    for (long rows : {1l, 512l, 4096l, 4097l, 28672l, 28673l, 32760l, 75600l, 1l << 31})
+      for (int max : {0, 1})
+        for (int cus : {32, 256}) {
+          const wanmi::QKPlan p = wanmi::qk_plan(heads, rows, max != 0, cus);
+          printf("%d %ld %d %d %d %d %d\n", heads, rows, max, cus, p.chunks, p.waves, p.tokens_per_wave);
+        }
+}
+""")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", f"-I{CSRC}", str(d / "main.cc"), "-o",
+                    str(d / "main")], check=True)
+    out = subprocess.run([str(d / "main")], check=True, capture_output=True, text=True).stdout
+    return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+
+def test_every_pass_takes_the_smallest_instantiation_that_holds_its_heads(plans):
+    for heads, rows, maxnorm, cus, chunks, waves, _ in plans:
+        assert chunks == min(c for c in (4, 10, 16, 32) if 4 * c >= heads), (heads, maxnorm)
+        assert waves in (4, 8) and (waves == 4 or (maxnorm and heads <= 40))
+
+
+def test_a_resident_round_of_waves_comes_before_a_second_token(plans):
+    for heads, rows, maxnorm, cus, _, _, tokens in plans:
+        assert 1 <= tokens <= 8 and (tokens == 8 or tokens * cus * 16 >= rows)
+        assert tokens == 1 or (tokens - 1) * cus * 16 < rows

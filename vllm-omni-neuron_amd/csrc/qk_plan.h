@@ -1,0 +1,44 @@
+// Launch rule of the Q/K pass (norm, RoPE, key-norm maximum). Plain C++ without HIP, so that it is checked on
+// the CPU.
+#pragma once
+
+#include <stdint.h>
+
+namespace wanmi {
+
+struct QKPlan {
+  int chunks;           // kernel instantiation: registers for this many chunks of four heads
+  int waves;            // waves per workgroup
+  int tokens_per_wave;
+};
+
+// `heads` a multiple of 4, at most 128; `rows`: tokens times parts; `maxnorm`: with the key-norm maximum.
+//
+// Tokens each wave walks. A token is one latency chain (its row, the reduction, the fp64 root, the
+// write), so a wave's tokens are served one after another while other waves hide the latency: as many
+// waves as one round holds (four workgroups of four waves per CU) come first, and only a sequence longer
+// than that gives a wave more than one token. At most 8: an S = 32760 launch is then one resident
+// round, and the gamma copy is shared by 32 tokens. With 8 tokens per wave throughout, 512 / 1560 /
+// 3600 tokens ran 34 / 43 / 47 us: 16 / 49 / 113 workgroups on 256 CUs, each eight such chains long. One
+// token per wave took 24 us off the first, 22 off the second, 21 off the third (the block's
+// cross-attention K/V 94 -> 69 us, row_mx_qkv_proj of 3600 tokens 387 -> 344).
+//
+// Waves per workgroup. With the key-norm maximum every workgroup ends in atomics on the same 160 bytes, which
+// the XCDs' separate L2s leave to the memory side: about 45 ns a workgroup, one after another, so half as
+// many workgroups of eight waves take half of it off (16 waves: as good, and 392 against 356 us at 75600
+// tokens). With 4 / 8 waves, 40 heads: 19.0 / 16.2 us at 2500 tokens, 28.7 / 22.5 at 4096, 37.5 / 31.1 at
+// 7800.
+// The instantiation is the smallest that holds the heads, for every pass: with the key-norm maximum 16 heads of
+// 32760 tokens, halves, took 59.8 us with the registers and the gamma copy of 40 heads, 52.4 with their own.
+inline QKPlan qk_plan(int heads, int64_t rows, bool maxnorm, int64_t cus) {
+  constexpr int64_t kTokensPerWaveMax = 8;
+  const int64_t resident = cus * 4 * 4;
+  const int64_t n = (rows + resident - 1) / resident;
+  QKPlan p{};
+  p.tokens_per_wave = (int)(n < 1 ? 1 : n > kTokensPerWaveMax ? kTokensPerWaveMax : n);
+  p.chunks = heads <= 16 ? 4 : heads <= 40 ? 10 : heads <= 64 ? 16 : 32;
+  p.waves = maxnorm && heads <= 40 ? 8 : 4;
+  return p;
+}
+
+}  // namespace wanmi

@@ -19,6 +19,7 @@
 // the order in which the attention kernel's P^T registers hand keys to the PV MFMA, so each lane
 // reads its 8 keys with a single 16-byte LDS load.
 #include "wanmi_common.h"
+#include "qk_plan.h"
 
 namespace wanmi {
 
@@ -65,7 +66,7 @@ struct QKNormArgs {
 // Up to 40 heads the fp32 gamma (8 bytes per column, as much as the token's own bf16 read and write)
 // is copied into LDS once per workgroup of 32 tokens instead of being read from L2 per token: per
 // chunk, every lane's first four values (16 bytes, lane-major), then the second four.
-// kWgWaves: waves per workgroup; with the key-norm maximum, more of them (launch_qk_waves has the reason).
+// kWgWaves: waves per workgroup; with the key-norm maximum, more of them (qk_plan has the reason).
 // kPair: Q and K in one launch, its own instantiation: selected at run time, the second part's pointers and the
 // tables' stride took the single passes (the block's, at 128 registers) from 2 / 11 spilled registers
 // (interleaved / halves) to 5 / 21. 40 heads, halves, 32760 tokens: with the maximum 166.5 us in one
@@ -292,22 +293,6 @@ __global__ void zero_f32_kernel(float* p, int n) {
   if (i < n) p[i] = 0.0f;
 }
 
-// Tokens each wave walks. A token is one latency chain (its row, the reduction, the fp64 root, the
-// write), so a wave's tokens are served one after another while other waves hide the latency: as many
-// waves as one round holds (four workgroups of four waves per CU, kQKWavesResident) come first, and
-// only a sequence longer than that gives a wave more than one token. At most 8: an S = 32760 launch is
-// then one resident round, and the gamma copy is shared by 32 tokens. With 8 tokens per wave
-// throughout, 512 / 1560 / 3600 tokens ran 34 / 43 / 47 us: 16 / 49 / 113 workgroups on 256 CUs, each
-// eight such chains long. One token per wave took 24 us off the first, 22 off the second, 21 off the
-// third (the block's cross-attention K/V 94 -> 69 us, row_mx_qkv_proj of 3600 tokens 387 -> 344).
-constexpr int64_t kQKWavesResident = 256 * 4 * 4;
-constexpr int kQKTokensPerWaveMax = 8;
-
-static int qk_tokens_per_wave(int64_t rows) {
-  const int64_t n = (rows + kQKWavesResident - 1) / kQKWavesResident;
-  return (int)(n < 1 ? 1 : n > kQKTokensPerWaveMax ? kQKTokensPerWaveMax : n);
-}
-
 struct TransposeArgs {
   const uint16_t* v;  // element (s, h, d) at v[s*ld + h*hs + d]
   int64_t S, ld, hs;
@@ -358,10 +343,6 @@ __global__ __launch_bounds__(256) void transpose_heads_kernel(TransposeArgs a) {
 }  // namespace wanmi
 
 namespace wanmi {
-// With the key-norm maximum every workgroup ends in atomics on the same 160 bytes, which the XCDs' separate
-// L2s leave to the memory side: about 45 ns a workgroup, one after another, so half as many workgroups
-// of eight waves take half of it off (16 waves: as good, and 392 against 356 us at 75600 tokens). With 4 / 8
-// waves: 20.6 / 17.9 us at 2500 tokens, 30.2 / 23.9 at 4096, 39.3 / 32.9 at 7800, 144 either way at 32760.
 template <int NCH, bool kHalves, bool kOut, int kWgWaves, bool kPair>
 static void launch_qk_waves(const QKNormArgs& a, hipStream_t s) {
   const int64_t waves = (a.S + a.tokens_per_wave - 1) / a.tokens_per_wave;
@@ -370,21 +351,22 @@ static void launch_qk_waves(const QKNormArgs& a, hipStream_t s) {
 }
 
 template <bool kHalves, bool kPair>
-static void launch_qk(const QKNormArgs& a, hipStream_t s) {
+static void launch_qk(const QKNormArgs& a, const QKPlan& plan, hipStream_t s) {
   if (a.out) {
-    if (a.nch <= 4) launch_qk_waves<4, kHalves, true, 4, kPair>(a, s);
+    if (plan.chunks == 4) launch_qk_waves<4, kHalves, true, 4, kPair>(a, s);
     else launch_qk_waves<10, kHalves, true, 4, kPair>(a, s);
     return;
   }
   if constexpr (!kPair) {
-    if (a.nch <= 10 && a.maxnorm) {
-      launch_qk_waves<10, kHalves, false, 8, false>(a, s);
+    if (plan.waves == 8) {
+      if (plan.chunks == 4) launch_qk_waves<4, kHalves, false, 8, false>(a, s);
+      else launch_qk_waves<10, kHalves, false, 8, false>(a, s);
       return;
     }
   }
-  if (a.nch <= 4) launch_qk_waves<4, kHalves, false, 4, kPair>(a, s);
-  else if (a.nch <= 10) launch_qk_waves<10, kHalves, false, 4, kPair>(a, s);
-  else if (a.nch <= 16) launch_qk_waves<16, kHalves, false, 4, kPair>(a, s);
+  if (plan.chunks == 4) launch_qk_waves<4, kHalves, false, 4, kPair>(a, s);
+  else if (plan.chunks == 10) launch_qk_waves<10, kHalves, false, 4, kPair>(a, s);
+  else if (plan.chunks == 16) launch_qk_waves<16, kHalves, false, 4, kPair>(a, s);
   else launch_qk_waves<32, kHalves, false, 4, kPair>(a, s);
 }
 
@@ -419,8 +401,9 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.ld = ld;
   a.heads = heads;
   a.nch = heads / 4;
-  const int parts = gamma1 ? 2 : 1;
-  a.tokens_per_wave = qk_tokens_per_wave(S * parts);
+  const int cus = device_cu_count();
+  const QKPlan plan = qk_plan(heads, gamma1 ? 2 * S : S, maxnorm != nullptr, cus > 0 ? cus : 256);
+  a.tokens_per_wave = plan.tokens_per_wave;
   a.gamma = gamma;
   a.cos = cos_tab;
   a.sin = sin_tab;
@@ -440,8 +423,8 @@ static int qk_rmsnorm_rope_impl(void* x, int64_t S, int64_t ld, int heads, const
   a.out_part = out_part;
   if (out) WANMI_REQUIRE(a.nch <= 10, WANMI_ERR_UNSUPPORTED, "wanmi_qk_rmsnorm_rope_to: at most 40 heads");
   const bool halves = rope_pairs == WANMI_ROTATE_HALVES;
-  if (gamma1) halves ? launch_qk<true, true>(a, s) : launch_qk<false, true>(a, s);
-  else halves ? launch_qk<true, false>(a, s) : launch_qk<false, false>(a, s);
+  if (gamma1) halves ? launch_qk<true, true>(a, plan, s) : launch_qk<false, true>(a, plan, s);
+  else halves ? launch_qk<true, false>(a, plan, s) : launch_qk<false, false>(a, plan, s);
   return check_launch("wanmi_qk_rmsnorm_rope");
 }
 }  // namespace wanmi
