@@ -42,3 +42,11 @@ def test_a_resident_round_of_waves_comes_before_a_second_token(plans):
     for heads, rows, maxnorm, cus, _, _, tokens in plans:
         assert 1 <= tokens <= 8 and (tokens == 8 or tokens * cus * 16 >= rows)
         assert tokens == 1 or (tokens - 1) * cus * 16 < rows
+
+
+def test_long_passes_end_in_workgroups_of_four_waves(plans):
+    """With every wave at its most tokens the pass is bound by memory, and larger workgroups only lengthen its
+    end; up to 8 heads the maxima's atomics still bound it."""
+    for heads, rows, maxnorm, cus, _, waves, tokens in plans:
+        if maxnorm and heads <= 40:
+            assert waves == (4 if tokens == 8 and heads > 8 else 8), (heads, rows, cus)

@@ -27,7 +27,10 @@ struct QKPlan {
 // the XCDs' separate L2s leave to the memory side: about 45 ns a workgroup, one after another, so half as
 // many workgroups of eight waves take half of it off (16 waves: as good, and 392 against 356 us at 75600
 // tokens). With 4 / 8 waves, 40 heads: 19.0 / 16.2 us at 2500 tokens, 28.7 / 22.5 at 4096, 37.5 / 31.1 at
-// 7800.
+// 7800. Not once every wave has its 8 tokens (more than 28672): the pass is then bound by memory, and larger
+// workgroups lengthen its end: 16 heads 49.7 / 51.0 us at 32760 tokens and 122.8 / 129.6 at 75600, 12 heads 96.5 /
+// 99.5, 32 heads 270 / 278, 40 heads 338 / 338 (halves 352 / 356). Up to 8 heads the atomics still bound it: 71.3 /
+// 62.5, 4 heads 46.2 / 41.1.
 // The instantiation is the smallest that holds the heads, for every pass: with the key-norm maximum 16 heads of
 // 32760 tokens, halves, took 59.8 us with the registers and the gamma copy of 40 heads, 52.4 with their own.
 inline QKPlan qk_plan(int heads, int64_t rows, bool maxnorm, int64_t cus) {
@@ -37,7 +40,7 @@ inline QKPlan qk_plan(int heads, int64_t rows, bool maxnorm, int64_t cus) {
   QKPlan p{};
   p.tokens_per_wave = (int)(n < 1 ? 1 : n > kTokensPerWaveMax ? kTokensPerWaveMax : n);
   p.chunks = heads <= 16 ? 4 : heads <= 40 ? 10 : heads <= 64 ? 16 : 32;
-  p.waves = maxnorm && heads <= 40 ? 8 : 4;
+  p.waves = maxnorm && heads <= 40 && (p.tokens_per_wave < kTokensPerWaveMax || heads <= 8) ? 8 : 4;
   return p;
 }
 
