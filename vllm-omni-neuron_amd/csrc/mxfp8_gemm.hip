@@ -1135,9 +1135,11 @@ __global__ __launch_bounds__(256, 1) void mxfp8_gemm_ring_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint8_t sWh[5][kHalfBytes];
   __shared__ __attribute__((aligned(16))) uint8_t sAct[2][64 * kNj * BK];
   __shared__ __attribute__((aligned(16))) uint32_t ssc[2][2 * 256 * 4];
-  if ((int)blockIdx.x >= g.tile_wgs) {
-    fetch_ahead_wg<EPI, 64 * kNj, TN, kGroupM * TM / (64 * kNj)>(g, ssc[0]);
-    return;
+  if constexpr (kNj < 4) {  // (nothing is fetched ahead of 256 x 256 tiles)
+    if ((int)blockIdx.x >= g.tile_wgs) {
+      fetch_ahead_wg<EPI, 64 * kNj, TN, kGroupM * TM / (64 * kNj)>(g, ssc[0]);
+      return;
+    }
   }
   if constexpr (EPI == kEpiQkv) {
     // workgroups [0, qk_wgs) walk the Q|K tiles, the others the V tiles
