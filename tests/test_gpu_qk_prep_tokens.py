@@ -61,3 +61,14 @@ def test_key_norm_maximum_of_every_workgroup_size(pkg, dev, S, heads, pairs):
     ref = y.double().view(S, heads, 128).norm(dim=-1).amax(0)
     # fp32 sums of 128 squares, every partial sum rounded up or down by at most 2^-24 of itself
     assert bool(((kmax.double() - ref).abs() <= 128 * 2.0**-24 * ref).all())
+
+
+@pytest.mark.parametrize("S,heads", [(1, 4), (640, 40), (641, 40), (25000, 40), (25008, 40)])
+def test_key_norm_maximum_alone_of_every_workgroup_size(pkg, dev, S, heads):
+    g = torch.Generator(device=dev).manual_seed(S)
+    k = torch.randn(S, heads, 128, device=dev, generator=g).to(torch.bfloat16)
+    k[-1, ::2] *= 4
+    k[0, 1::2] *= 4
+    ref = k.double().norm(dim=-1).amax(0)
+    # fp32 sums of 128 squares, every partial sum rounded up or down by at most 2^-24 of itself
+    assert bool(((pkg.attention_ops.head_max_norm(k).double() - ref).abs() <= 128 * 2.0**-24 * ref).all())

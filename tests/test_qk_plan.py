@@ -8,14 +8,19 @@ import pytest
 CSRC = pathlib.Path(__file__).resolve().parents[1] / "vllm-omni-neuron_amd" / "csrc"
 
 
+def _run(d, body):
+    """What a C++ main over qk_plan.h prints: a tuple of numbers per line."""
+    (d / "main.cc").write_text('#include "qk_plan.h"\n#include <cstdio>\n#include <initializer_list>\n' + body)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", f"-I{CSRC}", str(d / "main.cc"), "-o",
+                    str(d / "main")], check=True)
+    out = subprocess.run([str(d / "main")], check=True, capture_output=True, text=True).stdout
+    return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+
 @pytest.fixture(scope="module")
 def plans(tmp_path_factory):
     """[(heads, rows, maxnorm, cus, chunks, waves, tokens per wave)]"""
-    d = tmp_path_factory.mktemp("qk_plan")
-    (d / "main.cc").write_text(r"""
-#include "qk_plan.h"
-#include <cstdio>
-#include <initializer_list>
+    return _run(tmp_path_factory.mktemp("qk_plan"), r"""
 int main() {
   for (int heads = 4; heads <= 128; heads += 4)
     for (long rows : {1l, 512l, 4096l, 4097l, 28672l, 28673l, 32760l, 75600l, 1l << 31})
@@ -26,10 +31,6 @@ int main() {
         }
 }
 """)
-    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", f"-I{CSRC}", str(d / "main.cc"), "-o",
-                    str(d / "main")], check=True)
-    out = subprocess.run([str(d / "main")], check=True, capture_output=True, text=True).stdout
-    return [tuple(map(int, line.split())) for line in out.splitlines()]
 
 
 def test_every_pass_takes_the_smallest_instantiation_that_holds_its_heads(plans):
@@ -50,3 +51,11 @@ def test_long_passes_end_in_workgroups_of_four_waves(plans):
     for heads, rows, maxnorm, cus, _, waves, tokens in plans:
         if maxnorm and heads <= 40:
             assert waves == (4 if tokens == 8 and heads > 8 else 8), (heads, rows, cus)
+
+
+def test_the_maximum_alone_takes_large_workgroups_only_where_atomics_bound_it(tmp_path):
+    """Eight waves per workgroup neither over a few hundred tokens nor over more than memory streams anyway."""
+    faster = {(64, 4): 4, (256, 40): 4, (512, 24): 4, (1024, 40): 8, (2500, 4): 8, (7800, 40): 8, (32760, 24): 8,
+              (32760, 40): 4, (50000, 32): 4, (75600, 40): 4}  # (tokens, heads): as measured
+    calls = "".join(f'printf("%d\\n", wanmi::head_max_norm_waves({r}, {h}));' for r, h in faster)
+    assert [w for w, in _run(tmp_path, "int main() {" + calls + "}")] == list(faster.values())

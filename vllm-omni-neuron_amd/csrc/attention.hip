@@ -19,6 +19,7 @@
 // 16 (wanmi_transpose_heads) to match P^T's register order. ||q_i|| is taken from the same bf16
 // Q fragments the MFMA consumes.
 #include "wanmi_common.h"
+#include "qk_plan.h"
 
 #include <algorithm>
 #include <mutex>
@@ -1224,18 +1225,18 @@ __global__ __launch_bounds__(256) void head_max_norm_kernel(const uint16_t* x, i
 // loads of two tokens in flight) instead of one head's 256 bytes per token row, so the reads are
 // sequential; lane group l >> 4 of chunk c holds head 4 c + (l >> 4). Each wave keeps per-head maxima
 // of ||x||^2 in registers; the workgroup reduces them through LDS and issues one atomic per head.
-constexpr int kHmnRowWaves = 8;
-__global__ __launch_bounds__(64 * kHmnRowWaves) void head_max_norm_rows_kernel(const uint16_t* x, int64_t ss, int64_t S, int heads,
-                                                                 float* out) {
-  __shared__ float smax[kHmnRowWaves][40];
+template <int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void head_max_norm_rows_kernel(const uint16_t* x, int64_t ss, int64_t S,
+                                                                         int heads, float* out) {
+  __shared__ float smax[kWaves][40];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nch = heads / 4;
   float kmx[10];
 #pragma unroll
   for (int c = 0; c < 10; ++c) kmx[c] = 0.0f;
-  const int64_t stride = (int64_t)gridDim.x * kHmnRowWaves;
-  for (int64_t t = (int64_t)blockIdx.x * kHmnRowWaves + wave; t < S; t += 2 * stride) {
+  const int64_t stride = (int64_t)gridDim.x * kWaves;
+  for (int64_t t = (int64_t)blockIdx.x * kWaves + wave; t < S; t += 2 * stride) {
     u32x4 v[2][10];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -1273,7 +1274,7 @@ __global__ __launch_bounds__(64 * kHmnRowWaves) void head_max_norm_rows_kernel(c
   if (hd < heads) {
     float m = smax[0][hd];
 #pragma unroll
-    for (int w = 1; w < kHmnRowWaves; ++w) m = fmaxf(m, smax[w][hd]);
+    for (int w = 1; w < kWaves; ++w) m = fmaxf(m, smax[w][hd]);
     atomicMax(reinterpret_cast<unsigned int*>(out) + hd, __float_as_uint(sqrtf(m)));
   }
 }
@@ -1305,9 +1306,14 @@ extern "C" int wanmi_head_max_norm(const void* x, int64_t head_stride, int64_t t
   WANMI_REQUIRE(x && ((uintptr_t)x % 16) == 0, WANMI_ERR_ARG, "wanmi_head_max_norm: x must be 16-byte aligned");
   if (head_stride == 128 && heads % 4 == 0 && heads <= 40 && token_stride >= heads * 128) {
     // heads contiguous within a token: whole rows per wave, two tokens per step
-    const int64_t blocks = min((S + 2 * kHmnRowWaves - 1) / (2 * kHmnRowWaves), (int64_t)1024);
-    hipLaunchKernelGGL(head_max_norm_rows_kernel, dim3((unsigned)blocks), dim3(64 * kHmnRowWaves), 0, s,
-                       static_cast<const uint16_t*>(x), token_stride, S, heads, out);
+    const int waves = head_max_norm_waves(S, heads);
+    const int64_t blocks = min((S + 2 * waves - 1) / (2 * waves), (int64_t)1024);
+    if (waves == 4)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(head_max_norm_rows_kernel<4>), dim3((unsigned)blocks), dim3(256), 0, s,
+                         static_cast<const uint16_t*>(x), token_stride, S, heads, out);
+    else
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(head_max_norm_rows_kernel<8>), dim3((unsigned)blocks), dim3(512), 0, s,
+                         static_cast<const uint16_t*>(x), token_stride, S, heads, out);
     return check_launch("wanmi_head_max_norm");
   }
   const int64_t blocks = min((S + 15) / 16, (int64_t)256);

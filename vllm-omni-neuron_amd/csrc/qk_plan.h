@@ -1,4 +1,4 @@
-// Launch rule of the Q/K pass (norm, RoPE, key-norm maximum). Plain C++ without HIP, so that it is checked on
+// Launch rules of the Q/K pass (norm, RoPE, key-norm maximum) and of the maximum alone. Plain C++ without HIP, so that it is checked on
 // the CPU.
 #pragma once
 
@@ -43,5 +43,12 @@ inline QKPlan qk_plan(int heads, int64_t rows, bool maxnorm, int64_t cus) {
   p.waves = maxnorm && heads <= 40 && (p.tokens_per_wave < kTokensPerWaveMax || heads <= 8) ? 8 : 4;
   return p;
 }
+
+// Waves per workgroup of the key-norm maximum alone over `rows` tokens: eight, which halve its atomics as above
+// (4 / 8 waves, 40 heads: 9.2 / 7.7 us at 2500 tokens, 22.3 / 17.4 at 7800), but four where there are few
+// workgroups anyway and the larger ones only take longer to end (5.2 / 5.7 at 256 tokens, 5.6 / 5.8 at 512, 6.1 / 6.0
+// at 768), and four where memory bounds it (32 heads 71.5 / 78.6 at 50000, 40 heads 134.3 / 137.3 at 75600;
+// below 256 MB eight: 24 heads 34.5 / 32.1 at 32760).
+inline int head_max_norm_waves(int64_t rows, int heads) { return rows <= 640 || rows * heads > 1000000 ? 4 : 8; }
 
 }  // namespace wanmi
