@@ -147,3 +147,47 @@ int main() {
 }
 """)
     assert out.splitlines()[-1].startswith("checked ") and " fetched 0 " not in out and out.endswith(" bad 0\n"), out
+
+
+def test_qkv_split_is_that_of_the_search_over_all_splits(run):
+    """Cost and tile as a search over every split of the CUs finds them, in well under a microsecond a call (the
+    search took four)."""
+    out = run("split", "#include <chrono>\n" + QKV_SWEEP + r"""
+TilePlan search(int64_t M, int64_t qk, int64_t v, int64_t cus, int64_t vt_ld) {
+  TilePlan best{4, INT64_MAX, 0};
+  for (int nj : {4, 3, 2, 0}) {
+    const int64_t tm = nj ? 64 * nj : TS, mt = ceil_div(M, tm);
+    if (mt * tm < vt_ld) continue;
+    if (nj == 0) {
+      const int64_t cost = kTileCost[0] * ceil_div(mt * ((qk + v) / TS), cus);
+      if (cost < best.cost) best = TilePlan{0, cost, 0};
+      continue;
+    }
+    const int64_t tq = mt * (qk / TN), tv = mt * (v / TN);
+    for (int64_t w = 1; w < std::min(cus, tq + tv); ++w) {
+      const int64_t cost = kTileCost[nj] * std::max(ceil_div(tq, w), ceil_div(tv, std::min(cus, tq + tv) - w));
+      if (cost < best.cost) best = TilePlan{nj, cost, (int)w};
+    }
+  }
+  return best;
+}
+int main() {
+  long checked = 0, bad = 0;
+  sweep([&](int64_t M, int64_t qk, int64_t v, int64_t cus, const TilePlan& p) {
+    const TilePlan want = search(M, qk, v, cus, (M + 63) / 64 * 64);
+    ++checked;
+    if (p.nj != want.nj || p.cost != want.cost) ++bad;
+  });
+  printf("checked %ld bad %ld\n", checked, bad);
+  int64_t sum = 0;
+  double best = 1e9;
+  for (int rep = 0; rep < 5; ++rep) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int64_t M = 1; M <= 20000; ++M) sum += select_qkv_tile(M, 10240, 5120, 256, (M + 63) / 64 * 64).cost;
+    best = std::min(best, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() / 20000);
+  }
+  printf("%lld\n%.3f\n", (long long)sum, best);
+}
+""").splitlines()
+    assert out[0].startswith("checked ") and out[0].endswith(" bad 0"), out
+    assert float(out[2]) < 1.0, f"{out[2]} us per call"

@@ -113,10 +113,12 @@ inline TilePlan select_qkv_tile(int64_t M, int64_t qk, int64_t v, int64_t cus, i
       if (kTileCost[nj] < best.cost) best = TilePlan{nj, kTileCost[nj], (int)tq};
       continue;
     }
-    for (int64_t w = std::max<int64_t>(1, cus - tv); w <= std::min(tq, cus - 1); ++w) {
-      const int64_t cost = kTileCost[nj] * std::max(ceil_div(tq, w), ceil_div(tv, cus - w));
-      if (cost < best.cost) best = TilePlan{nj, cost, (int)w};
-    }
+    if (cus < 2) continue;  // no CU for one of the parts
+    // The fewest rounds in which both parts fit: from the rounds of all tiles on, one or two steps.
+    int64_t rounds = ceil_div(tq + tv, cus);
+    while (ceil_div(tq, rounds) + ceil_div(tv, rounds) > cus) ++rounds;
+    const int64_t cost = kTileCost[nj] * rounds;
+    if (cost < best.cost) best = TilePlan{nj, cost, (int)std::max(ceil_div(tq, rounds), cus - tv)};
   }
   return best;
 }

@@ -1513,12 +1513,13 @@ static bool aligned_weight(const WeightPart& w) {
          ((uintptr_t)w.bias % 16) == 0;
 }
 
-// `v`: the V weight of kEpiQkv (columns [vt_col0, N)).
+// `v`: the V weight of kEpiQkv (columns [vt_col0, N)), `qkv_plan` its tile and split.
 static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint8_t* w_codes, const uint8_t* w_scales,
                      const float* row_scale, const float* col_scale, const float* bias, int64_t M, int64_t N,
                      int64_t K, int64_t lda, int epilogue, void* out, int64_t ldo, uint8_t* out_scales,
                      const void* residual, const float* gate, float* row_sumsq, int64_t sumsq_cols, int64_t sumsq_ld,
-                     void* vt, int64_t vt_ld, int64_t vt_col0, void* stream, const WeightPart& v = WeightPart{}) {
+                     void* vt, int64_t vt_ld, int64_t vt_col0, void* stream, const WeightPart& v = WeightPart{},
+                     const TilePlan& qkv_plan = TilePlan{}) {
   WANMI_REQUIRE(M >= 0 && N > 0 && K > 0, WANMI_ERR_ARG, "wanmi_mxfp8_gemm: bad sizes M=%lld N=%lld K=%lld",
                 (long long)M, (long long)N, (long long)K);
   WANMI_REQUIRE(N % TN == 0, WANMI_ERR_UNSUPPORTED, "wanmi_mxfp8_gemm: N=%lld must be a multiple of %d",
@@ -1596,9 +1597,7 @@ static int gemm_impl(const uint8_t* a_codes, const uint8_t* a_scales, const uint
   const int cus = device_cu_count();
   WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm: cannot query the device's compute units");
   if ((K / BK) % 4 == 0) {
-    const int64_t pad = to_vt || to_qkv ? vt_ld : 0;
-    const TilePlan plan = to_qkv ? select_qkv_tile(M, vt_col0, N - vt_col0, cus, pad) : select_tile(M, N, cus, pad);
-    return launch_plan(epilogue, plan, g, cus, (hipStream_t)stream);
+    return launch_plan(epilogue, to_qkv ? qkv_plan : select_tile(M, N, cus, to_vt ? vt_ld : 0), g, cus, (hipStream_t)stream);
   }
   launch_simple(epilogue, dim3((unsigned)std::min<int64_t>(tiles, cus)), (hipStream_t)stream, g);
   return check_launch("wanmi_mxfp8_gemm");
@@ -1644,10 +1643,11 @@ static int projection_with_vt(const uint8_t* a_codes, const uint8_t* a_scales, c
     const int cus = device_cu_count();
     WANMI_REQUIRE(cus > 0, WANMI_ERR_HIP, "wanmi_mxfp8_gemm_qkv: cannot query the device's compute units");
     const int64_t apart = select_tile(M, n_out, cus, 0).cost + select_tile(M, n_v, cus, vt_ld).cost;
-    if (select_qkv_tile(M, n_out, n_v, cus, vt_ld).cost <= apart)
+    const TilePlan together = select_qkv_tile(M, n_out, n_v, cus, vt_ld);
+    if (together.cost <= apart)
       return gemm_impl(a_codes, a_scales, w.codes, w.scales, row_scale, w.col_scale, w.bias, M, n_out + n_v, K, lda,
                        kEpiQkv, out, ldo, nullptr, nullptr, nullptr, row_sumsq, sumsq_cols, n_out / 128, vt, vt_ld, n_out,
-                       stream, v);
+                       stream, v, together);
   }
   // the plain bf16 epilogue (with the partial sums)
   int st = gemm_impl(a_codes, a_scales, w.codes, w.scales, row_scale, w.col_scale, w.bias, M, n_out, K, lda,
