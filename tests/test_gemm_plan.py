@@ -105,50 +105,6 @@ int main() {
     assert out.splitlines()[-1].startswith("checked ") and out.endswith(" bad 0\n"), out
 
 
-def test_fetching_workgroups_keep_pace_with_the_tiles(run):
-    """Wherever a product's idle CUs fetch ahead, they walk the longest run's panels about as fast as the
-    tiles do; overtaken, the launch waits for them. Their pace as measured where tiles overtook them (lines per us
-    of 1, 2, 4, 6 and 9 workgroups of an XCD, which share its path to memory), between those straight lines."""
-    out = run("pace", r"""
-static const double kN[] = {0, 1, 2, 4, 6, 9, 32}, kPace[] = {0, 900, 1750, 3190, 4200, 5110, 5110};
-double pace(int64_t n) {
-  int i = 1;
-  while (kN[i] < n) ++i;
-  return kPace[i - 1] + (kPace[i] - kPace[i - 1]) * (n - kN[i - 1]) / (kN[i] - kN[i - 1]);
-}
-static long checked, fetched, bad;
-template <int kTm, int kTn, int kGroup>
-void product(int64_t M, int64_t N, int nj) {
-  const int mt = (int)ceil_div(M, kTm), nt = (int)(N / kTn);
-  const int64_t tiles = (int64_t)mt * nt, idle = (256 - (std::min<int64_t>(tiles, 256) + 7) / 8 * 8) / 8;
-  if (idle <= 0) return;
-  const int64_t n = fetch_wgs<kTm, kTn, kGroup>(M, mt, nt, idle, nj);
-  ++checked;
-  if (n == 0) return;
-  ++fetched;
-  int64_t lines = 0;
-  for (int x = 0; x < 8; ++x) {
-    const RunPanels p = run_panels<kTm, kGroup>(M, mt, nt, x);
-    lines = std::max(lines, p.m_hi - p.m_lo + (int64_t)(p.n_hi + p.n_lo) * kTn);
-  }
-  const double need = 1000.0 * lines / kStageNs[nj];
-  if (n > idle || pace(n) < 0.87 * need)
-    if (bad++ < 5) printf("%ld x %ld, nj=%d: %ld workgroups, %.0f lines per us of %.0f\n", (long)M, (long)N, nj, (long)n, pace(n), need);
-}
-int main() {
-  for (int64_t N = 256; N <= 15360; N += 256)
-    for (int64_t M = 1; M <= 8200; M += 7) {
-      const TilePlan p = select_tile(M, N, 256, 0);
-      if (p.nj == 0) product<TS, TS, kTsGroupM>(M, N, 0);
-      if (p.nj == 2) product<128, TN, kGroupM * TM / 128>(M, N, 2);
-      if (p.nj == 3) product<192, TN, kGroupM * TM / 192>(M, N, 3);
-    }
-  printf("checked %ld fetched %ld bad %ld\n", checked, fetched, bad);
-}
-""")
-    assert out.splitlines()[-1].startswith("checked ") and " fetched 0 " not in out and out.endswith(" bad 0\n"), out
-
-
 def test_qkv_split_is_that_of_the_search_over_all_splits(run):
     """Cost and tile as a search over every split of the CUs finds them, in well under a microsecond a call (the
     search took four)."""

@@ -131,18 +131,16 @@ inline int64_t tile_workgroups(const TilePlan& plan, int64_t tiles, int64_t cus)
 
 // Workgroups per XCD that fetch ahead of a product of one round: as many as walk the longest run's panels at
 // twice the tiles' pace, one CU touching about 900 lines per us and a k stage (one line per row) taking the
-// tiles of nj `kStageNs`; none if the idle CUs cannot reach nine tenths of the tiles' pace (at 0.93 of it, 1100
-// tokens of 2048 columns, 23.2 us without and 22.6 with). 1000 tokens, 13824 deep, 0 / 2 / 3 / 4 / 5 / 6 / 8 of
-// them: 120 / 117 / 108 / 92 / 87 / 89 / 91 us; 512 tokens 72 / 74 / 70 / 61 / 54 / 50 / 51; four where the rule
-// asks for thirteen (2000 tokens) 127 -> 212. Not with 256 x 256 tiles, whose MFMAs take as long as the
-// loads (216 tiles: 56.5 -> 58.2 us).
+// tiles of nj `kStageNs`; none if the idle CUs cannot at least keep pace. 1000 tokens, 13824 deep, 0 / 2 / 3 /
+// 4 / 5 / 6 / 8 of them: 120 / 117 / 108 / 92 / 87 / 89 / 91 us; 512 tokens 72 / 74 / 70 / 61 / 54 / 50 / 51;
+// four where the rule asks for thirteen (2000 tokens) 127 -> 212. Not with 256 x 256 tiles, whose MFMAs take
+// as long as the loads (216 tiles: 56.5 -> 58.2 us).
+// (Those figures with the weights in memory. n workgroups of an XCD share its path: 2, 4, 6, 9 of them touch 1750,
+// 3190, 4200, 5110 lines per us where tiles overtake them. Nine at 900 each seem to keep pace with the deep run
+// that 1025 to 1152 tokens of 5120 columns have, and do not: with the weights in the caches 1100 tokens take 45 us
+// with them and 37 without, 13824 deep 130 and 91. From memory, as a model's layers come, it is 44.5 and 48.9,
+// and 125 and 118; 1152 tokens 43.9 and 51.9, 124 and 125: there they stay.)
 constexpr int kStageNs[5] = {560, 0, 920, 1100, 0};
-
-// Lines per us that n workgroups of one XCD touch: they share its path to memory (measured where the tiles
-// overtook them: 2, 4, 6, 9 workgroups 1750, 3190, 4200, 5110). Taken as 900 each, nine were to keep pace with
-// the one deep run that 1025 to 1152 tokens of 5120 columns have (9 m tiles in groups of 8), and did not: 5120
-// deep 37 us without them and 45 with, 13824 deep 90 and 131.
-inline int64_t fetch_pace(int64_t n) { return std::min<int64_t>(900 * n * 100 / (94 + 6 * n), 5100); }
 
 template <int kTm, int kTn, int kGroup>
 inline int64_t fetch_wgs(int64_t M, int tiles_m, int tiles_n, int64_t idle, int nj) {
@@ -151,9 +149,9 @@ inline int64_t fetch_wgs(int64_t M, int tiles_m, int tiles_n, int64_t idle, int 
     const RunPanels p = run_panels<kTm, kGroup>(M, tiles_m, tiles_n, x);
     lines = std::max(lines, p.m_hi - p.m_lo + (int64_t)(p.n_hi + p.n_lo) * kTn);
   }
-  const int64_t one = 900 * kStageNs[nj] / 1000;  // lines per stage of one workgroup
-  const int64_t n = std::min(idle, (2 * lines + one / 2) / one);
-  return fetch_pace(n) * kStageNs[nj] >= 900 * lines ? n : 0;
+  const int64_t pace = 900 * kStageNs[nj] / 1000;  // lines per stage and workgroup
+  const int64_t n = std::min(idle, (2 * lines + pace / 2) / pace);
+  return n * pace >= lines ? n : 0;
 }
 
 }  // namespace wanmi
