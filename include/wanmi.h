@@ -80,6 +80,8 @@ int wanmi_adaln_quant(const void* hidden, const void* residual, const float* gat
  * out: bf16 or e4m3fn [M, ldo]; out_scales: e8m0 [M, N/32] (GELU_MX); residual: bf16 [M, ldo].
  * Requires N % 256 == 0, K % 128 == 0, 256 * K and 256 * lda below 2^31, M * ldo below 2^32 and
  * ldo below 2^22 (32-bit buffer offsets).
+ * A product of fewer tiles than the device has CUs may occupy some of the others too, with workgroups
+ * that fetch its operands ahead; launches on other streams find those taken until it ends.
  * Replaces the ROW_MX projection kernels behind row_mx_qkv_proj / row_mx_o_proj / row_mx_mlp
  * (vllm_omni_neuron/diffusion/quantization/row_mx_kernels.py:48-198): _qkv_cte_mx_impl
  * (kernels/nkilib/core/qkv/qkv_cte.py:2725) and mlp_cte_mx (kernels/nkilib/core/mlp/mlp_cte/mx/).
@@ -117,9 +119,9 @@ int wanmi_mxfp8_gemm_rowsumsq(const uint8_t* a_codes, const uint8_t* a_scales, c
  * [(N - vt_col0)/128 heads][128][vt_ld] bf16 in the key order of wanmi_transpose_heads (inside each
  * group of 16 keys: 0-3, 8-11, 4-7, 12-15), zero for tokens M .. vt_ld - 1. vt_col0 and N - vt_col0
  * are multiples of 256; M > 0; M <= vt_ld <= M rounded up to 256 (every token column up to vt_ld is
- * written, zeros past M), vt_ld % 64 == 0. One launch on `stream` or two (Q|K, then V), whichever needs
- * fewer rounds of tiles (V's MFMAs take the token operand first so that four consecutive tokens of a
- * feature are lane-local).
+ * written, zeros past M), vt_ld % 64 == 0. One launch on `stream` or two (Q|K, then V), whichever costs
+ * less in rounds of tiles weighted by a tile's time, one at equal cost (V's MFMAs take the token operand
+ * first so that four consecutive tokens of a feature are lane-local).
  * Replaces the QKV kernel of row_mx_qkv_proj (vllm_omni_neuron/diffusion/quantization/
  * row_mx_kernels.py:48-111, kernels/nkilib/core/qkv/qkv_cte.py:2725) together with the V transpose
  * the reference's attention kernels do internally (ring_attention_const_max_fwd.py:1180-1220).
@@ -208,6 +210,11 @@ int wanmi_head_max_norm(const void* x, int64_t head_stride, int64_t token_stride
  *   c_i = s ||q_i|| kmax[h]   (kmax[h] >= max_j ||k_j||, e.g. from wanmi_head_max_norm)
  * q, k: element (h, s, d) at x[h*head_stride + s*token_stride + d]; vt: [heads, 128, vt_ld] from
  * wanmi_transpose_heads (vt_ld % 64 == 0, >= Sk).
+ * The queries behind the last whole block of 256 may be served by two or four waves each whose partial
+ * sums are added (fp32, in the waves' order), where that saves a round over the CUs: equal calls give
+ * equal bits, but such a query's last bits may depend on Sq, Sk and the number of heads, so a sequence
+ * split by queries need not give the bits of one call. Calls of fewer than 256 queries or of a multiple of
+ * 256 always add in the whole blocks' order.
  * Replaces ring_attention_const_max_fwd on one device (vllm_omni_neuron/kernels/nkilib/
  * experimental/attention/ring_attention_const_max_fwd.py:959) and the flash attention behind
  * _nki_attend / wan_cp_self_attention (diffusion/models/wan2_2/wan2_2_transformer.py:653, 806).

@@ -96,7 +96,9 @@ inline TilePlan select_tile(int64_t M, int64_t n, int64_t cus, int64_t vt_ld) {
 
 // The same for Q|K (qk columns) and V (v columns) in one launch: on 256-feature tiles the CUs are split
 // between the two parts so that the longer one is shortest, neither part with more of them than it has tiles;
-// 128 x 128 tiles mix freely.
+// 128 x 128 tiles mix freely. The first such split is taken. Where a part's count is no multiple of 8 its later tiles
+// leave its XCDs' runs; whole eights at the same cost helped or hurt by what else the split changed (10240 + 5120
+// columns: 1560 tokens 124.5 -> 121.5 us, 1200 104.8 -> 102.9, 3600 258 -> 263, nine other counts within 1%).
 inline TilePlan select_qkv_tile(int64_t M, int64_t qk, int64_t v, int64_t cus, int64_t vt_ld) {
   TilePlan best{4, INT64_MAX, 0};
   for (int nj : {4, 3, 2, 0}) {

@@ -34,7 +34,8 @@
 //
 // The kernel is persistent: one workgroup per CU walks tiles v = blockIdx.x, + tile_wgs, ... in an
 // order where each XCD (workgroup ids are dealt round-robin over 8 XCDs) owns a contiguous,
-// L2-friendly run of tiles grouped 4 deep along m (measured against 2, 8 and 16: 1-5% faster). The
+// L2-friendly run of tiles grouped 4 deep along m (measured against 2, 8 and 16: 1-5% faster; the parts of
+// Q|K and V in one launch may leave it in their later rounds, see select_qkv_tile). The
 // next tile's first stage is loaded while the current tile's epilogue runs, so the epilogue overlaps
 // the next tile's load latency.
 //
@@ -1064,7 +1065,8 @@ __device__ __forceinline__ void ring_tiles(GemmArgs g, uint8_t (&sWh)[5][kHalfBy
 // first request finds it absent and the others wait with it. A few of the idle CUs of every XCD then walk
 // that XCD's panels in the order of k, one 4-byte load per 128-byte line, and leave the lines in its L2.
 // They set their own pace, and the launch ends with them if the tiles overtake them (fetch_wgs says how many
-// it takes). Results do not depend on it. Measured, weights not in the caches, without / with: 1560 tokens,
+// it takes). They carry the tile kernel's LDS, so their CUs are not free to other streams' launches
+// meanwhile. Results do not depend on it. Measured, weights not in the caches, without / with: 1560 tokens,
 // 5120 columns, 5120 deep 49.4 / 45.4 us, 13824 deep 119 / 113; 1000 tokens 36.3 / 33.9 and 120 / 87; 512
 // tokens 22.3 / 18.4 and 72 / 50; 100 tokens 20.7 / 16.2.
 // ------------------------------------------------------------------------------------------------

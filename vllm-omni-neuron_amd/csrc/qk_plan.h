@@ -18,7 +18,7 @@ struct QKPlan {
 // write), so a wave's tokens are served one after another while other waves hide the latency: as many
 // waves as one round holds (four workgroups of four waves per CU) come first, and only a sequence longer
 // than that gives a wave more than one token. At most 8: an S = 32760 launch is then one resident
-// round, and the gamma copy is shared by 32 tokens. With 8 tokens per wave throughout, 512 / 1560 /
+// round, and the gamma copy is shared by four waves' tokens. With 8 tokens per wave throughout, 512 / 1560 /
 // 3600 tokens ran 34 / 43 / 47 us: 16 / 49 / 113 workgroups on 256 CUs, each eight such chains long. One
 // token per wave took 24 us off the first, 22 off the second, 21 off the third (the block's
 // cross-attention K/V 94 -> 69 us, row_mx_qkv_proj of 3600 tokens 387 -> 344).

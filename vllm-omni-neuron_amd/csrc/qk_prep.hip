@@ -64,8 +64,9 @@ struct QKNormArgs {
 // kHalves: rotate-half pairs (i, i+64) (the drop-in path for the reference's de-interleaved
 // weights; it keeps the register budget but may spill a little), else interleaved pairs.
 // Up to 40 heads the fp32 gamma (8 bytes per column, as much as the token's own bf16 read and write)
-// is copied into LDS once per workgroup of 32 tokens instead of being read from L2 per token: per
-// chunk, every lane's first four values (16 bytes, lane-major), then the second four.
+// is copied into LDS once per workgroup (kWgWaves x tokens_per_wave tokens: 4 to 64) instead of being
+// read from L2 per token: per chunk, every lane's first four values (16 bytes, lane-major), then the
+// second four.
 // kWgWaves: waves per workgroup; with the key-norm maximum, more of them (qk_plan has the reason).
 // kPair: Q and K in one launch, its own instantiation: selected at run time, the second part's pointers and the
 // tables' stride took the single passes (the block's, at 128 registers) from 2 / 11 spilled registers
